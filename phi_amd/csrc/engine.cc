@@ -83,7 +83,12 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
   if (!rc) rc = e->Check(Upload(&e->d_next_, h.next.data(), h.next.size()), "upload next");
   if (!rc) rc = e->Check(Upload(&e->d_prev_, h.prev.data(), h.prev.size()), "upload prev");
   if (!rc) rc = e->Check(Upload(&e->d_occ_, h.occ.data(), h.occ.size()), "upload occ");
-  if (!rc) rc = e->Check(Upload(&e->d_mu_, h.mu.data(), h.mu.size()), "upload mu");
+  {
+    // (padded by a tile: the packed kernels load past a short tile's end)
+    std::vector<double> mu(h.mu);
+    mu.resize(mu.size() + kPackedPad / NE + 1, 0.0);
+    if (!rc) rc = e->Check(Upload(&e->d_mu_, mu.data(), mu.size()), "upload mu");
+  }
   if (!rc) rc = e->Check(Upload(&e->d_site_ptr_, h.site_ptr.data(), h.site_ptr.size()), "upload site_ptr");
   if (!rc) rc = e->Check(Upload(&e->d_site_modes_, h.site_modes.data(), h.site_modes.size()), "upload site_modes");
   if (!rc) rc = e->Check(Upload(&e->d_next_s_, h.next_s.data(), h.next_s.size()), "upload next_s");
@@ -100,6 +105,31 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
   if (mps == 0) mps = 1;
   e->mps_ = mps;
   if (!rc && mps <= 2) rc = e->UploadEdges(0, 0, 0);
+  // Packed Hermitian element order: 4 x 4 blocks of the upper triangle, block
+  // column by block column; a diagonal block's pairs, then its reals.
+  if (!rc && N <= 32 && mps <= 2) {
+    std::vector<int4> elem;
+    std::vector<int> place(NE, 0);
+    int o = 0;
+    auto put = [&](int i, int j) {
+      elem.push_back(make_int4(i, j, o, 0));
+      place[i + j * N] = 4 * o + (i == j ? 0 : 1);
+      if (i != j) place[j + i * N] = 4 * o + 2;
+      o += i == j ? 1 : 2;
+    };
+    for (int bj = 0; bj < N; bj += 4) {
+      const int ej = std::min(bj + 4, N);
+      for (int bi = 0; bi < bj; bi += 4)
+        for (int j = bj; j < ej; ++j)
+          for (int i = bi; i < bi + 4; ++i) put(i, j);
+      for (int j = bj; j < ej; ++j)
+        for (int i = bj; i < j; ++i) put(i, j);
+      for (int j = bj; j < ej; ++j) put(j, j);
+    }
+    rc = e->Check(Upload(&e->d_elem_, elem.data(), elem.size()), "upload elements");
+    if (!rc) rc = e->Check(Upload(&e->d_place_, place.data(), place.size()), "upload places");
+    e->h_place_ = place;
+  }
   e->slab_nodes_ = h.num_nodes;
   e->rho0_init_.assign(p.initial_density_matrix.begin(), p.initial_density_matrix.end());
   const size_t bytes = e->state_elems() * 2 * sizeof(double);
@@ -178,6 +208,10 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
   a.Hadj = e->d_Hadj_;
   a.edge = e->d_edge_;
   a.mps = e->mps_;
+  a.PE = N * (N + 1) / 2;
+  a.elem = e->d_elem_;
+  a.mPE = ((1ull << 32) + a.PE - 1) / a.PE;
+  a.mNM = ((1ull << 32) + (unsigned)(N * mps) - 1) / (unsigned)(N * mps);
   rc = e->SetLaunch(-1, 0, 0, 0);
   if (rc) {
     *why = e->err_;
@@ -196,7 +230,10 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
 int Engine::BuildEdges(int first, int nb, int vbase, int4** out) {
   const HierarchyTables& h = h_;
   const int N = h.N, mps = mps_;
-  std::vector<int4> edge((size_t)h.num_nodes * N * mps);
+  // (padded by a tile of absent neighbours: the packed kernels load past a
+  // short tile's end)
+  std::vector<int4> edge((size_t)(h.num_nodes + kPackedPad / (N * N) + 1) * N * mps,
+                         make_int4(-1, -1, -1, 0));
   for (int n = 0; n < h.num_nodes; ++n)
     for (int b = 0; b < N; ++b)
       for (int q = 0; q < mps; ++q) {
@@ -312,6 +349,8 @@ int Engine::CreateEnsemble(const PhiParameters& base, int members,
   const size_t bytes = e->state_elems() * 2 * sizeof(double);
   rc = e->Check(Upload(&e->d_Hm_, Hm.data(), Hm.size()), "upload member H");
   if (!rc) rc = e->Check(Upload(&e->d_moff_, e->moff_.data(), e->moff_.size()), "upload offsets");
+  const std::vector<int> zeros(16 * 16, 0);
+  if (!rc) rc = e->Check(Upload(&e->d_tile_ctr_, zeros.data(), zeros.size()), "upload counters");
   if (!rc) rc = e->Check(hipMalloc((void**)&e->d_rho_, bytes), "alloc ensemble rho");
   if (!rc) rc = e->Check(hipMemset(e->d_rho_, 0, bytes), "zero ensemble rho");
   // rho_0 of every member from the base initial density matrix.
@@ -329,6 +368,7 @@ int Engine::CreateEnsemble(const PhiParameters& base, int members,
   RhsArgs& a = e->args_;
   a.num_nodes = e->slab_nodes_;
   a.H = e->d_Hm_;
+  a.tile_ctr = e->d_tile_ctr_;
   a.real_h = real_h;
   rc = e->SetLaunch(2, 0, 0, 0);
   if (rc) {
@@ -344,7 +384,10 @@ int Engine::CreateEnsemble(const PhiParameters& base, int members,
 // nodes cut into tiles of at most `tile` nodes, members in order.
 int Engine::BuildTiles() {
   if (members_ == 0) return kOk;
-  const int T = args_.col_tile[fp32_ ? 1 : 0];
+  const int T = ActiveTile();
+  // launches in flight still read the list
+  const int rs = Synchronize();
+  if (rs) return rs;
   std::vector<TileDesc> t;
   for (int m = 0; m < members_; ++m)
     for (int lb = 0; lb < mreal_[m]; lb += T)
@@ -374,8 +417,11 @@ int Engine::GetMemberRho0(std::complex<double>* host) {
   // One gather kernel and one copy (a copy per member costs a round trip each).
   const size_t bytes = (size_t)members_ * NE * sizeof(double2);
   if (!d_mrho_) rc = Check(hipMalloc((void**)&d_mrho_, bytes), "alloc member rho0");
-  if (!rc) rc = Check(LaunchGatherNode0(d_rho_, d_moff_, members_, NE, d_mrho_, stream_),
-                      "gather member rho0");
+  if (!rc)
+    rc = Check(packed_ ? LaunchGatherNode0Packed(d_prho_, d_place_, d_moff_, members_, NE,
+                                                 d_mrho_, stream_)
+                       : LaunchGatherNode0(d_rho_, d_moff_, members_, NE, d_mrho_, stream_),
+               "gather member rho0");
   if (!rc) rc = Check(hipMemcpyAsync(host, d_mrho_, bytes, hipMemcpyDeviceToHost, stream_),
                       "member rho0");
   return rc ? rc : Synchronize();
@@ -390,7 +436,8 @@ Engine::~Engine() {
                   d_err_, d_hist_, d_hist_count_, d_partial_, d_dot_, d_moff_, d_Hm_,
                   d_tiles_, d_cbmi_, d_csite_, d_cslot_, d_cx_, d_cs_, d_cy_, d_cpack_, d_cfall_, d_active_, d_kf_[0], d_kf_[1],
                   d_kf_[2], d_kf_[3], d_kf_[4], d_kf_[5], d_rot_,
-                  d_ops_, d_alpha_, d_corr_, d_tlq_, d_tlsite_, d_mrho_};
+                  d_ops_, d_alpha_, d_corr_, d_tlq_, d_tlsite_, d_mrho_,
+                  d_elem_, d_place_, d_prho_, d_pnew_, d_hfrag_, d_tile_ctr_};
   for (void* p : ptrs) Free(p);
   if (h_stage_) (void)hipHostFree(h_stage_);
   if (h_ops_) (void)hipHostFree(h_ops_);
@@ -474,6 +521,9 @@ int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
         --t;
       const int rt = StreamThreads(t, f == 1, threads, &th);
       if (rt) return rt;
+      // Packed kernels: the given tile, or by default about 256 elements of
+      // one thread each.
+      a.pk_tile[f] = tile > 0 ? t : std::max(1, 256 / a.PE);
       // Kernels without a persistent form (RKF45) run the one-shot
       // matrix-core kernels with 256 threads and their default tile.
       int t1 = std::max(1, std::min(64, 256 / NE));
@@ -648,11 +698,17 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   if (N <= 32) cands.push_back({1, 0, 0, 0});
   cands.push_back({0, 0, 0, 0});
   // Save the state; tuning steps advance it.
-  const size_t bytes = state_elems() * 2 * sizeof(double);
+  rc = EnterState(stream_ok && !closure_ && rk4_form_ == kRk4Increment && PackedUsable());
+  if (rc) return rc;
+  // (the candidates run on the state's current form; one of another form
+  // runs on the other buffer, whose values do not matter)
+  const bool was_packed = packed_;
+  const size_t bytes = StateBytes();
   double* saved = nullptr;
   rc = Check(hipMalloc((void**)&saved, bytes), "alloc tune state");
   if (rc) return rc;
-  rc = Check(hipMemcpyAsync(saved, d_rho_, bytes, hipMemcpyDeviceToDevice, stream_), "save state");
+  rc = Check(hipMemcpyAsync(saved, StateBuf(), bytes, hipMemcpyDeviceToDevice, stream_),
+             "save state");
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc) rc = Check(hipEventCreate(&e0), "event");
   if (!rc) rc = Check(hipEventCreate(&e1), "event");
@@ -749,7 +805,9 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
-  const int rc_restore = Check(hipMemcpyAsync(d_rho_, saved, bytes, hipMemcpyDeviceToDevice,
+  packed_ = was_packed;
+  full_fresh_ = false;
+  const int rc_restore = Check(hipMemcpyAsync(StateBuf(), saved, bytes, hipMemcpyDeviceToDevice,
                                               stream_), "restore state");
   const int rc_sync = Synchronize();
   Free(saved);
@@ -788,29 +846,137 @@ int Engine::AllocBulk() {
   Free(d_tmp_);
   d_tmp_ = nullptr;
   rkf45_alloc_ = false;
-  const size_t bytes = state_elems() * 2 * (fp32_ ? sizeof(float) : sizeof(double));
+  const size_t real = fp32_ ? sizeof(float) : sizeof(double);
+  const size_t bytes = (state_elems() * 2 + kPackedPad) * real;
   int rc = Check(hipMalloc(&d_y_[0], bytes), "alloc y0");
   if (!rc) rc = Check(hipMalloc(&d_y_[1], bytes), "alloc y1");
-  if (!rc && !d_aux_) rc = Check(hipMalloc((void**)&d_aux_, state_elems() * 2 * sizeof(double)), "alloc aux");
+  if (!rc && !d_aux_)
+    rc = Check(hipMalloc((void**)&d_aux_, (state_elems() * 2 + kPackedPad) * sizeof(double)),
+               "alloc aux");
   if (rc) return rc;
   bulk_alloc_ = true;
   bulk_is_fp32_ = fp32_;
   return kOk;
 }
 
+bool Engine::PackedUsable() const {
+  const int f = fp32_ ? 1 : 0;
+  // Below 4 sites the diagonal, whose elements take both sides' gathers for
+  // half the data, outweighs the pairs: 55 members of 3 sites 41 us a step
+  // on the full kernels, 50 packed; 96 members of 4 sites 46 and 46.
+  if (h_.N < 4) return false;
+  // 32-bit byte offsets from a member's first node, 24-bit node ids, and no
+  // more LDS than the other kernels take.
+  if (!d_elem_ || !d_edge_ || h_.num_nodes >= (1 << 24)) return false;
+  const long long nodes = members_ ? h_.num_nodes : slab_nodes_;
+  if ((nodes + kPackedPad) * h_.N * h_.N * (long long)sizeof(double) >= (1LL << 32)) return false;
+  if (args_.col_nm != 2) return true;
+  return PackedTileLdsBytes(h_.N, h_.D, h_.L, mps_, args_.pk_tile[f], f == 1) <= kLdsBudget;
+}
+
+int Engine::UseFull() {
+  const int rc = SyncFull();
+  packed_ = full_fresh_ = false;
+  return rc;
+}
+
+int Engine::SyncFull() {
+  if (!packed_ || full_fresh_) return kOk;
+  const int rc = Check(LaunchUnpack(args_, slab_nodes_, d_prho_, d_rho_, stream_), "unpack state");
+  full_fresh_ = !rc;
+  return rc;
+}
+
+// The packed kernels' fragments of the current H (rebuilt after the precision
+// or H changed).
+int Engine::BuildFrag() {
+  if (hfrag_fp32_ == (fp32_ ? 1 : 0)) return kOk;
+  const int members = std::max(members_, 1);
+  int rc = kOk;
+  if (!d_hfrag_) {
+    rc = Check(hipMalloc(&d_hfrag_, (size_t)members * PackedFragElems(h_.N) * sizeof(double2)),
+               "alloc H fragments");
+    if (rc) {
+      d_hfrag_ = nullptr;
+      return rc;
+    }
+    args_.hfrag = d_hfrag_;
+  }
+  rc = Check(LaunchBuildFrag(args_, fp32_, members, d_hfrag_, stream_), "H fragments");
+  if (!rc) hfrag_fp32_ = fp32_ ? 1 : 0;
+  return rc;
+}
+
+int Engine::EnterState(bool want_packed) {
+  int rc = kOk;
+  if (!want_packed || not_hermitian_) {
+    rc = UseFull();
+  } else if (!packed_) {
+    const size_t reals = state_elems() + kPackedPad;
+    if (prho_reals_ != reals) {
+      Free(d_prho_);
+      Free(d_pnew_);
+      d_prho_ = d_pnew_ = nullptr;
+      prho_reals_ = 0;
+      if (hipMalloc((void**)&d_prho_, reals * sizeof(double)) != hipSuccess) {
+        // no room for the packed copy: the full kernels need none
+        (void)hipGetLastError();
+        d_prho_ = nullptr;
+        return EnsureTiles();
+      }
+      prho_reals_ = reals;
+    }
+    int bad = 0;
+    rc = Check(LaunchFillU64(reinterpret_cast<unsigned long long*>(d_err_), 0ull, 1, stream_),
+               "zero flag");
+    if (!rc) rc = Check(LaunchPack(args_, slab_nodes_, d_rho_, d_prho_,
+                                   reinterpret_cast<int*>(d_err_), stream_), "pack state");
+    if (!rc) rc = Check(hipMemcpyAsync(&bad, d_err_, sizeof(int), hipMemcpyDeviceToHost, stream_),
+                        "hermitian flag");
+    if (!rc) rc = Synchronize();
+    if (rc) return rc;
+    not_hermitian_ = bad != 0;
+    packed_ = !not_hermitian_;
+    full_fresh_ = packed_;
+  }
+  if (!rc && packed_) rc = BuildFrag();
+  if (!rc && tile_ctr_dirty_ && d_tile_ctr_) {
+    rc = Check(LaunchFillU64(reinterpret_cast<unsigned long long*>(d_tile_ctr_), 0ull, 128,
+                             stream_), "clear counters");
+    tile_ctr_dirty_ = rc != kOk;
+  }
+  return rc ? rc : EnsureTiles();
+}
+
 int Engine::SetState(const std::complex<double>* host) {
+  StateReplaced();
   int rc = Check(hipMemcpyAsync(d_rho_, host, state_elems() * sizeof(std::complex<double>),
                                 hipMemcpyHostToDevice, stream_), "set state");
   return rc ? rc : Synchronize();
 }
 
 int Engine::GetState(std::complex<double>* host) {
-  int rc = Check(hipMemcpyAsync(host, d_rho_, state_elems() * sizeof(std::complex<double>),
+  int rc = SyncFull();
+  if (!rc) rc = Check(hipMemcpyAsync(host, d_rho_, state_elems() * sizeof(std::complex<double>),
                                 hipMemcpyDeviceToHost, stream_), "get state");
   return rc ? rc : Synchronize();
 }
 
 int Engine::GetNode0(std::complex<double>* host) {
+  if (packed_) {
+    // N^2 reals, expanded here
+    const int NE = N() * N();
+    std::vector<double> p(NE + 1);
+    int rc = Check(hipMemcpyAsync(p.data(), d_prho_, NE * sizeof(double), hipMemcpyDeviceToHost,
+                                  stream_), "get node 0");
+    if (!rc) rc = Synchronize();
+    for (int e = 0; e < NE; ++e) {
+      const int w = h_place_[e], kind = w & 3;
+      const double im = kind ? p[(w >> 2) + 1] : 0.0;
+      host[e] = std::complex<double>(p[w >> 2], kind == 2 ? -im : im);
+    }
+    return rc;
+  }
   int rc = Check(hipMemcpyAsync(host, d_rho_, (size_t)N() * N() * sizeof(std::complex<double>),
                                 hipMemcpyDeviceToHost, stream_), "get node 0");
   return rc ? rc : Synchronize();
@@ -868,6 +1034,7 @@ int Engine::RhsNodes(const int* nodes, int count, std::complex<double>* y) {
                "node ids upload");
   // The general operator on the live state (current flags and H, as PHI's
   // Get reads the node's linked neighbours), then the requested blocks.
+  if (!rc) rc = SyncFull();
   if (!rc) rc = OperatorRhs(d_rho_, dy);
   if (!rc) rc = Check(LaunchGatherNode0(dy, dids, count, NE, dout, stream_), "gather nodes");
   if (!rc) rc = Check(hipMemcpyAsync(y, dout, out_bytes, hipMemcpyDeviceToHost, stream_),
@@ -892,7 +1059,7 @@ void Engine::StageBuffers(int form, const void* in[4], void* out[4], void** aux)
   if (form == kRk4Increment) {
     // K = L rho in y0 (read again by stages 2 and 3), D in y1, D' in aux
     // (FP64-sized, unused by this form otherwise).
-    in[0] = d_rho_, in[1] = d_y_[0], in[2] = d_y_[1], in[3] = d_aux_;
+    in[0] = RunsPacked() ? d_prho_ : d_rho_, in[1] = d_y_[0], in[2] = d_y_[1], in[3] = d_aux_;
     out[0] = d_y_[0], out[1] = d_y_[1], out[2] = d_aux_, out[3] = nullptr;
     *aux = d_y_[0];
     return;
@@ -902,6 +1069,23 @@ void Engine::StageBuffers(int form, const void* in[4], void* out[4], void** aux)
   *aux = d_aux_;
 }
 
+// ctr_set: the claim counter set of an ensemble's packed launch; it
+// alternates from launch to launch, starting with set 0 on every step (a
+// step is four launches).
+int Engine::Rk4Stage(int s, int form, const void* in, void* aux, void* out, double dt,
+                     int ctr_set) {
+  if (RunsPacked()) {
+    RhsArgs a = StageArgs(s);
+    a.ctr_set = ctr_set;
+    const int rc = Check(LaunchRk4Packed(a, fp32_, s, in, d_prho_, aux, out, dt, stream_),
+                         "rk4 stage");
+    if (rc) tile_ctr_dirty_ = true;
+    return rc;
+  }
+  return Check(LaunchRk4Stage(StageArgs(s), fp32_, s, form, in, d_rho_, aux, out, dt, stream_),
+               "rk4 stage");
+}
+
 int Engine::Rk4Step(double dt, bool snapshot) {
   const int form = StepForm();
   const void* in[4];
@@ -909,15 +1093,22 @@ int Engine::Rk4Step(double dt, bool snapshot) {
   void* aux;
   StageBuffers(form, in, out, &aux);
   int rc = kOk;
+  const bool pk = RunsPacked();
   for (int s = 0; s < 4 && !rc; ++s) {
     if (closure_) rc = ClosurePredict(in[s], s > 0 && fp32_);
-    if (!rc)
-      rc = Check(LaunchRk4Stage(StageArgs(s), fp32_, s, form, in[s], d_rho_, aux, out[s], dt,
-                                stream_), "rk4 stage");
+    if (!rc) rc = Rk4Stage(s, form, in[s], aux, out[s], dt, s & 1);
   }
+  if (pk) full_fresh_ = false;
   if (!rc && snapshot) {
     // A single hierarchy records rho_0; an ensemble the member average.
-    if (members_)
+    if (pk && members_)
+      rc = Check(LaunchSnapshotMeanPacked(d_prho_, d_place_, d_moff_, members_, d_hist_,
+                                          d_hist_count_, N() * N(), hist_capacity_, stream_),
+                 "snapshot mean");
+    else if (pk)
+      rc = Check(LaunchSnapshotPacked(d_prho_, d_place_, d_hist_, d_hist_count_, N() * N(),
+                                      hist_capacity_, stream_), "snapshot");
+    else if (members_)
       rc = Check(LaunchSnapshotMean(d_rho_, d_moff_, members_, d_hist_, d_hist_count_, N() * N(),
                                     hist_capacity_, stream_), "snapshot mean");
     else
@@ -938,7 +1129,8 @@ void Engine::DropGraph() {
 int Engine::GraphBlock(int steps, int snap_every, double dt) {
   GraphKey key{steps, snap_every, dt, fp32_, StepForm(), args_.col_nm,
                args_.col_tile[0], args_.col_tile[1], args_.col_threads[0], args_.col_threads[1],
-               args_.col_grid[0], args_.col_grid[1], d_y_[0], d_rho_, d_tiles_, {}};
+               args_.col_grid[0], args_.col_grid[1], d_y_[0],
+               RunsPacked() ? d_prho_ : d_rho_, d_tiles_, {}};
   for (int f = 0; f < 2; ++f)
     for (int s = 0; s < 4; ++s) {
       key.stage[f * 8 + s] = stage_threads_[f][s];
@@ -975,6 +1167,8 @@ int Engine::Rk4Steps(long long nsteps, double dt, long long step_offset, int sna
     last_eager_steps_ = nsteps;
     return rc;
   }
+  rc = EnterState(PackedForm());
+  if (rc) return rc;
   // Graph blocks of G steps, G a multiple of the snapshot period, aligned so
   // that every block starts on a snapshot step.
   int G = 0;
@@ -996,6 +1190,7 @@ int Engine::Rk4Steps(long long nsteps, double dt, long long step_offset, int sna
     for (; s + G <= nsteps; s += G) {
       rc = Check(hipGraphLaunch(graph_exec_, stream_), "graph launch");
       if (rc) return rc;
+      full_fresh_ = false;
       last_graph_steps_ += G;
     }
   }
@@ -1038,11 +1233,14 @@ int Engine::Rk4StageTimes(long long nsteps, double dt, double ms[4]) {
   // (an event between every kernel would add its own gap to each), after
   // one untimed launch.  The stages run in RK4 order on RK4's buffers; the
   // repeated last stage moves rho, so the state is saved and restored.
-  const size_t bytes = state_elems() * 2 * sizeof(double);
+  rc = EnterState(PackedForm());
+  if (rc) return rc;
+  const size_t bytes = StateBytes();
   double* saved = nullptr;
   rc = Check(hipMalloc((void**)&saved, bytes), "alloc timing state");
   if (rc) return rc;
-  rc = Check(hipMemcpyAsync(saved, d_rho_, bytes, hipMemcpyDeviceToDevice, stream_), "save state");
+  rc = Check(hipMemcpyAsync(saved, StateBuf(), bytes, hipMemcpyDeviceToDevice, stream_),
+             "save state");
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc) rc = Check(hipEventCreate(&e0), "event");
   if (!rc) rc = Check(hipEventCreate(&e1), "event");
@@ -1054,8 +1252,7 @@ int Engine::Rk4StageTimes(long long nsteps, double dt, double ms[4]) {
   for (int s = 0; s < 4 && !rc; ++s) {
     for (long long i = 0; i <= nsteps && !rc; ++i) {
       if (i == 1) rc = Check(hipEventRecord(e0, stream_), "record");
-      if (!rc) rc = Check(LaunchRk4Stage(StageArgs(s), fp32_, s, form, in[s], d_rho_, aux, out[s],
-                                         dt, stream_), "rk4 stage");
+      if (!rc) rc = Rk4Stage(s, form, in[s], aux, out[s], dt, ((nsteps + 1) * s + i) & 1);
     }
     if (!rc) rc = Check(hipEventRecord(e1, stream_), "record");
     if (!rc) rc = Check(hipEventSynchronize(e1), "event sync");
@@ -1065,7 +1262,7 @@ int Engine::Rk4StageTimes(long long nsteps, double dt, double ms[4]) {
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
-  const int rc_restore = Check(hipMemcpyAsync(d_rho_, saved, bytes, hipMemcpyDeviceToDevice,
+  const int rc_restore = Check(hipMemcpyAsync(StateBuf(), saved, bytes, hipMemcpyDeviceToDevice,
                                               stream_), "restore state");
   const int rc_sync = Synchronize();
   Free(saved);
@@ -1099,6 +1296,9 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
     err_ = "BiCGSTAB(ell) takes max_iter >= 0";
     return kErrInvalidArgument;
   }
+  const int ru = UseFull();
+  if (ru) return ru;
+  not_hermitian_ = false;
   const size_t n = state_elems();
   const size_t bytes = n * 2 * sizeof(double);
   // r_0..r_ell, u_0..u_ell, rtilde
@@ -1343,14 +1543,27 @@ int Engine::Rkf45Attempt(const Rkf45Coefs& c, double* err, double t, const doubl
   int rc = AllocBulk();
   if (rc) return rc;
   if (!rkf45_alloc_) {
-    const size_t bytes = state_elems() * 2 * (fp32_ ? sizeof(float) : sizeof(double));
+    const size_t bytes = (state_elems() * 2 + kPackedPad) * (fp32_ ? sizeof(float) : sizeof(double));
     for (auto& k : d_k_)
       if (!rc) rc = Check(hipMalloc(&k, bytes), "alloc k");
     if (!rc) rc = Check(hipMalloc(&d_tmp_, bytes), "alloc tmp");
     if (rc) return rc;
     rkf45_alloc_ = true;
   }
+  attempt_packed_ = false;
   if (explicit_path()) return ExplicitRkf45Attempt(c, err, t, a, src);
+  // A time-dependent H may rotate the buffers, which the full layout takes.
+  rc = EnterState(!src && !closure_ && args_.col_nm == 2 && PackedUsable());
+  if (rc) return rc;
+  if (packed_ && !d_pnew_) {
+    if (hipMalloc((void**)&d_pnew_, prho_reals_ * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      d_pnew_ = nullptr;
+      rc = UseFull();
+      if (rc) return rc;
+    }
+  }
+  attempt_packed_ = packed_;
   Rkf45Bufs<float> bf{};
   Rkf45Bufs<double> bd{};
   for (int i = 0; i < 5; ++i) {
@@ -1359,7 +1572,7 @@ int Engine::Rkf45Attempt(const Rkf45Coefs& c, double* err, double t, const doubl
   }
   // Stage inputs ping-pong between d_tmp_ and d_y_[0].
   void* tin[2] = {d_tmp_, d_y_[0]};
-  bf.rho_new = bd.rho_new = d_aux_;
+  bf.rho_new = bd.rho_new = packed_ ? d_pnew_ : d_aux_;
   bf.err = bd.err = d_err_;
   rc = Check(LaunchFillU64(d_err_, 0ull, 1, stream_), "zero err");
   for (int s = 0; s < 6 && !rc; ++s) {
@@ -1389,8 +1602,10 @@ int Engine::Rkf45Attempt(const Rkf45Coefs& c, double* err, double t, const doubl
     }
     bf.tmp_out = (float*)tin[s & 1];
     bd.tmp_out = (double*)tin[s & 1];
-    const void* in = s == 0 ? (const void*)d_rho_ : tin[(s - 1) & 1];
-    rc = Check(LaunchRkf45Stage(args_, fp32_, s, in, d_rho_, bf, bd, c, stream_), "rkf45 stage");
+    const void* in = s == 0 ? (const void*)StateBuf() : tin[(s - 1) & 1];
+    rc = Check(packed_ ? LaunchRkf45Packed(args_, fp32_, s, in, d_prho_, bf, bd, c, stream_)
+                       : LaunchRkf45Stage(args_, fp32_, s, in, d_rho_, bf, bd, c, stream_),
+               "rkf45 stage");
   }
   unsigned long long bits = 0;
   if (!rc) rc = Check(hipMemcpyAsync(&bits, d_err_, sizeof(bits), hipMemcpyDeviceToHost, stream_), "err");
@@ -1403,7 +1618,14 @@ int Engine::Rkf45Attempt(const Rkf45Coefs& c, double* err, double t, const doubl
 }
 
 int Engine::Rkf45Accept() {
+  if (attempt_packed_) {
+    std::swap(d_prho_, d_pnew_);
+    packed_ = true;
+    full_fresh_ = false;
+    return kOk;
+  }
   std::swap(d_rho_, d_aux_);
+  packed_ = full_fresh_ = false;
   if (tl_) {
     // Time-local matrices to t + dt (a4 = dt), saved for the next step.
     int rc = TlStep(tl_a_[3] - tl_a_[4]);
@@ -1431,6 +1653,9 @@ int Engine::SteadyState(double tol, int max_iter, int* iters, double* resid,
   // Unpreconditioned complex BiCGSTAB (van der Vorst 1992) on A x = b with
   // b = e_(node 0, element (0,0)); inner products conjugate the first
   // argument; all scalars and reductions in FP64.
+  const int ru = UseFull();
+  if (ru) return ru;
+  not_hermitian_ = false;
   const size_t n = state_elems();
   const size_t bytes = n * 2 * sizeof(double);
   double* v[7] = {nullptr};  // r, rhat, p, vv, s, t, tmp

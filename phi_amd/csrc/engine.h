@@ -251,6 +251,7 @@ class Engine {
   int Check(hipError_t e, const char* where);
   int AllocBulk();
   int Rk4Step(double dt, bool snapshot);
+  int Rk4Stage(int s, int form, const void* in, void* aux, void* out, double dt, int ctr_set);
   // The stage order a step runs now, and each stage's input, output and
   // auxiliary buffer for it (inputs alternate so that a stage never
   // overwrites what its own neighbour gathers read).
@@ -348,13 +349,50 @@ class Engine {
   double* d_mrho_ = nullptr;  // node 0 of every member (GetMemberRho0)
   double2* d_Hm_ = nullptr;
   TileDesc* d_tiles_ = nullptr;
+  int* d_tile_ctr_ = nullptr;
+  bool tile_ctr_dirty_ = false;  // a stage launch failed: clear before the next run
   int tiles_cap_ = 0;
   int tiles_for_ = 0;  // tile size the descriptors were built for
   int BuildTiles();
   // Rebuilds the ensemble tile descriptors when the active tile size
   // changed (precision or launch shape); a no-op for a single hierarchy.
-  int EnsureTiles() {
-    return members_ && tiles_for_ != args_.col_tile[fp32_ ? 1 : 0] ? BuildTiles() : 0;
+  int EnsureTiles() { return members_ && tiles_for_ != ActiveTile() ? BuildTiles() : 0; }
+
+  // Packed Hermitian state (heom_packed.h).  The increment-form RK4 steps and
+  // RKF45 attempts of a Hermitian state run on packed slabs: packed_ says
+  // that the state is d_prho_ (d_rho_ then mirrors it only while
+  // full_fresh_); every other path runs on d_rho_ after UseFull().  The
+  // state is checked (every ADO equal to its conjugate transpose) once after
+  // it was set; not_hermitian_ keeps a state that failed on the full kernels.
+  int4* d_elem_ = nullptr;
+  int* d_place_ = nullptr;
+  std::vector<int> h_place_;
+  void* d_hfrag_ = nullptr;     // H fragments of the packed kernels
+  int hfrag_fp32_ = -1;         // precision they are built for (-1: stale)
+  int BuildFrag();
+  double* d_prho_ = nullptr;
+  double* d_pnew_ = nullptr;    // RKF45 5th-order solution
+  size_t prho_reals_ = 0;       // reals d_prho_ and d_pnew_ were allocated for
+  bool packed_ = false, full_fresh_ = false, not_hermitian_ = false, attempt_packed_ = false;
+  bool PackedUsable() const;    // sizes fit the packed kernels in this precision
+  bool PackedForm() const {     // RK4 steps would take the packed kernels now
+    return PackedUsable() && !closure_ && args_.col_nm == 2 && rk4_form_ == kRk4Increment;
+  }
+  bool RunsPacked() const { return packed_ && PackedForm(); }  // an RK4 step launched now
+  int ActiveTile() const {
+    const int f = fp32_ ? 1 : 0;
+    return RunsPacked() ? args_.pk_tile[f] : args_.col_tile[f];
+  }
+  int EnterState(bool want_packed);  // makes packed_ as wanted where it can
+  int UseFull();                     // d_rho_ becomes the state
+  int SyncFull();                    // d_rho_ mirrors the state
+  void StateReplaced() {             // d_rho_ holds a new state
+    packed_ = full_fresh_ = not_hermitian_ = false;
+  }
+  // Reals of the state buffer a step runs on.
+  double* StateBuf() const { return packed_ ? d_prho_ : d_rho_; }
+  size_t StateBytes() const {
+    return state_elems() * (packed_ ? 1 : 2) * sizeof(double);
   }
   int Unsupported(const char* what);
 

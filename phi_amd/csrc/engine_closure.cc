@@ -74,6 +74,7 @@ int Engine::ClosureSamples(int shallow_lh, float* X, float* T, long long cap_row
   if (!rc) rc = Check(hipMalloc((void**)&dX, (size_t)nrows * n_in * 4), "alloc X");
   if (!rc) rc = Check(hipMalloc((void**)&dT, (size_t)nrows * n_out * 4), "alloc T");
   if (!rc) rc = Check(hipMalloc((void**)&dS, (size_t)nrows * 4), "alloc S");
+  if (!rc) rc = SyncFull();
   if (!rc)
     rc = Check(LaunchClosureInputs(d_rho_, false, dM, members, first, nb, NE, D, dB, dX, dS,
                                    stream_), "closure inputs");
@@ -191,6 +192,7 @@ int Engine::AttachClosure(Mlp* mlp) {
   DropGraph();
   FreeD(d_rho_);
   d_rho_ = rho;
+  StateReplaced();
   FreeD(d_aux_);
   d_aux_ = nullptr;
   FreeD(d_y_[0]);
@@ -202,6 +204,10 @@ int Engine::AttachClosure(Mlp* mlp) {
   }
   FreeD(d_tmp_);
   d_tmp_ = nullptr;
+  FreeD(d_prho_);
+  FreeD(d_pnew_);
+  d_prho_ = d_pnew_ = nullptr;
+  prho_reals_ = 0;
   bulk_alloc_ = false;
   rkf45_alloc_ = false;
   FreeD(d_moff_);

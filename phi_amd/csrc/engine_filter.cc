@@ -80,6 +80,7 @@ int Engine::ExplicitRk4Step(double t, double dt, bool snapshot, HamiltonianSourc
     return kErrUnsupported;
   }
   int rc = ExplicitAlloc(4);
+  if (!rc) rc = UseFull();
   if (rc) return rc;
   const size_t n = state_elems();
   double* y = (double*)d_y_[0];
@@ -134,6 +135,7 @@ int Engine::ExplicitRkf45Attempt(const Rkf45Coefs& c, double* err, double t, con
     return kErrUnsupported;
   }
   int rc = ExplicitAlloc(6);
+  if (!rc) rc = UseFull();
   if (rc) return rc;
   const size_t n = state_elems();
   double* y = (double*)d_y_[0];

@@ -40,6 +40,7 @@ static constexpr int kSlotsPerStep = 3;
 int Engine::SetHamiltonian(const std::complex<double>* H) {
   const int N = this->N(), NE = N * N;
   h_hcur_.assign(H, H + NE);
+  hfrag_fp32_ = -1;
   int rc = kOk;
   if (!h_stage_) {
     rc = Check(hipHostMalloc((void**)&h_stage_, (size_t)kSlotsPerStep * 4 * NE * sizeof(double2)),
@@ -96,6 +97,7 @@ int Engine::Rk4StepsTD(long long nsteps, const double* t_before, double dt, long
     return kErrUnsupported;
   }
   int rc = AllocBulk();
+  if (!rc) rc = EnterState(false);
   if (rc) return rc;
   if (explicit_path()) {
     // Diagonal / full coupling operators, time-local truncation: the

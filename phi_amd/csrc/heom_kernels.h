@@ -36,12 +36,24 @@ struct RhsArgs {
   // site b ({-1, -1, -1, 0} when absent).
   const int4* edge;
   int mps;
+  // Packed Hermitian kernels (heom_packed.h): PE = N (N + 1) / 2 elements per
+  // node, elem[e] = {row, column, real offset, 0} in storage order; nodes per
+  // block per precision.
+  int PE;
+  int pk_tile[2];
+  const int4* elem;
+  const void* hfrag;           // H / hbar fragments in the bulk precision, per member
+  unsigned long long mPE, mNM; // ceil(2^32 / PE), ceil(2^32 / (N mps))
   // Ensembles (persistent kernels only): slab of several members of one
   // bath model sharing the tables of the deepest member.  tiles[t] describes
   // tile t (TileDesc) and H holds every member's shifted H (stride N*N).
   // tiles is nullptr for a single hierarchy.
   const TileDesc* tiles;
   int ntiles;
+  // Packed kernels: two sets of the 8 runs' claim counters, 64 bytes apart;
+  // a launch uses set ctr_set and clears the other for the next launch.
+  int* tile_ctr;
+  int ctr_set;
   int real_h;                 // imag(H) == 0 everywhere
   unsigned long long mN, mNE; // ceil(2^32 / N), ceil(2^32 / N^2)
   double inv_hbar;
@@ -99,6 +111,39 @@ hipError_t LaunchRk4Stage(const RhsArgs& a, bool fp32, int stage, int form, cons
 hipError_t LaunchRkf45Stage(const RhsArgs& a, bool fp32, int stage, const void* in,
                             const double* rho, const Rkf45Bufs<float>& bf,
                             const Rkf45Bufs<double>& bd, const Rkf45Coefs& c, hipStream_t s);
+
+// Packed Hermitian slabs (heom_packed.h).  LDS bytes of a block.
+size_t PackedTileLdsBytes(int N, int D, int L, int mps, int tile, bool fp32);
+// Nodes past a slab's (and its tables') end that a short tile's loads touch
+// reals of: buffers and tables are this much longer.
+constexpr int kPackedPad = 1024 + 64;
+// The increment form's stage and RKF45's on packed slabs (rho, K, yout and
+// the RKF45 buffers all packed).
+hipError_t LaunchRk4Packed(const RhsArgs& a, bool fp32, int stage, const void* in, double* rho,
+                           const void* kk, void* yout, double dt, hipStream_t s);
+hipError_t LaunchRkf45Packed(const RhsArgs& a, bool fp32, int stage, const void* in,
+                             const double* rho, const Rkf45Bufs<float>& bf,
+                             const Rkf45Bufs<double>& bd, const Rkf45Coefs& c, hipStream_t s);
+// hfrag (members x fragment elements, complex of the bulk precision) from a.H.
+size_t PackedFragElems(int N);
+hipError_t LaunchBuildFrag(const RhsArgs& a, bool fp32, int members, void* out, hipStream_t s);
+// packed <- full; *flag (zeroed before) = 1 unless every ADO equals its
+// conjugate transpose exactly.
+hipError_t LaunchPack(const RhsArgs& a, int nodes, const double* full, double* packed, int* flag,
+                      hipStream_t s);
+// full <- packed for `nodes` nodes.
+hipError_t LaunchUnpack(const RhsArgs& a, int nodes, const double* packed, double* full,
+                        hipStream_t s);
+// LaunchSnapshot, LaunchSnapshotMean and LaunchGatherNode0 from a packed
+// slab; place[e] = 4 * offset + (0 diagonal, 1 upper, 2 lower triangle) of
+// column-major element e.
+hipError_t LaunchSnapshotPacked(const double* src, const int* place, double* hist, int* counter,
+                                int ne, int capacity, hipStream_t s);
+hipError_t LaunchSnapshotMeanPacked(const double* src, const int* place,
+                                    const int* member_offsets, int members, double* hist,
+                                    int* counter, int ne, int capacity, hipStream_t s);
+hipError_t LaunchGatherNode0Packed(const double* src, const int* place, const int* member_offsets,
+                                   int members, int ne, double* dst, hipStream_t s);
 // PHI's Get on any complex input, FP64.  active: the adaptive truncation's
 // node flags (inactive neighbours' terms skipped), or null.
 hipError_t LaunchRhsGeneral(const RhsArgs& a, const double* x, double* y, int trace_row,

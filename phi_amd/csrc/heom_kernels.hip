@@ -8,7 +8,7 @@
 #include <mutex>
 #include <tuple>
 
-#include "heom_stream.h"
+#include "heom_packed.h"
 
 namespace phi {
 namespace dev {
@@ -202,15 +202,34 @@ __global__ void __launch_bounds__(256) rhs_general_lds(RhsArgs A, const double* 
 
 // --- Small utility kernels ----------------------------------------------------
 
+// Column-major element e of node n of a full slab, or of a packed one
+// (place[e] = 4 * offset + kind, kind 0 diagonal, 1 upper, 2 lower triangle).
+struct FullSrc {
+  const double* p;
+  __device__ __forceinline__ double2 at(size_t n, int ne, int e) const {
+    return reinterpret_cast<const double2*>(p)[n * ne + e];
+  }
+};
+struct PackedSrc {
+  const double* p;
+  const int* place;
+  __device__ __forceinline__ double2 at(size_t n, int ne, int e) const {
+    const int w = place[e], kind = w & 3;
+    const double* q = p + n * ne + (w >> 2);
+    const double im = kind ? q[1] : 0.;
+    return make_double2(q[0], kind == 2 ? -im : im);
+  }
+};
+
 // dst[slot] = node 0 of src (N*N complex), slot read from *counter, then
 // ++*counter.  One block.
-__global__ void snapshot_node0(const double* __restrict__ src, double* __restrict__ hist,
-                               int* __restrict__ counter, int ne, int capacity) {
+template <class SRC>
+__global__ void snapshot_node0(SRC src, double* __restrict__ hist, int* __restrict__ counter,
+                               int ne, int capacity) {
   const int slot = *counter;
   if (slot < capacity) {
     for (int e = threadIdx.x; e < ne; e += blockDim.x)
-      reinterpret_cast<double2*>(hist)[(size_t)slot * ne + e] =
-          reinterpret_cast<const double2*>(src)[e];
+      reinterpret_cast<double2*>(hist)[(size_t)slot * ne + e] = src.at(0, ne, e);
   }
   __syncthreads();
   if (threadIdx.x == 0) *counter = slot + 1;
@@ -222,7 +241,8 @@ __global__ void snapshot_node0(const double* __restrict__ src, double* __restric
 // left unchanged; bump_counter advances it).  One block per element: each
 // thread sums members tid, tid + blockDim.x, ... in order, then a fixed-order
 // tree over the block, so the sum is the same on every run.
-__global__ void __launch_bounds__(256) snapshot_mean(const double* __restrict__ src,
+template <class SRC>
+__global__ void __launch_bounds__(256) snapshot_mean(SRC src,
                                                      const int* __restrict__ moff, int members,
                                                      double* __restrict__ hist,
                                                      const int* __restrict__ counter, int ne,
@@ -230,10 +250,9 @@ __global__ void __launch_bounds__(256) snapshot_mean(const double* __restrict__ 
   __shared__ double2 red[256];
   const int slot = *counter;
   const int e = blockIdx.x;
-  const double2* s = reinterpret_cast<const double2*>(src);
   double x = 0, y = 0;
   for (int m = threadIdx.x; m < members; m += blockDim.x) {
-    const double2 v = s[(size_t)moff[m] * ne + e];
+    const double2 v = src.at(moff[m], ne, e);
     x += v.x;
     y += v.y;
   }
@@ -256,14 +275,51 @@ __global__ void __launch_bounds__(256) snapshot_mean(const double* __restrict__ 
 __global__ void bump_counter(int* counter) { *counter += 1; }
 
 // dst[m] = node 0 of member m (members x ne complex), for one copy to the host.
-__global__ void gather_node0(const double* __restrict__ src, const int* __restrict__ moff,
-                             int members, int ne, double* __restrict__ dst) {
+template <class SRC>
+__global__ void gather_node0(SRC src, const int* __restrict__ moff, int members, int ne,
+                             double* __restrict__ dst) {
   const long long n = (long long)members * ne;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const int m = (int)(i / ne), e = (int)(i - (long long)m * ne);
-    reinterpret_cast<double2*>(dst)[i] =
-        reinterpret_cast<const double2*>(src)[(size_t)moff[m] * ne + e];
+    reinterpret_cast<double2*>(dst)[i] = src.at(moff[m], ne, e);
+  }
+}
+
+// packed <- full over the elements of `nodes` nodes; *flag = 1 where an ADO
+// differs from its conjugate transpose (NaN included).
+__global__ void __launch_bounds__(256) pack_nodes(RhsArgs A, long long nodes,
+                                                  const double2* __restrict__ full,
+                                                  double* __restrict__ packed, int* flag) {
+  const long long tot = nodes * A.PE;
+  bool bad = false;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
+       i += (long long)gridDim.x * blockDim.x) {
+    const long long n = i / A.PE;
+    const int4 el = A.elem[(int)(i - n * A.PE)];
+    const double2 u = full[n * A.NE + el.y * A.N + el.x];
+    const double2 v = full[n * A.NE + el.x * A.N + el.y];
+    if (!(u.x == v.x && u.y == -v.y)) bad = true;
+    double* o = packed + n * A.NE + el.z;
+    o[0] = u.x;
+    if (el.x != el.y) o[1] = u.y;
+  }
+  if (bad) *flag = 1;
+}
+
+__global__ void __launch_bounds__(256) unpack_nodes(RhsArgs A, long long nodes,
+                                                    const double* __restrict__ packed,
+                                                    double2* __restrict__ full) {
+  const long long tot = nodes * A.PE;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
+       i += (long long)gridDim.x * blockDim.x) {
+    const long long n = i / A.PE;
+    const int4 el = A.elem[(int)(i - n * A.PE)];
+    const double* o = packed + n * A.NE + el.z;
+    const bool dg = el.x == el.y;
+    const double re = o[0], im = dg ? 0. : o[1];
+    full[n * A.NE + el.y * A.N + el.x] = make_double2(re, im);
+    if (!dg) full[n * A.NE + el.x * A.N + el.y] = make_double2(re, -im);
   }
 }
 
@@ -707,6 +763,65 @@ size_t StreamTileLdsBytes(int N, int D, int L, int tile, bool fp32) {
   return dev::StreamLdsBytes(N, D, L, tile, fp32 ? sizeof(float) : sizeof(double));
 }
 
+hipError_t LaunchRk4PackedF64(const RhsArgs& a, int stage, const void* in, double* rho,
+                              const void* kk, void* yout, double dt, hipStream_t s);
+hipError_t LaunchRk4PackedF32(const RhsArgs& a, int stage, const void* in, double* rho,
+                              const void* kk, void* yout, double dt, hipStream_t s);
+hipError_t LaunchRkf45PackedF64(const RhsArgs& a, int stage, const void* in, const double* rho,
+                                const Rkf45Bufs<double>& b, const Rkf45Coefs& c, hipStream_t s);
+hipError_t LaunchRkf45PackedF32(const RhsArgs& a, int stage, const void* in, const double* rho,
+                                const Rkf45Bufs<float>& b, const Rkf45Coefs& c, hipStream_t s);
+
+hipError_t LaunchRk4Packed(const RhsArgs& a, bool fp32, int stage, const void* in, double* rho,
+                           const void* kk, void* yout, double dt, hipStream_t s) {
+  return fp32 ? LaunchRk4PackedF32(a, stage, in, rho, kk, yout, dt, s)
+              : LaunchRk4PackedF64(a, stage, in, rho, kk, yout, dt, s);
+}
+
+hipError_t LaunchRkf45Packed(const RhsArgs& a, bool fp32, int stage, const void* in,
+                             const double* rho, const Rkf45Bufs<float>& bf,
+                             const Rkf45Bufs<double>& bd, const Rkf45Coefs& c, hipStream_t s) {
+  return fp32 ? LaunchRkf45PackedF32(a, stage, in, rho, bf, c, s)
+              : LaunchRkf45PackedF64(a, stage, in, rho, bd, c, s);
+}
+
+size_t PackedTileLdsBytes(int N, int D, int L, int mps, int tile, bool fp32) {
+  return dev::PackedLdsBytes(N, D, L, mps, tile, fp32 ? sizeof(float) : sizeof(double));
+}
+
+size_t PackedFragElems(int N) { return (size_t)dev::StreamFragCount(N); }
+
+hipError_t LaunchBuildFrag(const RhsArgs& a, bool fp32, int members, void* out, hipStream_t s) {
+  const long long n = (long long)members * dev::StreamFragCount(a.N);
+  const unsigned blocks = (unsigned)std::min<long long>((n + 255) / 256, 4096);
+  if (fp32)
+    hipLaunchKernelGGL(dev::build_hfrag<float>, dim3(blocks), dim3(256), 0, s, a, members,
+                       (float2*)out);
+  else
+    hipLaunchKernelGGL(dev::build_hfrag<double>, dim3(blocks), dim3(256), 0, s, a, members,
+                       (double2*)out);
+  return hipGetLastError();
+}
+
+static unsigned PackBlocks(const RhsArgs& a, int nodes) {
+  const long long b = ((long long)nodes * a.PE + 255) / 256;
+  return (unsigned)(b < 1 ? 1 : (b > 16384 ? 16384 : b));
+}
+
+hipError_t LaunchPack(const RhsArgs& a, int nodes, const double* full, double* packed, int* flag,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(dev::pack_nodes, dim3(PackBlocks(a, nodes)), dim3(256), 0, s, a,
+                     (long long)nodes, (const double2*)full, packed, flag);
+  return hipGetLastError();
+}
+
+hipError_t LaunchUnpack(const RhsArgs& a, int nodes, const double* packed, double* full,
+                        hipStream_t s) {
+  hipLaunchKernelGGL(dev::unpack_nodes, dim3(PackBlocks(a, nodes)), dim3(256), 0, s, a,
+                     (long long)nodes, packed, (double2*)full);
+  return hipGetLastError();
+}
+
 hipError_t LaunchRk4F64(const RhsArgs& a, int stage, int form, const void* in, double* rho,
                         void* aux, void* yout, double dt, hipStream_t s);
 hipError_t LaunchRk4F32(const RhsArgs& a, int stage, int form, const void* in, double* rho,
@@ -790,14 +905,32 @@ hipError_t LaunchRhsGeneral(const RhsArgs& a, const double* x, double* y, int tr
 
 hipError_t LaunchSnapshot(const double* src, double* hist, int* counter, int ne, int capacity,
                           hipStream_t s) {
-  hipLaunchKernelGGL(dev::snapshot_node0, dim3(1), dim3(256), 0, s, src, hist, counter, ne, capacity);
+  hipLaunchKernelGGL(dev::snapshot_node0<dev::FullSrc>, dim3(1), dim3(256), 0, s,
+                     dev::FullSrc{src}, hist, counter, ne, capacity);
+  return hipGetLastError();
+}
+
+hipError_t LaunchSnapshotPacked(const double* src, const int* place, double* hist, int* counter,
+                                int ne, int capacity, hipStream_t s) {
+  hipLaunchKernelGGL(dev::snapshot_node0<dev::PackedSrc>, dim3(1), dim3(256), 0, s,
+                     dev::PackedSrc{src, place}, hist, counter, ne, capacity);
   return hipGetLastError();
 }
 
 hipError_t LaunchSnapshotMean(const double* src, const int* member_offsets, int members,
                               double* hist, int* counter, int ne, int capacity, hipStream_t s) {
-  hipLaunchKernelGGL(dev::snapshot_mean, dim3(ne), dim3(256), 0, s, src, member_offsets, members,
-                     hist, counter, ne, capacity);
+  hipLaunchKernelGGL(dev::snapshot_mean<dev::FullSrc>, dim3(ne), dim3(256), 0, s,
+                     dev::FullSrc{src}, member_offsets, members, hist, counter, ne, capacity);
+  hipLaunchKernelGGL(dev::bump_counter, dim3(1), dim3(1), 0, s, counter);
+  return hipGetLastError();
+}
+
+hipError_t LaunchSnapshotMeanPacked(const double* src, const int* place,
+                                    const int* member_offsets, int members, double* hist,
+                                    int* counter, int ne, int capacity, hipStream_t s) {
+  hipLaunchKernelGGL(dev::snapshot_mean<dev::PackedSrc>, dim3(ne), dim3(256), 0, s,
+                     dev::PackedSrc{src, place}, member_offsets, members, hist, counter, ne,
+                     capacity);
   hipLaunchKernelGGL(dev::bump_counter, dim3(1), dim3(1), 0, s, counter);
   return hipGetLastError();
 }
@@ -806,8 +939,17 @@ hipError_t LaunchGatherNode0(const double* src, const int* member_offsets, int m
                              double* dst, hipStream_t s) {
   const long long n = (long long)members * ne;
   const int blocks = (int)std::min<long long>((n + 255) / 256, 4096);
-  hipLaunchKernelGGL(dev::gather_node0, dim3(blocks), dim3(256), 0, s, src, member_offsets,
-                     members, ne, dst);
+  hipLaunchKernelGGL(dev::gather_node0<dev::FullSrc>, dim3(blocks), dim3(256), 0, s,
+                     dev::FullSrc{src}, member_offsets, members, ne, dst);
+  return hipGetLastError();
+}
+
+hipError_t LaunchGatherNode0Packed(const double* src, const int* place, const int* member_offsets,
+                                   int members, int ne, double* dst, hipStream_t s) {
+  const long long n = (long long)members * ne;
+  const int blocks = (int)std::min<long long>((n + 255) / 256, 4096);
+  hipLaunchKernelGGL(dev::gather_node0<dev::PackedSrc>, dim3(blocks), dim3(256), 0, s,
+                     dev::PackedSrc{src, place}, member_offsets, members, ne, dst);
   return hipGetLastError();
 }
 

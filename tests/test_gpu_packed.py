@@ -1,0 +1,174 @@
+"""The packed Hermitian stage kernels (RK4 increment form and RKF45 of
+Hermitian states) against the full-layout kernels (classic order) and the
+oracle: block edges of the packed order, one and two modes per site, real
+and complex H, single tiles and long tile sequences, ensembles, and the
+changes between the two state layouts."""
+
+import os
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
+
+import phi_amd as P  # noqa: E402
+from oracle import heom_oracle as HO  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+# One step of either form is the same polynomial; with |dt L| < 1 the FP64
+# results differ by a few ulp of the largest entry per step (FP32 bulk: of
+# the increments, which are below the state).
+TOL = {"fp64": 1e-13, "fp32": 2e-6}
+
+
+def problem(N, lh, terms, complex_h, seed=0):
+    rng = np.random.default_rng([seed, N, lh, terms])
+    H = rng.normal(0.0, 0.4, (N, N))
+    H = H + H.T + 0j
+    if complex_h:
+        A = rng.normal(0.0, 0.3, (N, N))
+        H = H + 1j * (A - A.T)
+    g = rng.normal(size=(N, N)) + 1j * rng.normal(size=(N, N))
+    rho0 = g @ g.conj().T
+    rho0 = (rho0 + rho0.conj().T) / 2
+    rho0 /= np.trace(rho0).real
+    kw = dict(gamma=[1.0 + 0.1 * i for i in range(N)], lambda_=[0.05] * N, temperature=0.7,
+              lh=lh, num_terms=terms)
+    return H, rho0, kw
+
+
+def context(H, rho0, kw, precision):
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    ctx = P.Context(p, precision=precision)
+    rng = np.random.default_rng(5)
+    x = rng.normal(size=(ctx.num_nodes,) + H.shape) + 1j * rng.normal(
+        size=(ctx.num_nodes,) + H.shape)
+    x = (x + x.conj().transpose(0, 2, 1)) / 2
+    return ctx, x / np.abs(x).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,lh,terms,complex_h", [
+    (4, 5, 1, False), (4, 4, 2, True), (5, 4, 1, True), (7, 5, 1, False), (7, 3, 2, False),
+    (8, 4, 1, False), (9, 3, 2, True), (13, 3, 1, False), (16, 3, 1, False), (17, 3, 1, True),
+    (24, 2, 1, False), (24, 3, 1, False)])
+def test_packed_steps_equal_the_full_layout(N, lh, terms, complex_h, precision):
+    H, rho0, kw = problem(N, lh, terms, complex_h)
+    ctx, x = context(H, rho0, kw, precision)
+    ctx.set_state(x)
+    assert np.array_equal(ctx.state(), x)
+    hist = ctx.rk4_history(7, 0.01, 3)
+    got = ctx.state()
+    ctx.set_rk4_form("classic")
+    ctx.set_state(x)
+    ref_hist = ctx.rk4_history(7, 0.01, 3)
+    ref = ctx.state()
+    tol = TOL[precision]
+    print(N, lh, terms, precision, np.abs(got - ref).max(), flush=True)
+    assert np.abs(got - ref).max() <= tol * 7
+    assert np.abs(hist - ref_hist).max() <= tol * 7
+    # exactly Hermitian, rho0 read from either layout alike
+    assert np.array_equal(got, got.conj().transpose(0, 2, 1))
+    assert np.array_equal(ctx.rho0(), ref[0])
+
+
+@pytest.mark.parametrize("tile,threads,blocks", [(1, 0, 0), (1, 0, 3), (3, 0, 5), (9, 0, 2),
+                                                 (10, 256, 3), (16, 256, 1), (20, 0, 7)])
+def test_tile_sequences(tile, threads, blocks):
+    H, rho0, kw = problem(7, 5, 1, False)
+    ctx, x = context(H, rho0, kw, "fp64")
+    ctx.set_state(x)
+    ctx.rk4_steps(3, 0.01)
+    ref = ctx.state()
+    ctx.set_launch(2, tile, threads, blocks)
+    ctx.set_state(x)
+    ctx.rk4_steps(3, 0.01)
+    assert np.abs(ctx.state() - ref).max() <= 3e-14
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,terms,depths,blocks", [
+    (5, 1, [3, 6, 4, 2, 5], 0), (7, 1, [5, 3, 6, 2], 11), (4, 2, [4, 3, 5], 2),
+    (7, 1, [6] * 6 + [3] * 5, 24)])
+def test_ensemble_members_equal_single_runs(N, terms, depths, blocks, precision):
+    Hs = []
+    for m in range(len(depths)):
+        H, rho0, kw = problem(N, max(depths), terms, m % 2 == 1, seed=m)
+        Hs.append(H)
+    p = P.params_from_problem(Hs[0], rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    ens = P.Ensemble(p, Hs, depths, precision=precision)
+    if blocks:
+        ens.set_launch(2, 2, 0, blocks)   # many tiles and several claims per block
+    ens.rk4_steps(40, 0.01)               # eager head, graph blocks
+    got = ens.member_rho0()
+    for m, (H, d) in enumerate(zip(Hs, depths)):
+        kw["lh"] = d
+        q = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+        ctx = P.Context(q, precision=precision)
+        x = np.zeros((ctx.num_nodes, N, N), dtype=complex)
+        x[0] = rho0
+        ctx.set_state(x)
+        ctx.rk4_steps(40, 0.01)
+        assert np.abs(got[m] - ctx.rho0()).max() <= TOL[precision] * 40
+
+
+def test_a_state_that_is_not_hermitian_takes_the_full_layout():
+    H, rho0, kw = problem(7, 4, 1, False)
+    ctx, x = context(H, rho0, kw, "fp64")
+    x[3, 1, 2] += 0.25j
+    ctx.set_state(x)
+    ctx.rk4_steps(5, 0.01)
+    got = ctx.state()
+    ctx.set_launch(1, 0, 0, 0)            # one-shot kernels: nested order, full layout
+    ctx.set_state(x)
+    ctx.rk4_steps(5, 0.01)
+    assert np.abs(got - ctx.state()).max() <= 1e-13
+    # and a Hermitian state set afterwards is stepped as one again
+    ctx.set_launch()
+    y = (x + x.conj().transpose(0, 2, 1)) / 2
+    ctx.set_state(y)
+    ctx.rk4_steps(5, 0.01)
+    assert np.array_equal(ctx.state(), ctx.state().conj().transpose(0, 2, 1))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_layout_changes_between_calls(precision):
+    """RK4, an RKF45 attempt, an accepted one, the RHS and the autotuner on one
+    context, against the oracle's stepping of the same sequence."""
+    H, rho0, kw = problem(6, 4, 1, False)
+    ctx, _ = context(H, rho0, kw, precision)
+    x = np.zeros((ctx.num_nodes, 6, 6), dtype=complex)
+    x[0] = rho0
+    dt = 0.01
+    b = np.array([2. / 9., 1. / 12., 1. / 4., 69. / 128., -243. / 128., 135. / 64., -17. / 12.,
+                  27. / 4., -27. / 5., 16. / 15., 65. / 432., -5. / 16., 13. / 16., 4. / 27.,
+                  5. / 144., 1. / 9., 9. / 20., 16. / 45., 1. / 12., 47. / 450., 12. / 25.,
+                  32. / 225., 1. / 30., 6. / 25.]) * dt
+    ctx.set_state(x)
+    ctx.rk4_steps(2, dt)
+    ctx.rkf45_attempt(b)              # not accepted: the state stays
+    before = ctx.state()
+    ctx.rk4_steps(1, dt)
+    ctx.rkf45_attempt(b)
+    ctx.rkf45_accept()
+    ctx.autotune(dt, steps=1)
+    nodes = ctx.rhs_nodes([0, 3])
+    got = ctx.state()
+    orc = HO.Oracle(HO.Problem(H, rho0, hbar=1.0, kb=1.0, **kw))
+    orc.rk4(2 * dt - dt / 2, dt, 1.0)
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    assert np.abs(before - orc.state()).max() <= tol
+    assert np.abs(nodes - orc.rhs(got)[[0, 3]]).max() <= 1e-12
+
+    def rk4(y):
+        k0 = orc.rhs(y)
+        k1 = orc.rhs(y + dt / 2 * k0)
+        k2 = orc.rhs(y + dt / 2 * k1)
+        k3 = orc.rhs(y + dt * k2)
+        return y + dt / 6 * (k0 + 2 * k1 + 2 * k2 + k3)
+
+    # RK4 and the 5th-order Fehlberg step agree to dt^5 |L|^5 / 120
+    assert np.abs(got - rk4(rk4(orc.state()))).max() <= 1e-9 + tol
