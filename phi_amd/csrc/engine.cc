@@ -451,6 +451,11 @@ void Engine::set_fp32(bool v) { fp32_ = v; }
 namespace {
 // Dynamic LDS a stage-kernel block may take.
 constexpr size_t kLdsBudget = 64 * 1024;
+// Largest stage of the one-workgroup kernel, in clocks of LDS reads.  Both
+// ways of stepping, us a step: dimer of 495 nodes (FP64, 2 228 clocks) 8.8
+// against 17.5 on the stage kernels, 84 6-site nodes (3 528) 9.7 against 16.4,
+// 66 10-site nodes (FP32, 5 445) 17.8 against 14.9.
+constexpr double kResidentReads = 4000;
 }  // namespace
 
 int Engine::StreamThreads(int t, bool fp32, int threads, int* th) {
@@ -476,6 +481,7 @@ int Engine::StreamThreads(int t, bool fp32, int threads, int* th) {
 
 int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
   RhsArgs a = args_;
+  const bool by_default = col_nm < 0 && tile == 0 && threads == 0 && blocks == 0;
   const int N = h_.N, D = h_.D, L = h_.L, NE = N * N;
   const bool stream_ok = N <= 32 && mps_ <= 2 && d_edge_ != nullptr;
   if (col_nm < 0) {
@@ -547,6 +553,7 @@ int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
   a.col_nm = col_nm;
   a.tile = a.col_tile[0];
   args_ = a;
+  default_shape_ = by_default;
   for (int f = 0; f < 2; ++f)
     for (int s = 0; s < 4; ++s) {
       stage_threads_[f][s] = a.col_threads[f];
@@ -581,6 +588,7 @@ int Engine::SetStageLaunch(int stage, int threads, int blocks) {
     stage_threads_[f][stage] = th[f];
     stage_grid_[f][stage] = blocks;
   }
+  default_shape_ = false;
   return kOk;
 }
 
@@ -648,6 +656,33 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   if (rc) return rc;
   const int N = h_.N, NE = N * N;
   const int f = fp32_ ? 1 : 0;
+  if (ResidentForm()) {
+    // One launch of one workgroup: there is no shape to choose.
+    rc = EnterState(true);
+    if (rc) return rc;
+    if (packed_) {
+      const size_t bytes = StateBytes();
+      double* saved = nullptr;
+      rc = Check(hipMalloc((void**)&saved, bytes), "alloc tune state");
+      if (!rc) rc = Check(hipMemcpyAsync(saved, StateBuf(), bytes, hipMemcpyDeviceToDevice,
+                                         stream_), "save state");
+      double ms = 0;
+      if (!rc) rc = Rk4StepsTimed(steps, dt, &ms);
+      full_fresh_ = false;
+      const int rs = saved ? Check(hipMemcpyAsync(StateBuf(), saved, bytes,
+                                                  hipMemcpyDeviceToDevice, stream_),
+                                   "restore state") : kOk;
+      const int ry = Synchronize();
+      Free(saved);
+      if (rc || rs || ry) return rc ? rc : rs ? rs : ry;
+      *best_ms = ms / steps;
+      shape_out[0] = args_.col_nm;
+      shape_out[1] = args_.col_tile[f];
+      shape_out[2] = args_.col_threads[f];
+      shape_out[3] = args_.col_grid[f];
+      return kOk;
+    }
+  }
   int dev = 0;
   (void)hipGetDevice(&dev);
   const TuneKey key{dev, N, h_.D, h_.L, slab_nodes_, mps_, members_, fp32_, rk4_form_};
@@ -859,19 +894,34 @@ int Engine::AllocBulk() {
   return kOk;
 }
 
+bool Engine::PackedLayout() const {
+  // 32-bit byte offsets from a member's first node, 24-bit node ids.
+  if (!d_elem_ || !d_edge_ || h_.num_nodes >= (1 << 24)) return false;
+  const long long nodes = members_ ? h_.num_nodes : slab_nodes_;
+  return (nodes + kPackedPad) * h_.N * h_.N * (long long)sizeof(double) < (1LL << 32);
+}
+
 bool Engine::PackedUsable() const {
   const int f = fp32_ ? 1 : 0;
   // Below 4 sites the diagonal, whose elements take both sides' gathers for
   // half the data, outweighs the pairs: 55 members of 3 sites 41 us a step
   // on the full kernels, 50 packed; 96 members of 4 sites 46 and 46.
-  if (h_.N < 4) return false;
-  // 32-bit byte offsets from a member's first node, 24-bit node ids, and no
-  // more LDS than the other kernels take.
-  if (!d_elem_ || !d_edge_ || h_.num_nodes >= (1 << 24)) return false;
-  const long long nodes = members_ ? h_.num_nodes : slab_nodes_;
-  if ((nodes + kPackedPad) * h_.N * h_.N * (long long)sizeof(double) >= (1LL << 32)) return false;
+  if (h_.N < 4 || !PackedLayout()) return false;
   if (args_.col_nm != 2) return true;
+  // no more LDS than the other kernels take
   return PackedTileLdsBytes(h_.N, h_.D, h_.L, mps_, args_.pk_tile[f], f == 1) <= kLdsBudget;
+}
+
+bool Engine::ResidentForm() const {
+  if (members_ || closure_ || !default_shape_ || args_.col_nm != 2 ||
+      rk4_form_ != kRk4Increment || !PackedLayout() || !ResidentFits(args_, fp32_))
+    return false;
+  // One workgroup's LDS reads of a stage (4 gathers per mode slot and 2 N
+  // matrix elements, both ways through 128 bytes a clock) against the stage
+  // kernels' launches.
+  const double reads = (double)h_.num_nodes * args_.PE * (4.0 * mps_ + 2.0 * h_.N) *
+                       (fp32_ ? sizeof(float2) : sizeof(double2)) / 128.0;
+  return reads <= kResidentReads;
 }
 
 int Engine::UseFull() {
@@ -1167,8 +1217,19 @@ int Engine::Rk4Steps(long long nsteps, double dt, long long step_offset, int sna
     last_eager_steps_ = nsteps;
     return rc;
   }
-  rc = EnterState(PackedForm());
+  const bool resident = ResidentForm();
+  rc = EnterState(resident || PackedForm());
   if (rc) return rc;
+  if (resident && packed_) {
+    // at most 4096 steps (some 20 ms) a launch
+    for (long long s = 0; s < nsteps && !rc; s += 4096)
+      rc = Check(LaunchResidentRk4(args_, fp32_, d_prho_, std::min(nsteps - s, 4096LL), dt,
+                                   step_offset + s, snap_every, d_hist_, d_hist_count_,
+                                   hist_capacity_, stream_), "rk4 steps");
+    full_fresh_ = false;
+    last_eager_steps_ = nsteps;
+    return rc;
+  }
   // Graph blocks of G steps, G a multiple of the snapshot period, aligned so
   // that every block starts on a snapshot step.
   int G = 0;

@@ -374,10 +374,14 @@ class Engine {
   double* d_pnew_ = nullptr;    // RKF45 5th-order solution
   size_t prho_reals_ = 0;       // reals d_prho_ and d_pnew_ were allocated for
   bool packed_ = false, full_fresh_ = false, not_hermitian_ = false, attempt_packed_ = false;
-  bool PackedUsable() const;    // sizes fit the packed kernels in this precision
+  bool PackedLayout() const;    // the packed layout's offsets fit
+  bool PackedUsable() const;    // and its stage kernels serve this system in this precision
   bool PackedForm() const {     // RK4 steps would take the packed kernels now
     return PackedUsable() && !closure_ && args_.col_nm == 2 && rk4_form_ == kRk4Increment;
   }
+  bool default_shape_ = true;   // no shape was asked for (SetLaunch(-1, 0, 0, 0))
+  // A small single hierarchy's increment-form steps inside one workgroup.
+  bool ResidentForm() const;
   bool RunsPacked() const { return packed_ && PackedForm(); }  // an RK4 step launched now
   int ActiveTile() const {
     const int f = fp32_ ? 1 : 0;

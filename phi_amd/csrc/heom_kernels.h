@@ -127,6 +127,13 @@ hipError_t LaunchRkf45Packed(const RhsArgs& a, bool fp32, int stage, const void*
 // hfrag (members x fragment elements, complex of the bulk precision) from a.H.
 size_t PackedFragElems(int N);
 hipError_t LaunchBuildFrag(const RhsArgs& a, bool fp32, int members, void* out, hipStream_t s);
+// A small hierarchy's steps inside one workgroup (heom_resident.hip): whether
+// it fits, and nsteps steps of the packed state rho in one launch, recording
+// node 0 after every step i with (step_offset + i) % snap_every == 0.
+bool ResidentFits(const RhsArgs& a, bool fp32);
+hipError_t LaunchResidentRk4(const RhsArgs& a, bool fp32, double* rho, long long nsteps,
+                             double dt, long long step_offset, int snap_every, double* hist,
+                             int* counter, int capacity, hipStream_t s);
 // packed <- full; *flag (zeroed before) = 1 unless every ADO equals its
 // conjugate transpose exactly.
 hipError_t LaunchPack(const RhsArgs& a, int nodes, const double* full, double* packed, int* flag,

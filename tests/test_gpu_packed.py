@@ -172,3 +172,42 @@ def test_layout_changes_between_calls(precision):
 
     # RK4 and the 5th-order Fehlberg step agree to dt^5 |L|^5 / 120
     assert np.abs(got - rk4(rk4(orc.state()))).max() <= 1e-9 + tol
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,lh,terms,complex_h", [
+    (1, 9, 1, False), (2, 9, 2, False), (2, 2, 1, True), (3, 4, 2, True), (3, 8, 1, False),
+    (4, 6, 1, True), (5, 3, 2, False), (7, 3, 1, False), (8, 2, 1, True)])
+def test_one_workgroup_steps_equal_the_stage_kernels(N, lh, terms, complex_h, precision):
+    H, rho0, kw = problem(N, lh, terms, complex_h, seed=3)
+    ctx, x = context(H, rho0, kw, precision)
+    ctx.set_state(x)
+    hist = ctx.rk4_history(23, 0.01, 4)
+    ctx.rk4_steps(1, 0.01)
+    got = ctx.state()
+    ctx.set_rk4_form("classic")           # the full-layout stage kernels
+    ctx.set_state(x)
+    ref_hist = ctx.rk4_history(23, 0.01, 4)
+    ctx.rk4_steps(1, 0.01)
+    tol = TOL[precision] * 24
+    assert hist.shape == ref_hist.shape == (6, N, N)
+    assert np.abs(hist - ref_hist).max() <= tol
+    assert np.abs(got - ctx.state()).max() <= tol
+    assert np.array_equal(got, got.conj().transpose(0, 2, 1))
+
+
+def test_one_workgroup_runs_longer_than_a_launch_match_the_oracle():
+    """5000 steps (two launches) and the autotuner, which leaves the state."""
+    H, rho0, kw = problem(2, 4, 1, False, seed=4)
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, **kw)
+    ctx = P.Context(p)
+    x = np.zeros((ctx.num_nodes, 2, 2), dtype=complex)
+    x[0] = rho0
+    ctx.set_state(x)
+    ms, shape = ctx.autotune(0.001, steps=5)
+    assert ms > 0 and np.array_equal(ctx.state(), x)
+    hist = ctx.rk4_history(5000, 0.001, 500)
+    assert hist.shape[0] == 10
+    orc = HO.Oracle(HO.Problem(H, rho0, hbar=1.0, kb=1.0, **kw))
+    orc.rk4(5.0 - 0.0005, 0.001, 10.0)
+    assert np.abs(ctx.state() - orc.state()).max() <= 1e-10
