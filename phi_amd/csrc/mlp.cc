@@ -65,10 +65,6 @@ int Mlp::Create(int n_in, int n_hidden, int n_out, int max_batch, Mlp** out, std
     if (!rc) rc = m->Check(hipMalloc((void**)b, hb), "alloc activations");
   if (!rc) rc = m->Check(hipMalloc((void**)&m->d_y_, (size_t)max_batch * n_out * 4), "alloc y");
   if (!rc) rc = m->Check(hipMalloc((void**)&m->d_dy_, (size_t)max_batch * n_out * 4), "alloc dy");
-  m->partial_slots_ = 1;
-  if (!rc)
-    rc = m->Check(hipMalloc((void**)&m->d_partial_, m->partial_blocks_ * sizeof(double)),
-                  "alloc partial");
   if (rc) {
     *why = m->err_;
     delete m;
@@ -178,43 +174,47 @@ int Mlp::GetParams(float* flat) {
   return rc ? rc : Check(hipStreamSynchronize(stream_), "sync");
 }
 
-// The three layers for `batch` rows of x; activations kept for backward.
-int Mlp::ForwardBatch(const float* x, int batch, float* y, hipStream_t s) {
+// The three layers for `batch` rows of x (rows: the minibatch's rows of x, or
+// null); activations kept for backward.  With a target t, the last layer
+// leaves the loss gradient in y and its loss partials in `partial`.
+int Mlp::ForwardBatch(const float* x, const int* rows, int batch, float* y, hipStream_t s,
+                      const float* t, double* partial) {
   mlp::GemmArgs g{};
   g.M = batch;
   g.N = n_hid_;
   g.K = n_in_;
   g.A = x;
-  g.sa_i = n_in_;
-  g.sa_k = 1;
+  g.lda = n_in_;
+  g.rows = rows;
   g.B = d_p_ + off_[0];
-  g.sb_k = 1;
-  g.sb_j = n_in_;
+  g.ldb = n_in_;
   g.C = d_h1_;
-  g.sc_i = n_hid_;
+  g.ldc = n_hid_;
   g.bias = d_p_ + off_[1];
   g.Z = d_z1_;
-  g.gelu = 1;
-  int rc = Check(LaunchGemmBf16(g, s), "layer 1");
+  int rc = Check(LaunchLayer(g, mlp::kGelu, s), "layer 1");
   g.K = n_hid_;
   g.A = d_h1_;
-  g.sa_i = n_hid_;
+  g.lda = n_hid_;
+  g.rows = nullptr;
   g.B = d_p_ + off_[2];
-  g.sb_j = n_hid_;
+  g.ldb = n_hid_;
   g.C = d_h2_;
   g.bias = d_p_ + off_[3];
   g.Z = d_z2_;
-  if (!rc) rc = Check(LaunchGemmBf16(g, s), "layer 2");
+  if (!rc) rc = Check(LaunchLayer(g, mlp::kGelu, s), "layer 2");
   g.N = n_out_;
   g.A = d_h2_;
   g.B = d_p_ + off_[4];
-  g.sb_j = n_hid_;
   g.C = y;
-  g.sc_i = n_out_;
+  g.ldc = n_out_;
   g.bias = d_p_ + off_[5];
   g.Z = nullptr;
-  g.gelu = 0;
-  if (!rc) rc = Check(LaunchGemmBf16(g, s), "layer 3");
+  g.rows = rows;
+  g.T = t;
+  g.scale = 2.0f / (float)((long long)batch * n_out_);
+  g.partial = partial;
+  if (!rc) rc = Check(LaunchLayer(g, t ? mlp::kMseGrad : mlp::kBias, s), "layer 3");
   return rc;
 }
 
@@ -222,7 +222,7 @@ int Mlp::ForwardDevice(const float* x, int batch, float* y, hipStream_t s) {
   int rc = 0;
   for (int r0 = 0; r0 < batch && !rc; r0 += max_batch_) {
     const int b = std::min(max_batch_, batch - r0);
-    rc = ForwardBatch(x + (size_t)r0 * n_in_, b, y + (size_t)r0 * n_out_, s);
+    rc = ForwardBatch(x + (size_t)r0 * n_in_, nullptr, b, y + (size_t)r0 * n_out_, s, nullptr, nullptr);
   }
   return rc;
 }
@@ -234,68 +234,69 @@ int Mlp::Forward(const float* x, int batch, float* y) {
   }
   int rc = Check(hipMemcpyAsync(d_x_, x, (size_t)batch * n_in_ * 4, hipMemcpyHostToDevice,
                                 stream_), "upload x");
-  if (!rc) rc = ForwardBatch(d_x_, batch, d_y_, stream_);
+  if (!rc) rc = ForwardBatch(d_x_, nullptr, batch, d_y_, stream_, nullptr, nullptr);
   if (!rc) rc = Check(hipMemcpyAsync(y, d_y_, (size_t)batch * n_out_ * 4, hipMemcpyDeviceToHost,
                                      stream_), "download y");
   if (!rc) rc = Check(hipStreamSynchronize(stream_), "sync");
   return rc;
 }
 
-// Gradients of the batch in d_x_/d_t_ into d_g_; the loss partial sums of
-// the batch go to partial slot `slot`.
-int Mlp::BackwardBatch(const float* x, const float* t, int batch, int slot) {
+// Forward and backward of a minibatch (rows of x and t, or null): the
+// gradients go to d_g_, or, with adam, straight into an Adam step of the
+// parameters (the weight gradients run last, after every use of the
+// weights); the loss partial sums to `partial` (LayerBlocks of them).
+int Mlp::BackwardBatch(const float* x, const float* t, const int* rows, int batch,
+                       double* partial, const mlp::AdamArgs* adam) {
   hipStream_t s = stream_;
-  int rc = ForwardBatch(x, batch, d_y_, s);
-  const long long ny = (long long)batch * n_out_;
-  if (!rc)
-    rc = Check(LaunchMseGrad(d_y_, t, d_dy_, ny, d_partial_ + (size_t)slot * partial_blocks_,
-                             partial_blocks_, s), "loss");
-  // Layer 3: dW3 = dY^T H2, db3 = colsum dY, dH2 = dY W3.
-  mlp::GemmArgs g{};
-  auto weight_grad = [&](const float* dz, int nout, const float* h, int nin, long long woff) {
-    mlp::GemmArgs w{};
-    w.M = nout;
-    w.N = nin;
-    w.K = batch;
-    w.A = dz;
-    w.sa_i = 1;
-    w.sa_k = nout;
-    w.B = h;
-    w.sb_k = nin;
-    w.sb_j = 1;
-    w.C = d_g_ + woff;
-    w.sc_i = nin;
-    return Check(LaunchGemmBf16(w, s), "weight grad");
+  int rc = ForwardBatch(x, rows, batch, d_dy_, s, t, partial);
+  // dZ2 = (dY W3) GELU'(Z2), dZ1 = (dZ2 W2) GELU'(Z1)
+  mlp::GemmArgs a{};
+  a.M = batch;
+  a.N = n_hid_;
+  a.K = n_out_;
+  a.A = d_dy_;
+  a.lda = n_out_;
+  a.B = d_p_ + off_[4];
+  a.ldb = n_hid_;
+  a.C = d_dh2_;
+  a.ldc = n_hid_;
+  a.Z = d_z2_;
+  if (!rc) rc = Check(LaunchInputGrad(a, s), "input grad 2");
+  a.K = n_hid_;
+  a.A = d_dh2_;
+  a.lda = n_hid_;
+  a.B = d_p_ + off_[2];
+  a.C = d_dh1_;
+  a.Z = d_z1_;
+  if (!rc) rc = Check(LaunchInputGrad(a, s), "input grad 1");
+  // dW = dZ^T H, db = column sums of dZ
+  mlp::GemmArgs w[3] = {};
+  auto layer = [&](mlp::GemmArgs& g, const float* dz, int nout, const float* h, int nin,
+                   const int* hrows, long long woff, long long boff) {
+    g.M = nout;
+    g.N = nin;
+    g.K = batch;
+    g.A = dz;
+    g.lda = nout;
+    g.B = h;
+    g.ldb = nin;
+    g.rows = hrows;
+    g.C = d_g_ + woff;
+    g.ldc = nin;
+    g.bias_out = d_g_ + boff;
+    if (adam) {
+      g.p = d_p_ + woff;
+      g.m = d_m_ + woff;
+      g.v = d_v_ + woff;
+      g.bp = d_p_ + boff;
+      g.bm = d_m_ + boff;
+      g.bv = d_v_ + boff;
+    }
   };
-  auto input_grad = [&](const float* dz, int nout, long long woff, int nin, float* dh) {
-    mlp::GemmArgs a{};
-    a.M = batch;
-    a.N = nin;
-    a.K = nout;
-    a.A = dz;
-    a.sa_i = nout;
-    a.sa_k = 1;
-    a.B = d_p_ + woff;
-    a.sb_k = nin;
-    a.sb_j = 1;
-    a.C = dh;
-    a.sc_i = nin;
-    return Check(LaunchGemmBf16(a, s), "input grad");
-  };
-  (void)g;
-  if (!rc) rc = weight_grad(d_dy_, n_out_, d_h2_, n_hid_, off_[4]);
-  if (!rc) rc = Check(LaunchColumnSums(d_dy_, batch, n_out_, n_out_, d_g_ + off_[5], s), "db3");
-  if (!rc) rc = input_grad(d_dy_, n_out_, off_[4], n_hid_, d_dh2_);
-  // Layer 2.
-  const long long nh = (long long)batch * n_hid_;
-  if (!rc) rc = Check(LaunchGeluBackward(d_dh2_, d_z2_, d_dh2_, nh, s), "gelu 2");
-  if (!rc) rc = weight_grad(d_dh2_, n_hid_, d_h1_, n_hid_, off_[2]);
-  if (!rc) rc = Check(LaunchColumnSums(d_dh2_, batch, n_hid_, n_hid_, d_g_ + off_[3], s), "db2");
-  if (!rc) rc = input_grad(d_dh2_, n_hid_, off_[2], n_hid_, d_dh1_);
-  // Layer 1.
-  if (!rc) rc = Check(LaunchGeluBackward(d_dh1_, d_z1_, d_dh1_, nh, s), "gelu 1");
-  if (!rc) rc = weight_grad(d_dh1_, n_hid_, x, n_in_, off_[0]);
-  if (!rc) rc = Check(LaunchColumnSums(d_dh1_, batch, n_hid_, n_hid_, d_g_ + off_[1], s), "db1");
+  layer(w[0], d_dy_, n_out_, d_h2_, n_hid_, nullptr, off_[4], off_[5]);
+  layer(w[1], d_dh2_, n_hid_, d_h1_, n_hid_, nullptr, off_[2], off_[3]);
+  layer(w[2], d_dh1_, n_hid_, x, n_in_, rows, off_[0], off_[1]);
+  if (!rc) rc = Check(LaunchWeightGrads(w, 3, adam ? *adam : mlp::AdamArgs{}, s), "weight grads");
   return rc;
 }
 
@@ -308,8 +309,10 @@ int Mlp::Gradients(const float* x, const float* t, int batch, double* loss, floa
                                 stream_), "upload x");
   if (!rc) rc = Check(hipMemcpyAsync(d_t_, t, (size_t)batch * n_out_ * 4, hipMemcpyHostToDevice,
                                      stream_), "upload t");
-  if (!rc) rc = BackwardBatch(d_x_, d_t_, batch, 0);
-  std::vector<double> part(partial_blocks_);
+  const int blocks = LayerBlocks(batch, n_out_);
+  if (!rc) rc = EnsurePartials(blocks);
+  if (!rc) rc = BackwardBatch(d_x_, d_t_, nullptr, batch, d_partial_, nullptr);
+  std::vector<double> part(blocks);
   if (!rc) rc = Check(hipMemcpyAsync(part.data(), d_partial_, part.size() * sizeof(double),
                                      hipMemcpyDeviceToHost, stream_), "loss");
   if (!rc) rc = Check(hipMemcpyAsync(grads, d_g_, nparam_ * sizeof(float), hipMemcpyDeviceToHost,
@@ -323,14 +326,23 @@ int Mlp::Gradients(const float* x, const float* t, int batch, double* loss, floa
   return rc;
 }
 
-int Mlp::AdamStep(float lr) {
+mlp::AdamArgs Mlp::NextAdam(float lr) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   ++adam_t_;
   const double c1 = 1.0 - std::pow((double)b1, adam_t_);
   const double c2 = 1.0 - std::pow((double)b2, adam_t_);
-  const float lr_t = (float)(lr * std::sqrt(c2) / c1);
-  const float eps_t = (float)(eps * std::sqrt(c2));
-  return Check(LaunchAdam(d_p_, d_g_, d_m_, d_v_, nparam_, lr_t, b1, b2, eps_t, stream_), "adam");
+  return mlp::AdamArgs{(float)(lr * std::sqrt(c2) / c1), b1, b2, (float)(eps * std::sqrt(c2))};
+}
+
+int Mlp::EnsurePartials(long long n) {
+  if (partial_cap_ >= n) return 0;
+  FreeDev(d_partial_);
+  d_partial_ = nullptr;
+  partial_cap_ = 0;
+  const int rc = Check(hipMalloc((void**)&d_partial_, (size_t)n * sizeof(double)),
+                       "alloc partials");
+  if (!rc) partial_cap_ = n;
+  return rc;
 }
 
 int Mlp::Train(const float* X, const float* T, long long samples, int batch, int epochs,
@@ -353,17 +365,12 @@ int Mlp::Train(const float* X, const float* T, long long samples, int batch, int
                                      stream_), "upload data x");
   if (!rc) rc = Check(hipMemcpyAsync(dT, T, (size_t)samples * n_out_ * 4, hipMemcpyHostToDevice,
                                      stream_), "upload data t");
-  // One partial-sum slot per batch of an epoch.
-  if (!rc && partial_slots_ < nb) {
-    FreeDev(d_partial_);
-    d_partial_ = nullptr;
-    rc = Check(hipMalloc((void**)&d_partial_, (size_t)nb * partial_blocks_ * sizeof(double)),
-               "alloc partials");
-    partial_slots_ = rc ? 0 : (int)nb;
-  }
+  // The loss partials of every batch of an epoch.
+  const int blocks = LayerBlocks(batch, n_out_);
+  if (!rc) rc = EnsurePartials(nb * blocks);
   std::mt19937 gen(seed);
   std::vector<int> perm(samples);
-  std::vector<double> part((size_t)nb * partial_blocks_);
+  std::vector<double> part((size_t)nb * blocks);
   for (int ep = 0; ep < epochs && !rc; ++ep) {
     const float lr_ep = (lr_final > 0 && epochs > 1)
                             ? (float)(lr * std::pow((double)lr_final / lr, (double)ep / (epochs - 1)))
@@ -373,11 +380,8 @@ int Mlp::Train(const float* X, const float* T, long long samples, int batch, int
     rc = Check(hipMemcpyAsync(dIdx, perm.data(), perm.size() * sizeof(int),
                               hipMemcpyHostToDevice, stream_), "upload permutation");
     for (long long b = 0; b < nb && !rc; ++b) {
-      rc = Check(LaunchGatherRows(dX, dIdx + b * batch, batch, n_in_, d_x_, stream_), "gather x");
-      if (!rc) rc = Check(LaunchGatherRows(dT, dIdx + b * batch, batch, n_out_, d_t_, stream_),
-                          "gather t");
-      if (!rc) rc = BackwardBatch(d_x_, d_t_, batch, (int)b);
-      if (!rc) rc = AdamStep(lr_ep);
+      const mlp::AdamArgs adam = NextAdam(lr_ep);
+      rc = BackwardBatch(dX, dT, dIdx + b * batch, batch, d_partial_ + b * blocks, &adam);
     }
     if (!rc) rc = Check(hipMemcpyAsync(part.data(), d_partial_, part.size() * sizeof(double),
                                        hipMemcpyDeviceToHost, stream_), "epoch loss");

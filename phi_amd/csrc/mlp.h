@@ -59,9 +59,12 @@ class Mlp {
  private:
   Mlp() = default;
   int Check(hipError_t e, const char* where);
-  int ForwardBatch(const float* x, int batch, float* y, hipStream_t s);
-  int BackwardBatch(const float* x, const float* t, int batch, int partial_slot);
-  int AdamStep(float lr);
+  int ForwardBatch(const float* x, const int* rows, int batch, float* y, hipStream_t s,
+                   const float* t, double* partial);
+  int BackwardBatch(const float* x, const float* t, const int* rows, int batch, double* partial,
+                    const mlp::AdamArgs* adam);
+  mlp::AdamArgs NextAdam(float lr);
+  int EnsurePartials(long long n);
 
   int n_in_ = 0, n_hid_ = 0, n_out_ = 0, max_batch_ = 0;
   long long nparam_ = 0;
@@ -77,8 +80,7 @@ class Mlp {
   float *d_z1_ = nullptr, *d_h1_ = nullptr, *d_z2_ = nullptr, *d_h2_ = nullptr, *d_y_ = nullptr;
   float *d_dy_ = nullptr, *d_dh2_ = nullptr, *d_dh1_ = nullptr;
   double* d_partial_ = nullptr;
-  int partial_blocks_ = 64;
-  int partial_slots_ = 0;
+  long long partial_cap_ = 0;  // doubles in d_partial_
 };
 
 }  // namespace phi

@@ -7,36 +7,55 @@
 namespace phi {
 namespace mlp {
 
-// C(i, j) = sum_k A(i, k) B(k, j) (+ bias[j]) for i < M, j < N, k < K with
-// A(i, k) = A[i*sa_i + k*sa_k], B(k, j) = B[k*sb_k + j*sb_j], C(i, j) at
-// C[i*sc_i + j].  gelu: Z = pre-activation, C = GELU(Z); accumulate: C +=.
+// What a product's epilogue does with acc(i, j) = sum_k A(i, k) B(k, j).
+enum Epilogue {
+  kBias = 0,      // C = acc + bias[j]
+  kGelu,          // Z = acc + bias[j], C = GELU(Z)
+  kMseGrad,       // d = acc + bias[j] - T(row i, j): C = scale d, loss partials of d^2
+  kGeluGrad,      // C = acc GELU'(Z)
+  kWeight         // gradient, and row sums of A as the bias gradient: stored in C and
+                  // bias_out, or (p non-null) taken by an Adam step of p and bias p
+};
+
+struct AdamArgs {
+  float lr_t, beta1, beta2, eps_t;  // bias-corrected step sizes
+};
+
+// Operands: A(i, k) = A[row(i) * lda + k] (layers and input gradients) or
+// A[k * lda + i] (kWeight); B(k, j) = B[j * ldb + k] (layers) or
+// B[row(k) * ldb + j] (gradients).  rows (or null for the identity) gathers
+// minibatch rows out of a data set: of A for a layer, of B for kWeight, of T
+// for kMseGrad.
 struct GemmArgs {
   int M, N, K;
   const float* A;
-  long long sa_i, sa_k;
+  long long lda;
   const float* B;
-  long long sb_k, sb_j;
+  long long ldb;
   float* C;
-  long long sc_i;
+  long long ldc;
+  const int* rows;
   const float* bias;
-  float* Z;
-  int gelu;
-  int accumulate;
+  float* Z;             // ldc apart
+  const float* T;       // kMseGrad: N apart
+  float scale;
+  double* partial;      // kMseGrad: one sum per block
+  float* bias_out;      // kWeight
+  float *p, *m, *v;     // kWeight with Adam: parameters and moments (ldc = N apart)
+  float *bp, *bm, *bv;  // the bias'
 };
 
 }  // namespace mlp
 
-hipError_t LaunchGemmBf16(const mlp::GemmArgs& g, hipStream_t s);
-hipError_t LaunchGeluBackward(const float* dH, const float* Z, float* dZ, long long n,
-                              hipStream_t s);
-hipError_t LaunchColumnSums(const float* X, int rows, int cols, long long ld, float* out,
-                            hipStream_t s);
-hipError_t LaunchMseGrad(const float* Y, const float* T, float* dY, long long n, double* partial,
-                         int blocks, hipStream_t s);
-hipError_t LaunchAdam(float* p, const float* g, float* m, float* v, long long n, float lr_t,
-                      float beta1, float beta2, float eps_t, hipStream_t s);
-hipError_t LaunchGatherRows(const float* src, const int* index, int rows, int cols, float* dst,
-                            hipStream_t s);
+// Blocks of a layer (one loss partial each for kMseGrad).
+int LayerBlocks(int M, int N);
+// Layers: kBias, kGelu, kMseGrad.
+hipError_t LaunchLayer(const mlp::GemmArgs& g, mlp::Epilogue e, hipStream_t s);
+// kGeluGrad: input gradient dZ W through the previous layer's GELU.
+hipError_t LaunchInputGrad(const mlp::GemmArgs& g, hipStream_t s);
+// kWeight: up to three layers' weight and bias gradients in one launch.
+hipError_t LaunchWeightGrads(const mlp::GemmArgs* g, int count, const mlp::AdamArgs& adam,
+                             hipStream_t s);
 
 }  // namespace phi
 

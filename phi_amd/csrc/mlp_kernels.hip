@@ -1,11 +1,10 @@
 // Kernels of the truncation-closure network (gfx950): bfloat16 matrix-core
-// GEMMs with float32 accumulation, GELU, the squared-error loss, Adam, and
-// the fused inference pass that feeds the HEOM stage kernels.
+// products with float32 accumulation whose epilogues are GELU, the
+// squared-error loss, the gradients and Adam.
 //
 // Storage: float32 everywhere in HBM (weights (out, in) row-major,
-// activations (batch, features) row-major); GEMM operands are rounded to
-// bfloat16 (nearest even) when staged into LDS, products accumulate in
-// float32 on v_mfma_f32_16x16x32_bf16.
+// activations (batch, features) row-major); operands are rounded to bfloat16
+// (nearest even) when loaded, products accumulate in float32.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -21,248 +20,255 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 using act::gelu;
 using act::gelu_grad;
-using act::to_bf16;
 
-// --- Strided GEMM -----------------------------------------------------------------
-// C(i, j) = sum_k A(i, k) B(k, j), A(i, k) = A[i*sa_i + k*sa_k],
-// B(k, j) = B[k*sb_k + j*sb_j].  Block tile 64 x 64, K step 32, four
-// wavefronts of 32 x 32 (2 x 2 MFMA tiles of 16 x 16).  Lane l of
-// v_mfma_f32_16x16x32_bf16 holds A[l%16][8(l/16) .. 8(l/16)+7] and
+// --- Products ----------------------------------------------------------------------
+// The network's products are small (512 x 256 x 105 up to 686 x 256 x 512):
+// what bounds them is latency and launches, not the matrix cores (a training
+// step's 0.8 GFLOP is under 1 us of them) or bytes (all operands stay in L2).
+// So a wave takes a 32 x 32 tile straight from global memory into MFMA
+// fragments, with no LDS and no barrier in the loop.  The layers accumulate
+// over K in order (the fused closure pass does, and evaluates the same
+// function to the bit): a block's four waves own four tiles.  The gradients'
+// longer sums (K = outputs or batch rows) are split: the four waves take the
+// K steps w, w + 4, ... of one tile and are added through LDS in wave order
+// (deterministic).  The epilogue does what would be further launches: bias,
+// GELU, the loss and its gradient, GELU', the bias gradient (row sums of the
+// FP32 A operand) and Adam.  A training step of batch 512 is 6 launches
+// instead of 17.
+//
+// v_mfma_f32_16x16x32_bf16: lane l holds A[l%16][8(l/16) .. +7] and
 // B[8(l/16) .. +7][l%16]; output register r holds D[4(l/16) + r][l%16].
-// The next K step's operands load into registers while the current one is
-// multiplied from LDS (two LDS buffers, one barrier per step); the loads are
-// unconditional (an element outside the matrices reads element 0 and is
-// replaced by zero), so all of a step's loads are in flight at once.
-constexpr int kBM = 64, kBN = 64, kBK = 32, kPad = 8;
-constexpr int kPer = kBM * kBK / 256;  // elements per thread and operand
+// Operands are rounded to bfloat16 (nearest even) as they are loaded.
+constexpr int kTile = 32, kStep = 32;
 
-__global__ void __launch_bounds__(256) gemm_bf16(GemmArgs g) {
-  __shared__ __align__(16) unsigned short As[2][kBM][kBK + kPad];
-  __shared__ __align__(16) unsigned short Bs[2][kBN][kBK + kPad];  // Bs[j][k]
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int wm = wave >> 1, wn = wave & 1;
+typedef float F4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight consecutive k of one row r (k contiguous): two 16-byte loads where
+// the whole step is inside K, else masked elements.
+__device__ __forceinline__ void load_rowk(const float* p, int k, int K, bool whole, float* v) {
+  if (whole) {
+    const F4u a = *reinterpret_cast<const F4u*>(p + k);
+    const F4u b = *reinterpret_cast<const F4u*>(p + k + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = p[min(k + e, K - 1)];
+      v[e] = k + e < K ? x : 0.f;
+    }
+  }
+}
+
+// Eight consecutive k of one column c (k strided by ld; rows gathers them).
+__device__ __forceinline__ void load_colk(const float* base, long long ld, const int* rows,
+                                          int c, int k, int K, float* v) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int kk = min(k + e, K - 1);
+    const float x = base[(long long)(rows ? rows[kk] : kk) * ld + c];
+    v[e] = k + e < K ? x : 0.f;
+  }
+}
+
+__device__ __forceinline__ bf16x8 pack8(const float* v) {
+  bf16x8 r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = (__bf16)v[e];
+  return r;
+}
+
+__device__ __forceinline__ void adam_one(float* p, float* m, float* v, long long o, float g,
+                                         const AdamArgs& a) {
+  const float mi = a.beta1 * m[o] + (1.f - a.beta1) * g;
+  const float vi = a.beta2 * v[o] + (1.f - a.beta2) * g * g;
+  m[o] = mi;
+  v[o] = vi;
+  p[o] -= a.lr_t * mi / (sqrtf(vi) + a.eps_t);
+}
+
+template <int EPI>
+__device__ __forceinline__ void product(const GemmArgs& g, int block, const AdamArgs& adam) {
+  __shared__ float part[4][kTile][kTile + 1];
+  __shared__ float bsum[4][4][kTile];
+  constexpr bool kAk = EPI != kWeight;                 // A rows contiguous along k
+  constexpr bool kBk = EPI <= kMseGrad;                // B columns contiguous along k
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int q = lane >> 4, c = lane & 15;
-  const int i0 = blockIdx.y * kBM, j0 = blockIdx.x * kBN;
+  constexpr bool kSplit = EPI > kMseGrad;
+  const int tj = (g.N + kTile - 1) / kTile, tiles = (g.M + kTile - 1) / kTile * tj;
+  const int tile = kSplit ? block : min(4 * block + wave, tiles - 1);
+  const bool live = kSplit || 4 * block + wave < tiles;
+  const int i0 = tile / tj * kTile, j0 = tile % tj * kTile;
+  int ri[2], cj[2];
+  const float *pa[2], *pb[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    // (rows and columns past the matrices repeat the last one; unused)
+    ri[t] = min(i0 + 16 * t + c, g.M - 1);
+    cj[t] = min(j0 + 16 * t + c, g.N - 1);
+    pa[t] = nullptr;
+    pb[t] = nullptr;
+    if constexpr (kAk) {
+      const bool gather = EPI <= kMseGrad && EPI != kMseGrad && g.rows;
+      pa[t] = g.A + (long long)(gather ? g.rows[ri[t]] : ri[t]) * g.lda;
+    }
+    if constexpr (kBk) pb[t] = g.B + (long long)cj[t] * g.ldb;
+  }
   floatx4 acc[2][2];
+  float rs[2] = {0.f, 0.f};
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = (floatx4){0.f, 0.f, 0.f, 0.f};
-  // This thread's elements of a step, (tile row, k) = (tid / 32 + 8 t,
-  // tid % 32) when the operand is contiguous along k, else (tid % 64,
-  // tid / 64 + 4 t): consecutive lanes read consecutive addresses either way.
-  const bool a_rows = g.sa_k != 1, b_rows = g.sb_k != 1;
-  int ar[kPer], ak[kPer], br[kPer], bk[kPer];
+  const int nsteps = (g.K + kStep - 1) / kStep;
+#pragma unroll 2
+  for (int st = kSplit ? wave : 0; st < nsteps; st += kSplit ? 4 : 1) {
+    const int k = st * kStep + 8 * q;
+    const bool whole = (st + 1) * kStep <= g.K;
+    float va[2][8], vb[2][8];
 #pragma unroll
-  for (int t = 0; t < kPer; ++t) {
-    ar[t] = a_rows ? (tid & 63) : (tid >> 5) + 8 * t;
-    ak[t] = a_rows ? (tid >> 6) + 4 * t : (tid & (kBK - 1));
-    br[t] = b_rows ? (tid & 63) : (tid >> 5) + 8 * t;
-    bk[t] = b_rows ? (tid >> 6) + 4 * t : (tid & (kBK - 1));
-  }
-  float ra[kPer], rb[kPer];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-      const int i = i0 + ar[t], ka = k0 + ak[t], j = j0 + br[t], kb = k0 + bk[t];
-      const bool oa = i < g.M && ka < g.K, ob = j < g.N && kb < g.K;
-      const float va = g.A[oa ? (long long)i * g.sa_i + (long long)ka * g.sa_k : 0];
-      const float vb = g.B[ob ? (long long)kb * g.sb_k + (long long)j * g.sb_j : 0];
-      ra[t] = oa ? va : 0.f;
-      rb[t] = ob ? vb : 0.f;
+    for (int t = 0; t < 2; ++t) {
+      if constexpr (kAk) load_rowk(pa[t], k, g.K, whole, va[t]);
+      else load_colk(g.A, g.lda, nullptr, ri[t], k, g.K, va[t]);
+      if constexpr (kBk) load_rowk(pb[t], k, g.K, whole, vb[t]);
+      else load_colk(g.B, g.ldb, EPI == kWeight ? g.rows : nullptr, cj[t], k, g.K, vb[t]);
     }
-  };
-  auto put = [&](int buf) {
+    bf16x8 fa[2], fb[2];
 #pragma unroll
-    for (int t = 0; t < kPer; ++t) {
-      As[buf][ar[t]][ak[t]] = to_bf16(ra[t]);
-      Bs[buf][br[t]][bk[t]] = to_bf16(rb[t]);
-    }
-  };
-  load(0);
-  put(0);
-  __syncthreads();
-  const int nsteps = (g.K + kBK - 1) / kBK;
-  for (int st = 0; st < nsteps; ++st) {
-    const int cur = st & 1;
-    load((st + 1) * kBK);  // past the end: every element is outside, zero
-    bf16x8 af[2], bfr[2];
+    for (int t = 0; t < 2; ++t) {
+      if constexpr (EPI == kWeight) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      af[a] = *reinterpret_cast<const bf16x8*>(&As[cur][wm * 32 + a * 16 + c][8 * q]);
-      bfr[a] = *reinterpret_cast<const bf16x8*>(&Bs[cur][wn * 32 + a * 16 + c][8 * q]);
+        for (int e = 0; e < 8; ++e) rs[t] += va[t][e];
+      }
+      fa[t] = pack8(va[t]);
+      fb[t] = pack8(vb[t]);
     }
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < 2; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
-    if (st + 1 < nsteps) put(cur ^ 1);
-    __syncthreads();
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
   }
-  // Epilogue.
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wm * 32 + a * 16 + 4 * q + r;
-        const int j = j0 + wn * 32 + b * 16 + c;
-        if (i < g.M && j < g.N) {
-          float v = acc[a][b][r];
-          if (g.bias) v += g.bias[j];
-          const long long o = (long long)i * g.sc_i + j;
-          if (g.gelu) {
-            g.Z[o] = v;
-            g.C[o] = gelu(v);
-          } else if (g.accumulate) {
-            g.C[o] += v;
-          } else {
-            g.C[o] = v;
-          }
-        }
-      }
-}
-
-// dZ = dH * GELU'(Z), elementwise.
-__global__ void gelu_backward(const float* __restrict__ dH, const float* __restrict__ Z,
-                              float* __restrict__ dZ, long long n) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    dZ[i] = dH[i] * gelu_grad(Z[i]);
-}
-
-// out[j] = sum_i X[i*ld + j] over rows, in a fixed order (deterministic):
-// thread (g, c) of a block sums rows g, g + 16, ... of column
-// 16 blockIdx.x + c in row order (8 loads in flight), then the 16 row
-// groups' sums are added in group order: the same order on every launch.
-constexpr int kSumCols = 16, kSumGroups = 16;
-
-__global__ void __launch_bounds__(256) column_sums(const float* __restrict__ X, int rows,
-                                                   int cols, long long ld,
-                                                   float* __restrict__ out) {
-  __shared__ float part[kSumGroups][kSumCols];
-  const int c = threadIdx.x % kSumCols, grp = threadIdx.x / kSumCols;
-  const int j = blockIdx.x * kSumCols + c;
-  const int jc = j < cols ? j : cols - 1;  // loads stay in the matrix
-  float s = 0.f;
-  int i = grp;
-  for (; i + 7 * kSumGroups < rows; i += 8 * kSumGroups) {
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = X[(long long)(i + u * kSumGroups) * ld + jc];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u];
+      for (int r = 0; r < 4; ++r) part[wave][16 * a + 4 * q + r][16 * b + c] = acc[a][b][r];
+  if constexpr (EPI == kWeight) {
+    bsum[wave][q][c] = rs[0];
+    bsum[wave][q][16 + c] = rs[1];
   }
-  for (; i < rows; i += kSumGroups) s += X[(long long)i * ld + jc];
-  part[grp][c] = s;
   __syncthreads();
-  if (grp == 0 && j < cols) {
-    float t = part[0][c];
-    for (int q = 1; q < kSumGroups; ++q) t += part[q][c];
-    out[j] = t;
+  // Epilogue: thread t takes column t % 32 of rows t / 32, + 8, ... (its
+  // wave's own tile: lane / 32, + 2, ...)
+  const int col = tid & 31, j = j0 + col;
+  double loss = 0;
+#pragma unroll
+  for (int r = 0; r < (kSplit ? 4 : 16); ++r) {
+    const int row = kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r, i = i0 + row;
+    if (!live || i >= g.M || j >= g.N) continue;
+    float x = kSplit ? ((part[0][row][col] + part[1][row][col]) + part[2][row][col]) +
+                           part[3][row][col]
+                     : part[wave][row][col];
+    const long long o = (long long)i * g.ldc + j;
+    if constexpr (EPI == kBias) {
+      g.C[o] = x + g.bias[j];
+    } else if constexpr (EPI == kGelu) {
+      x += g.bias[j];
+      g.Z[o] = x;
+      g.C[o] = gelu(x);
+    } else if constexpr (EPI == kMseGrad) {
+      const float d = x + g.bias[j] - g.T[(long long)(g.rows ? g.rows[i] : i) * g.N + j];
+      g.C[o] = g.scale * d;
+      loss += (double)d * d;
+    } else if constexpr (EPI == kGeluGrad) {
+      g.C[o] = x * gelu_grad(g.Z[o]);
+    } else {
+      if (g.p) adam_one(g.p, g.m, g.v, o, x, adam);
+      else g.C[o] = x;
+    }
   }
-}
-
-// dY = 2 (Y - T) / n; partial[block] = sum of (Y - T)^2 over the block's
-// grid-stride range (summed by the host in block order).
-__global__ void __launch_bounds__(256) mse_grad(const float* __restrict__ Y,
-                                                const float* __restrict__ T,
-                                                float* __restrict__ dY, long long n,
-                                                double* __restrict__ partial) {
-  __shared__ double red[256];
-  double s = 0;
-  const float scale = 2.0f / (float)n;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float d = Y[i] - T[i];
-    dY[i] = scale * d;
-    s += (double)d * d;
+  if constexpr (EPI == kWeight) {
+    if (j0 == 0 && tid < kTile && i0 + tid < g.M) {
+      float x = 0.f;
+      for (int w = 0; w < 4; ++w)
+        for (int u = 0; u < 4; ++u) x += bsum[w][u][tid];
+      if (g.bp) adam_one(g.bp, g.bm, g.bv, i0 + tid, x, adam);
+      else g.bias_out[i0 + tid] = x;
+    }
   }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+  if constexpr (EPI == kMseGrad) {
+    __shared__ double red[4];
+    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
+    if (lane == 0) red[wave] = loss;
     __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// Adam on flat float32 arrays (bias-corrected step sizes from the host).
-__global__ void adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                     float* __restrict__ v, long long n, float lr_t, float beta1, float beta2,
-                     float eps_t) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float gi = g[i];
-    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
-    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr_t * mi / (sqrtf(vi) + eps_t);
+    if (tid == 0) g.partial[block] = ((red[0] + red[1]) + red[2]) + red[3];
   }
 }
 
-// rows[i] = src[index[i]] for rows of `cols` floats (minibatch gather).
-__global__ void gather_rows(const float* __restrict__ src, const int* __restrict__ index,
-                            int rows, int cols, float* __restrict__ dst) {
-  const long long n = (long long)rows * cols;
-  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (long long)gridDim.x * blockDim.x) {
-    const int r = (int)(e / cols), c = (int)(e - (long long)r * cols);
-    dst[e] = src[(long long)index[r] * cols + c];
-  }
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_bf16(GemmArgs g) {
+  product<EPI>(g, blockIdx.x, AdamArgs{});
+}
+
+// Layers' weight gradients, one after the other in the grid.
+struct WeightArgs {
+  GemmArgs g[3];
+  int first[4];
+  AdamArgs adam;
+};
+
+__global__ void __launch_bounds__(256) weight_grads(WeightArgs w) {
+  const int b = blockIdx.x;
+  if (b < w.first[1]) product<kWeight>(w.g[0], b, w.adam);
+  else if (b < w.first[2]) product<kWeight>(w.g[1], b - w.first[1], w.adam);
+  else product<kWeight>(w.g[2], b - w.first[2], w.adam);
 }
 
 }  // namespace mlp
 
 // --- Host launchers ---------------------------------------------------------------
 
-hipError_t LaunchGemmBf16(const mlp::GemmArgs& g, hipStream_t s) {
-  const dim3 grid((g.N + mlp::kBN - 1) / mlp::kBN, (g.M + mlp::kBM - 1) / mlp::kBM);
-  hipLaunchKernelGGL(mlp::gemm_bf16, grid, dim3(256), 0, s, g);
+static int Tiles(int M, int N) {
+  return (M + mlp::kTile - 1) / mlp::kTile * ((N + mlp::kTile - 1) / mlp::kTile);
+}
+
+int LayerBlocks(int M, int N) { return (Tiles(M, N) + 3) / 4; }
+
+hipError_t LaunchLayer(const mlp::GemmArgs& g, mlp::Epilogue e, hipStream_t s) {
+  const dim3 grid(LayerBlocks(g.M, g.N)), block(256);
+  if (e == mlp::kBias)
+    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kBias>, grid, block, 0, s, g);
+  else if (e == mlp::kGelu)
+    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kGelu>, grid, block, 0, s, g);
+  else if (e == mlp::kMseGrad)
+    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kMseGrad>, grid, block, 0, s, g);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-hipError_t LaunchGeluBackward(const float* dH, const float* Z, float* dZ, long long n,
-                              hipStream_t s) {
-  long long blocks = (n + 255) / 256;
-  if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL(mlp::gelu_backward, dim3((unsigned)blocks), dim3(256), 0, s, dH, Z, dZ, n);
+hipError_t LaunchInputGrad(const mlp::GemmArgs& g, hipStream_t s) {
+  hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kGeluGrad>, dim3(Tiles(g.M, g.N)), dim3(256), 0, s,
+                     g);
   return hipGetLastError();
 }
 
-hipError_t LaunchColumnSums(const float* X, int rows, int cols, long long ld, float* out,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(mlp::column_sums, dim3((cols + mlp::kSumCols - 1) / mlp::kSumCols),
-                     dim3(256), 0, s, X, rows, cols, ld, out);
-  return hipGetLastError();
-}
-
-hipError_t LaunchMseGrad(const float* Y, const float* T, float* dY, long long n, double* partial,
-                         int blocks, hipStream_t s) {
-  hipLaunchKernelGGL(mlp::mse_grad, dim3(blocks), dim3(256), 0, s, Y, T, dY, n, partial);
-  return hipGetLastError();
-}
-
-hipError_t LaunchAdam(float* p, const float* g, float* m, float* v, long long n, float lr_t,
-                      float beta1, float beta2, float eps_t, hipStream_t s) {
-  long long blocks = (n + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(mlp::adam, dim3((unsigned)blocks), dim3(256), 0, s, p, g, m, v, n, lr_t,
-                     beta1, beta2, eps_t);
-  return hipGetLastError();
-}
-
-hipError_t LaunchGatherRows(const float* src, const int* index, int rows, int cols, float* dst,
-                            hipStream_t s) {
-  long long n = (long long)rows * cols;
-  long long blocks = (n + 255) / 256;
-  if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL(mlp::gather_rows, dim3((unsigned)blocks), dim3(256), 0, s, src, index, rows,
-                     cols, dst);
+hipError_t LaunchWeightGrads(const mlp::GemmArgs* g, int count, const mlp::AdamArgs& adam,
+                             hipStream_t s) {
+  if (count != 3) return hipErrorInvalidValue;
+  mlp::WeightArgs w{};
+  w.adam = adam;
+  for (int i = 0; i < 3; ++i) {
+    w.g[i] = g[i];
+    w.first[i + 1] = w.first[i] + Tiles(g[i].M, g[i].N);
+  }
+  hipLaunchKernelGGL(mlp::weight_grads, dim3(w.first[3]), dim3(256), 0, s, w);
   return hipGetLastError();
 }
 
