@@ -28,10 +28,10 @@ using act::gelu_grad;
 // So a wave takes a 32 x 32 tile straight from global memory into MFMA
 // fragments, with no LDS and no barrier in the loop.  The layers accumulate
 // over K in order (the fused closure pass does, and evaluates the same
-// function to the bit): a block's four waves own four tiles.  The gradients'
-// longer sums (K = outputs or batch rows) are split: the four waves take the
-// K steps w, w + 4, ... of one tile and are added through LDS in wave order
-// (deterministic).  The epilogue does what would be further launches: bias,
+// function to the bit), one wave a block so that 128 tiles reach 128 CUs.  The
+// gradients' longer sums (K = outputs or batch rows) are split: a block's
+// four waves take the K steps w, w + 4, ... of one tile and are added through
+// LDS in wave order (deterministic).  The epilogue does what would be further launches: bias,
 // GELU, the loss and its gradient, GELU', the bias gradient (row sums of the
 // FP32 A operand) and Adam.  A training step of batch 512 is 6 launches
 // instead of 17.
@@ -41,12 +41,18 @@ using act::gelu_grad;
 // Operands are rounded to bfloat16 (nearest even) as they are loaded.
 constexpr int kTile = 32, kStep = 32;
 
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
 typedef float F4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Eight consecutive k of one row r (k contiguous): two 16-byte loads where
 // the whole step is inside K, else masked elements.
-__device__ __forceinline__ void load_rowk(const float* p, int k, int K, bool whole, float* v) {
-  if (whole) {
+template <bool WHOLE>
+__device__ __forceinline__ void load_rowk(const float* p, int k, int K, float* v) {
+  if constexpr (WHOLE) {
     const F4u a = *reinterpret_cast<const F4u*>(p + k);
     const F4u b = *reinterpret_cast<const F4u*>(p + k + 4);
 #pragma unroll
@@ -64,13 +70,20 @@ __device__ __forceinline__ void load_rowk(const float* p, int k, int K, bool who
 }
 
 // Eight consecutive k of one column c (k strided by ld; rows gathers them).
+template <bool WHOLE>
 __device__ __forceinline__ void load_colk(const float* base, long long ld, const int* rows,
                                           int c, int k, int K, float* v) {
+  int kk[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) kk[e] = WHOLE ? k + e : min(k + e, K - 1);
+  if (rows) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) kk[e] = rows[kk[e]];
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const int kk = min(k + e, K - 1);
-    const float x = base[(long long)(rows ? rows[kk] : kk) * ld + c];
-    v[e] = k + e < K ? x : 0.f;
+    const float x = base[(long long)kk[e] * ld + c];
+    v[e] = WHOLE || k + e < K ? x : 0.f;
   }
 }
 
@@ -81,28 +94,34 @@ __device__ __forceinline__ bf16x8 pack8(const float* v) {
   return r;
 }
 
+struct AdamIn {
+  float p, m, v;
+};
+__device__ __forceinline__ AdamIn adam_load(const float* p, const float* m, const float* v,
+                                            long long o) {
+  return AdamIn{p[o], m[o], v[o]};
+}
 __device__ __forceinline__ void adam_one(float* p, float* m, float* v, long long o, float g,
-                                         const AdamArgs& a) {
-  const float mi = a.beta1 * m[o] + (1.f - a.beta1) * g;
-  const float vi = a.beta2 * v[o] + (1.f - a.beta2) * g * g;
+                                         const AdamIn& x, const AdamArgs& a) {
+  const float mi = a.beta1 * x.m + (1.f - a.beta1) * g;
+  const float vi = a.beta2 * x.v + (1.f - a.beta2) * g * g;
   m[o] = mi;
   v[o] = vi;
-  p[o] -= a.lr_t * mi / (sqrtf(vi) + a.eps_t);
+  p[o] = x.p - a.lr_t * mi / (sqrtf(vi) + a.eps_t);
 }
 
 template <int EPI>
 __device__ __forceinline__ void product(const GemmArgs& g, int block, const AdamArgs& adam) {
-  __shared__ float part[4][kTile][kTile + 1];
-  __shared__ float bsum[4][4][kTile];
+  constexpr bool kSplit = EPI > kMseGrad;
+  constexpr int kWaves = kSplit ? 4 : 1;
+  __shared__ float part[kWaves][kTile][kTile + 1];
+  __shared__ float bsum[kWaves][4][kTile];
   constexpr bool kAk = EPI != kWeight;                 // A rows contiguous along k
   constexpr bool kBk = EPI <= kMseGrad;                // B columns contiguous along k
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int q = lane >> 4, c = lane & 15;
-  constexpr bool kSplit = EPI > kMseGrad;
-  const int tj = (g.N + kTile - 1) / kTile, tiles = (g.M + kTile - 1) / kTile * tj;
-  const int tile = kSplit ? block : min(4 * block + wave, tiles - 1);
-  const bool live = kSplit || 4 * block + wave < tiles;
-  const int i0 = tile / tj * kTile, j0 = tile % tj * kTile;
+  const int tj = (g.N + kTile - 1) / kTile;
+  const int i0 = block / tj * kTile, j0 = block % tj * kTile;
   int ri[2], cj[2];
   const float *pa[2], *pb[2];
 #pragma unroll
@@ -118,41 +137,92 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
     }
     if constexpr (kBk) pb[t] = g.B + (long long)cj[t] * g.ldb;
   }
+  // Epilogue: thread t takes column t % 32 of rows t / 32, + 8, ... (its
+  // wave's own tile: lane / 32, + 2, ...).  Its operands are loaded before
+  // the K loop (clamped inside the matrices, unused there).
+  constexpr int kRows = kSplit ? 4 : 16;
+  const int col = tid & 31, j = j0 + col, jc = min(j, g.N - 1);
+  int ie[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r)
+    ie[r] = min(i0 + (kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r), g.M - 1);
+  float in[kRows], bias = 0.f;
+  AdamIn ad[kRows], adb{0.f, 0.f, 0.f};
+  if constexpr (EPI <= kMseGrad) bias = g.bias[jc];
+  if constexpr (EPI == kMseGrad) {
+    int row[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) row[r] = g.rows ? g.rows[ie[r]] : ie[r];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) in[r] = g.T[(long long)row[r] * g.N + jc];
+  }
+  if constexpr (EPI == kGeluGrad) {
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) in[r] = g.Z[(long long)ie[r] * g.ldc + jc];
+  }
+  if constexpr (EPI == kWeight) {
+    if (g.p) {
+#pragma unroll
+      for (int r = 0; r < kRows; ++r)
+        ad[r] = adam_load(g.p, g.m, g.v, (long long)ie[r] * g.ldc + jc);
+      adb = adam_load(g.bp, g.bm, g.bv, min(i0 + (tid & 31), g.M - 1));
+    }
+  }
   floatx4 acc[2][2];
   float rs[2] = {0.f, 0.f};
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = (floatx4){0.f, 0.f, 0.f, 0.f};
-  const int nsteps = (g.K + kStep - 1) / kStep;
-#pragma unroll 2
-  for (int st = kSplit ? wave : 0; st < nsteps; st += kSplit ? 4 : 1) {
-    const int k = st * kStep + 8 * q;
-    const bool whole = (st + 1) * kStep <= g.K;
-    float va[2][8], vb[2][8];
+  // `count` K steps from st, all their loads in flight before the first use.
+  constexpr int kInc = kSplit ? 4 : 1;
+  auto steps = [&](int st, auto count, auto whole) {
+    constexpr int kCount = decltype(count)::value;
+    constexpr bool kWhole = decltype(whole)::value;
+    float va[kCount][2][8], vb[kCount][2][8];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if constexpr (kAk) load_rowk(pa[t], k, g.K, whole, va[t]);
-      else load_colk(g.A, g.lda, nullptr, ri[t], k, g.K, va[t]);
-      if constexpr (kBk) load_rowk(pb[t], k, g.K, whole, vb[t]);
-      else load_colk(g.B, g.ldb, EPI == kWeight ? g.rows : nullptr, cj[t], k, g.K, vb[t]);
-    }
-    bf16x8 fa[2], fb[2];
+    for (int u = 0; u < kCount; ++u) {
+      const int k = (st + u * kInc) * kStep + 8 * q;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if constexpr (EPI == kWeight) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) rs[t] += va[t][e];
+      for (int t = 0; t < 2; ++t) {
+        if constexpr (kAk) load_rowk<kWhole>(pa[t], k, g.K, va[u][t]);
+        else load_colk<kWhole>(g.A, g.lda, nullptr, ri[t], k, g.K, va[u][t]);
+        if constexpr (kBk) load_rowk<kWhole>(pb[t], k, g.K, vb[u][t]);
+        else load_colk<kWhole>(g.B, g.ldb, EPI == kWeight ? g.rows : nullptr, cj[t], k, g.K,
+                               vb[u][t]);
       }
-      fa[t] = pack8(va[t]);
-      fb[t] = pack8(vb[t]);
     }
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int u = 0; u < kCount; ++u) {
+      bf16x8 fa[2], fb[2];
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        if constexpr (EPI == kWeight) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) rs[t] += va[u][t][e];
+        }
+        fa[t] = pack8(va[u][t]);
+        fb[t] = pack8(vb[u][t]);
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+    }
+  };
+  const int nwhole = g.K / kStep;
+  int st = kSplit ? wave : 0;
+  for (; st + 3 * kInc < nwhole; st += 4 * kInc) steps(st, Int<4>{}, Int<1>{});
+  if (st + kInc < nwhole) {
+    steps(st, Int<2>{}, Int<1>{});
+    st += 2 * kInc;
   }
+  if (st < nwhole) {
+    steps(st, Int<1>{}, Int<1>{});
+    st += kInc;
+  }
+  if (g.K % kStep != 0 && st == nwhole) steps(st, Int<1>{}, Int<0>{});
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -164,33 +234,38 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
     bsum[wave][q][16 + c] = rs[1];
   }
   __syncthreads();
-  // Epilogue: thread t takes column t % 32 of rows t / 32, + 8, ... (its
-  // wave's own tile: lane / 32, + 2, ...)
-  const int col = tid & 31, j = j0 + col;
   double loss = 0;
 #pragma unroll
-  for (int r = 0; r < (kSplit ? 4 : 16); ++r) {
-    const int row = kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r, i = i0 + row;
-    if (!live || i >= g.M || j >= g.N) continue;
-    float x = kSplit ? ((part[0][row][col] + part[1][row][col]) + part[2][row][col]) +
-                           part[3][row][col]
-                     : part[wave][row][col];
-    const long long o = (long long)i * g.ldc + j;
+  for (int r = 0; r < kRows; ++r) {
+    const int row = kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r;
+    float x = part[0][row][col];
+    if constexpr (kSplit)
+      x = ((x + part[1][row][col]) + part[2][row][col]) + part[3][row][col];
+    const long long o = (long long)ie[r] * g.ldc + jc;
+    const bool ok = i0 + row < g.M && j < g.N;
     if constexpr (EPI == kBias) {
-      g.C[o] = x + g.bias[j];
+      if (ok) g.C[o] = x + bias;
     } else if constexpr (EPI == kGelu) {
-      x += g.bias[j];
-      g.Z[o] = x;
-      g.C[o] = gelu(x);
+      x += bias;
+      const float h = gelu(x);
+      if (ok) {
+        g.Z[o] = x;
+        g.C[o] = h;
+      }
     } else if constexpr (EPI == kMseGrad) {
-      const float d = x + g.bias[j] - g.T[(long long)(g.rows ? g.rows[i] : i) * g.N + j];
-      g.C[o] = g.scale * d;
-      loss += (double)d * d;
+      const float d = x + bias - in[r];
+      if (ok) {
+        g.C[o] = g.scale * d;
+        loss += (double)d * d;
+      }
     } else if constexpr (EPI == kGeluGrad) {
-      g.C[o] = x * gelu_grad(g.Z[o]);
+      const float d = x * gelu_grad(in[r]);
+      if (ok) g.C[o] = d;
     } else {
-      if (g.p) adam_one(g.p, g.m, g.v, o, x, adam);
-      else g.C[o] = x;
+      if (ok) {
+        if (g.p) adam_one(g.p, g.m, g.v, o, x, ad[r], adam);
+        else g.C[o] = x;
+      }
     }
   }
   if constexpr (EPI == kWeight) {
@@ -198,21 +273,18 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
       float x = 0.f;
       for (int w = 0; w < 4; ++w)
         for (int u = 0; u < 4; ++u) x += bsum[w][u][tid];
-      if (g.bp) adam_one(g.bp, g.bm, g.bv, i0 + tid, x, adam);
+      if (g.bp) adam_one(g.bp, g.bm, g.bv, i0 + tid, x, adb, adam);
       else g.bias_out[i0 + tid] = x;
     }
   }
   if constexpr (EPI == kMseGrad) {
-    __shared__ double red[4];
     for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
-    if (lane == 0) red[wave] = loss;
-    __syncthreads();
-    if (tid == 0) g.partial[block] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (lane == 0) g.partial[block] = loss;
   }
 }
 
 template <int EPI>
-__global__ void __launch_bounds__(256) gemm_bf16(GemmArgs g) {
+__global__ void __launch_bounds__(EPI > kMseGrad ? 256 : 64) gemm_bf16(GemmArgs g) {
   product<EPI>(g, blockIdx.x, AdamArgs{});
 }
 
@@ -238,10 +310,10 @@ static int Tiles(int M, int N) {
   return (M + mlp::kTile - 1) / mlp::kTile * ((N + mlp::kTile - 1) / mlp::kTile);
 }
 
-int LayerBlocks(int M, int N) { return (Tiles(M, N) + 3) / 4; }
+int LayerBlocks(int M, int N) { return Tiles(M, N); }
 
 hipError_t LaunchLayer(const mlp::GemmArgs& g, mlp::Epilogue e, hipStream_t s) {
-  const dim3 grid(LayerBlocks(g.M, g.N)), block(256);
+  const dim3 grid(LayerBlocks(g.M, g.N)), block(64);
   if (e == mlp::kBias)
     hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kBias>, grid, block, 0, s, g);
   else if (e == mlp::kGelu)
