@@ -160,6 +160,93 @@ __device__ __forceinline__ void load_tile(const RhsArgs& A, const TI* __restrict
   }
 }
 
+// Matrix-core operations on 16x16x4 tiles in the bulk precision; row(g, r) =
+// the row of a lane group's output register r.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+template <typename TB> struct Mfma;
+template <> struct Mfma<float> {
+  typedef floatx4 acc;
+  static __device__ __forceinline__ acc zero() { return (floatx4){0.f, 0.f, 0.f, 0.f}; }
+  static __device__ __forceinline__ acc mac(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
+};
+template <> struct Mfma<double> {
+  typedef doublex4 acc;
+  static __device__ __forceinline__ acc zero() { return (doublex4){0., 0., 0., 0.}; }
+  static __device__ __forceinline__ acc mac(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int g, int r) { return g + 4 * r; }
+};
+
+// The element path above kElementMaxN states: -(i/hbar) H Y of a tile added
+// into W on the matrix cores, Y in LDS and H's fragments from global memory
+// (they stay in L1/L2), so that a block's LDS is one third smaller.  Work
+// items are (16-column slice, 16-row tile of H) pairs dealt to the waves.
+// What bounds a stage there is the blocks that fit a CU and the chain of
+// gathers: 630 nodes of 34 sites, FP64, 28 us a stage with H in LDS (two
+// blocks a CU, two rounds) and one gather pair in flight per thread, the
+// product on the vector units or here alike; 20 with this form and the
+// gathers of all of a thread's elements in flight.
+constexpr int kElementMaxN = 32;
+
+template <typename TB>
+__device__ __forceinline__ void rhs_gemm_lds(const RhsArgs& A, int nt, const Lds<TB>& s) {
+  typedef typename C2<TB>::type V;
+  typedef Mfma<TB> M;
+  const int N = A.N, NE = A.NE, NP = N * (N + 1);
+  const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+  const int wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+  const int KS = (N + 3) >> 2, MT = (N + 15) >> 4, ncols = nt * N;
+  const int nitems = ((ncols + 15) >> 4) * MT;
+  const TB ih = (TB)A.inv_hbar;
+  const bool realh = A.real_h != 0;
+  for (int item = wave; item < nitems; item += nwaves) {
+    const int slice = item / MT, mt = item - slice * MT;
+    const int j = slice * 16 + c16;
+    const bool jok = j < ncols;
+    const int tj = jok ? fdiv(j, A.mN) : 0, bj = jok ? j - tj * N : 0;
+    const V* y = s.Y + tj * NE + bj * N;
+    const int row = 16 * mt + c16;
+    const double2* h = A.H + min(row, N - 1);
+    typename M::acc xr = M::zero(), xi = M::zero();
+#pragma unroll 5
+    for (int st = 0; st < KS; ++st) {
+      // lane group g covers k = g KS .. g KS + KS - 1; past N: zero
+      const int k = g * KS + st, kc = min(k, N - 1);
+      const bool ok = k < N;
+      V v = y[kc];
+      const double2 hd = h[kc * N];
+      V w = mk<TB>((TB)hd.x, (TB)hd.y);
+      if (!ok) v = mk<TB>((TB)0, (TB)0);
+      if (!ok || row >= N) w = mk<TB>((TB)0, (TB)0);
+      xr = M::mac(w.x, v.x, xr);
+      xi = M::mac(w.x, v.y, xi);
+      if (!realh) {
+        xr = M::mac(-w.y, v.y, xr);
+        xi = M::mac(w.y, v.x, xi);
+      }
+    }
+    if (jok) {
+      V* wcol = s.W + tj * NP + bj * (N + 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int o = 16 * mt + M::row(g, r);
+        if (o < N) {
+          V w = wcol[o];
+          w.x += ih * xi[r];
+          w.y -= ih * xr[r];
+          wcol[o] = w;
+        }
+      }
+    }
+  }
+}
+
 // Phase 1: W(a,b) = Y'(a,b) = -(i/hbar) (H Y)(a,b) - (mu/2 + (Delta_a +
 // Delta_b)/2 [a != b]) Y(a,b) + A(a,b), where column b of A gathers, over the
 // modes j coupled to site b, i s_j Y_{n+e_j}(a,b) - col_j Y_{n-e_j}(a,b).
@@ -171,6 +258,61 @@ __device__ __forceinline__ void rhs_phase(const RhsArgs& A, const TI* __restrict
   const int N = A.N, NE = A.NE, D = A.D, L = A.L;
   const int NP = N * (N + 1);
   const TB ih = (TB)A.inv_hbar;
+  if (N > kElementMaxN) {
+    // kBatch elements at a time, their first mode's gathers all in flight
+    // (an absent neighbour or an element past the tile loads its own).
+    constexpr int kBatch = 5;
+    const int tot = nt * NE;
+    for (int e0 = threadIdx.x; e0 < tot; e0 += kBatch * blockDim.x) {
+      V gn[kBatch], gp[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int e = min(e0 + i * (int)blockDim.x, tot - 1);
+        const int t = fdiv(e, A.mNE), r = e - t * NE, b = fdiv(r, A.mN);
+        int nx = -1, pv = -1;
+        if (!A.vacuum && s.sp[b] < s.sp[b + 1]) {
+          const int j = s.sm[s.sp[b]];
+          nx = s.nx[t * D + j];
+          pv = s.pv[t * D + j];
+        }
+        gn[i] = ld<TB, TI>(in, (size_t)max(nx, 0) * NE + r);
+        gp[i] = ld<TB, TI>(in, (size_t)max(pv, 0) * NE + r);
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int e = e0 + i * (int)blockDim.x;
+        if (e >= tot) break;
+        const int t = fdiv(e, A.mNE), r = e - t * NE, b = fdiv(r, A.mN), a = r - b * N;
+        TB ax = 0, ay = 0;
+        if (!A.vacuum) {
+          for (int q = s.sp[b]; q < s.sp[b + 1]; ++q) {
+            const int j = s.sm[q], k = s.oc[t * D + j];
+            const int nx = s.nx[t * D + j], pv = s.pv[t * D + j];
+            const bool first = q == s.sp[b];
+            if (nx >= 0) {
+              const TB sc = s.ns[j * L + k];
+              const V y = first ? gn[i] : ld<TB, TI>(in, (size_t)nx * NE + r);
+              ax -= sc * y.y;
+              ay += sc * y.x;
+            }
+            if (pv >= 0) {
+              const V c = s.pcol[j * L + k];
+              const V y = first ? gp[i] : ld<TB, TI>(in, (size_t)pv * NE + r);
+              ax -= c.x * y.x - c.y * y.y;
+              ay -= c.x * y.y + c.y * y.x;
+            }
+          }
+        }
+        const V y = s.Y[e];
+        TB f = s.mu2[t];
+        if (a != b) f += (TB)0.5 * (s.delta[a] + s.delta[b]);
+        s.W[t * NP + b * (N + 1) + a] = mk<TB>(ax - f * y.x, ay - f * y.y);
+      }
+    }
+    __syncthreads();
+    rhs_gemm_lds<TB>(A, nt, s);
+    return;
+  }
   for (int e = threadIdx.x; e < nt * NE; e += blockDim.x) {
     const int t = fdiv(e, A.mNE);
     const int r = e - t * NE;
@@ -224,27 +366,6 @@ __device__ __forceinline__ void rhs_phase(const RhsArgs& A, const TI* __restrict
 // permutation on both operands.  H fragments are read once from global
 // memory into registers; real H (the common case) takes one product per
 // real/imaginary part, complex H two.
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-template <typename TB> struct Mfma;
-template <> struct Mfma<float> {
-  typedef floatx4 acc;
-  static __device__ __forceinline__ acc zero() { return (floatx4){0.f, 0.f, 0.f, 0.f}; }
-  static __device__ __forceinline__ acc mac(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
-};
-template <> struct Mfma<double> {
-  typedef doublex4 acc;
-  static __device__ __forceinline__ acc zero() { return (doublex4){0., 0., 0., 0.}; }
-  static __device__ __forceinline__ acc mac(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int g, int r) { return g + 4 * r; }
-};
-
 template <typename TB, typename TI>
 __device__ __forceinline__ void rhs_phase_mfma(const RhsArgs& A, const TI* __restrict__ in,
                                                int nt, const Lds<TB>& s) {
@@ -476,10 +597,11 @@ __global__ void __launch_bounds__(256) rk4_stage(RhsArgs A, const TI* __restrict
   const int base = blockIdx.x * A.tile;
   const int nt = min(A.tile, A.num_nodes - base);
   if (nt <= 0) return;
-  const Lds<TB> s = carve<TB>(smem, A.N, A.D, A.L, A.tile, NM != 1);
+  const bool with_h = NM != 1 && A.N <= kElementMaxN;
+  const Lds<TB> s = carve<TB>(smem, A.N, A.D, A.L, A.tile, with_h);
   const int tot = nt * NE;
   const size_t off = (size_t)base * NE;
-  load_tile<TB, TI>(A, in, base, nt, s, NM != 1);
+  load_tile<TB, TI>(A, in, base, nt, s, with_h);
   // Epilogue operands stream in chunks of kPre elements per thread, the loads
   // of chunk c+1 in flight while chunk c is combined; chunk 0 is issued
   // with the tile loads.
@@ -565,10 +687,11 @@ __global__ void __launch_bounds__(256) rkf45_stage(RhsArgs A, const TI* __restri
   const int base = blockIdx.x * A.tile;
   const int nt = min(A.tile, A.num_nodes - base);
   if (nt <= 0) return;
-  const Lds<TB> s = carve<TB>(smem, A.N, A.D, A.L, A.tile, NM != 1);
+  const bool with_h = NM != 1 && A.N <= kElementMaxN;
+  const Lds<TB> s = carve<TB>(smem, A.N, A.D, A.L, A.tile, with_h);
   const int tot = nt * NE;
   const size_t off = (size_t)base * NE;
-  load_tile<TB, TI>(A, in, base, nt, s, NM != 1);
+  load_tile<TB, TI>(A, in, base, nt, s, with_h);
   double2 pr[kPre];
   auto prefetch = [&]() {
 #pragma unroll

@@ -756,7 +756,7 @@ size_t TileLdsBytes(int N, int D, int L, int tile, bool fp32, bool with_h) {
 
 size_t RhsSharedBytes(const RhsArgs& a, bool fp32) {
   return dev::LdsBytes(a.N, a.D, a.L, a.tile, fp32 ? sizeof(float) : sizeof(double),
-                       a.col_nm == 0);
+                       a.col_nm == 0 && a.N <= dev::kElementMaxN);
 }
 
 size_t StreamTileLdsBytes(int N, int D, int L, int tile, bool fp32) {

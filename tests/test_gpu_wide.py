@@ -1,6 +1,6 @@
 """Kernels by node size: full coupling operators (whole nodes in a wave, one
-to four elements a thread, operators all in LDS or bath by bath), against
-the oracle."""
+to four elements a thread, operators all in LDS or bath by bath) and states
+above 32 (the product on the matrix cores), against the oracle."""
 
 import os
 import sys
@@ -49,3 +49,39 @@ def test_full_operators(N, M, terms, lh):
     # of magnitudes: 16 N M ulp of it
     big = np.abs(ref).max() * np.sqrt(N) * M
     assert err <= 16 * N * M * 2.2e-16 * big
+
+
+@pytest.mark.parametrize("N,lh,terms,precision,complex_h", [
+    (33, 3, 1, "fp64", True), (34, 2, 2, "fp64", False), (36, 2, 1, "fp64", True),
+    (35, 2, 2, "fp32", True)])
+def test_more_than_32_states(N, lh, terms, precision, complex_h):
+    rng = np.random.default_rng([N, lh, terms])
+    H = rng.normal(0.0, 0.4, (N, N)) + 0j
+    H = H + H.T
+    if complex_h:
+        A = rng.normal(0.0, 0.3, (N, N))
+        H = H + 1j * (A - A.T)
+    M = N  # one site without a bath, one with two
+    site = list(range(M))
+    site[1] = 0
+    rho0 = np.zeros((N, N), dtype=complex)
+    rho0[0, 0] = 1
+    kw = dict(gamma=[1.0 + 0.02 * i for i in range(M)], lambda_=[0.05] * M, temperature=0.7,
+              lh=lh, num_terms=terms)
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    p.set_array("multiple_independent_bath_indices", site)
+    p.set_int("is_multiple_independent_baths", 1)
+    assert p.fix("rk4") == 0
+    ctx = P.Context(p, precision=precision)
+    orc = HO.Oracle(HO.Problem(H=H, rho0=rho0, hbar=1.0, kb=1.0, bath_site=site, **kw), threads=4)
+    x = random_state(rng, ctx.num_nodes, N)
+    x = x + x.conj().transpose(0, 2, 1)   # (the stage kernels' form of Hermitian states)
+    x /= np.abs(x).max()
+    ctx.set_state(x)
+    orc.set_state(x)
+    ctx.rk4_steps(3, 0.002)
+    orc.rk4(0.006, 0.002, 1.0)
+    err = np.abs(ctx.state() - orc.state()).max()
+    print("wide", N, lh, terms, precision, err, flush=True)
+    # FP32: the increments (|dt L| < 1 of the state) are rounded
+    assert err <= (3e-14 if precision == "fp64" else 2e-6)
