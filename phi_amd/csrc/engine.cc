@@ -1335,8 +1335,7 @@ int Engine::Rk4StageTimes(long long nsteps, double dt, double ms[4]) {
 // a^H b: each cycle takes ell BiCG steps (u_0..u_ell, r_0..r_ell and their
 // images under A), then minimises |r_0 - sum_j gamma_j r_j| over the
 // Krylov polynomial of degree ell (modified Gram-Schmidt on r_1..r_ell).
-// Scalars on the host: every inner product is one reduction and one
-// round trip.  PHI's BicgstabLSteadyState (hierarchy_integrator.cc:
+// Scalars on the device, derived by the passes that use them.  PHI's BicgstabLSteadyState (hierarchy_integrator.cc:
 // 3112-3489) follows the same outline.
 int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* resid,
                          std::vector<double>* history) {
@@ -1381,58 +1380,49 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
     return rc;
   }
   double* x = d_rho_;
-  // Scalars and the per-cycle residuals on the device.
+  // Two records of the scalars (each step reads one and writes the other;
+  // the first is current between batches), two buffers of partials (likewise)
+  // and the per-cycle residuals on the device.
   BicglScalars* S = nullptr;
   double* hist = nullptr;
+  double* part[2] = {nullptr, nullptr};
   // (the residual history keeps its first 2^20 cycles)
   const int hist_cap = (int)std::min<long long>((long long)max_iter / ell + 2, 1 << 20);
-  rc = Check(hipMalloc((void**)&S, sizeof(BicglScalars)), "alloc bicgstab(l) scalars");
-  if (!rc) rc = Check(hipMalloc((void**)&hist, (size_t)hist_cap * sizeof(double)), "alloc hist");
-  // dot product into S->dot[k], then the scalar step op in the same kernel
-  auto dot_step = [&](const double* a, const double* b, int k, int op, int i, int j) -> int {
-    return Check(LaunchBicglDotStep(a, b, n, d_partial_, red_blocks_, S, k, op, i, j, tol,
-                                    max_iter, hist, hist_cap, stream_),
-                 "bicgstab(l) step");
-  };
-  // (a, b) into S->dot[k] and (c, d) into S->dot[k + 1] in one pass, then
-  // the step op; the partials of 4 doubles per block fill d_partial_
-  // (2 * red_blocks_ doubles) with red_blocks_ / 2 blocks.
-  auto dot2_step = [&](const double* a, const double* b, const double* c, const double* d, int k,
-                       int op, int i, int j) -> int {
-    return Check(LaunchBicglDot2Step(a, b, c, d, n, d_partial_, red_blocks_ / 2, S, k, op, i, j,
-                                     tol, max_iter, hist, hist_cap, stream_),
-                 "bicgstab(l) step");
-  };
-  // y = a + sign * c * b, c a scalar of S
-  auto axpy = [&](double* y, const double* a, const double* b, const double2* c,
-                  double sign) -> int {
-    return Check(LaunchZaxpyDev(y, a, b, n, c, sign, &S->stop, stream_), "axpy");
-  };
-  // y = A x with (rtilde, y) into S->dot[0], then the step op: the matvec
-  // writes the dot product's partials itself when its LDS form fits.
+  // The matvec writes its dot products' partials itself when its LDS form fits.
   const int mb = RhsGeneralDotBlocks(args_);
-  double* pmv = nullptr;
-  if (!rc && mb > 0)
-    rc = Check(hipMalloc((void**)&pmv, (size_t)mb * 2 * sizeof(double)), "alloc matvec partials");
-  auto matvec_dot = [&](const double* xin, double* y, int op) -> int {
-    if (mb > 0) {
-      int e = Check(LaunchRhsGeneralDot(args_, xin, y, 1, 1, rt, nullptr, pmv, stream_),
-                    "rhs_general dot");
-      if (!e)
-        e = Check(LaunchBicglReduceStep(pmv, mb, S, 0, op, 0, 0, tol, max_iter, hist, hist_cap,
-                                        stream_),
-                  "bicgstab(l) step");
-      return e;
-    }
+  rc = Check(hipMalloc((void**)&S, 2 * sizeof(BicglScalars)), "alloc bicgstab(l) scalars");
+  if (!rc) rc = Check(hipMalloc((void**)&hist, (size_t)hist_cap * sizeof(double)), "alloc hist");
+  for (auto& p : part)
+    if (!rc)
+      rc = Check(hipMalloc((void**)&p, (size_t)std::max({mb, kBicglBlocks, red_blocks_}) * 6 *
+                                           sizeof(double)),
+                 "alloc bicgstab(l) partials");
+  int cur = 0;       // current record
+  int pb = 0;        // buffer of the latest partials
+  int npart = 0;     // and their blocks
+  // The step op on the latest partials, from the current record to the other.
+  auto take = [&](int op, int i, int j) {
+    BicglTake t{};
+    t.in = S + cur;
+    if (op != kBlNone) cur ^= 1;
+    t.out = S + cur;
+    t.part = part[pb];
+    t.nb = npart;
+    t.op = op, t.i = i, t.j = j;
+    t.tol = tol, t.max_iter = max_iter;
+    t.hist = hist, t.hist_cap = hist_cap;
+    return t;
+  };
+  // y = A x with the partials of (rtilde, y)
+  auto matvec_dot = [&](const double* xin, double* y) -> int {
+    pb ^= 1;
+    npart = mb > 0 ? mb : red_blocks_;
+    if (mb > 0)
+      return Check(LaunchRhsGeneralDot(args_, xin, y, 1, 1, rt, nullptr, part[pb], stream_),
+                   "rhs_general dot");
     int e = RhsDevice(xin, y, 1);
-    if (!e) e = dot_step(rt, y, 0, op, 0, 0);
+    if (!e) e = Check(LaunchDotPartial(rt, y, n, part[pb], red_blocks_, stream_), "dot");
     return e;
-  };
-  auto pairs = [&](const ZPairs& pr, const double2* c) -> int {
-    return Check(LaunchZaxpyPairs(pr, n, c, &S->stop, stream_), "axpy pairs");
-  };
-  auto comb = [&](double* y, const ZTerms& t) -> int {
-    return Check(LaunchZcombDev(y, y, t, n, &S->stop, stream_), "lincomb terms");
   };
   // r_0 = b - A x (b = e_0 of the trace row), rtilde = r_0, u_0 = 0
   if (!rc) rc = RhsDevice(x, vu[0], 1);
@@ -1452,14 +1442,15 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
   if (!rc) rc = Check(hipMemsetAsync(vu[0], 0, bytes, stream_), "u0");
   // |r_0|^2 into dot[2] and the first BiCG step's (rtilde, r_0) into dot[3];
   // every cycle ends the same way.
-  if (!rc) rc = dot2_step(vr[0], vr[0], rt, vr[0], 2, kBlInit, 0, 0);
-  // One cycle: ell BiCG steps, then the minimal-residual part (the first
-  // step's beta comes from the previous kBlInit / kBlEnd).
-  auto enqueue_cycle = [&]() -> int {
+  if (!rc)
+    rc = Check(LaunchBicglDot2Step(vr[0], vr[0], rt, vr[0], n, d_partial_, red_blocks_ / 2, S, 2,
+                                   kBlInit, 0, 0, tol, max_iter, hist, hist_cap, stream_),
+               "bicgstab(l) start");
+  // One cycle: ell BiCG steps, then the minimal-residual part; first: the
+  // record is that of a finished cycle.
+  auto enqueue_cycle = [&](bool first) -> int {
     int e = kOk;
     for (int j = 0; j < ell && !e; ++j) {
-      // (beta: from kBlInit / kBlEnd for j = 0, else from the matvec that
-      // made r_j)
       // u_i = r_i - beta u_i, i <= j
       ZPairs up{};
       for (int i = 0; i <= j; ++i) {
@@ -1469,8 +1460,9 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
         up.sign[i] = -1.;
       }
       up.count = j + 1;
-      if (!e) e = pairs(up, &S->beta);
-      if (!e) e = matvec_dot(vu[j], vu[j + 1], kBlAlpha);
+      const int op = j > 0 ? kBlBeta : (first ? kBlNone : kBlEnd);
+      e = Check(LaunchBicglPairs(up, n, take(op, ell, 0), false, stream_), "bicgstab(l) u");
+      if (!e) e = matvec_dot(vu[j], vu[j + 1]);
       // r_i -= alpha u_{i+1}, i <= j, and x += alpha u_0
       ZPairs rp{};
       for (int i = 0; i <= j; ++i) {
@@ -1484,36 +1476,47 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
       rp.b[j + 1] = vu[0];
       rp.sign[j + 1] = 1.;
       rp.count = j + 2;
-      if (!e) e = pairs(rp, &S->alpha);
-      // r_{j+1} = A r_j, and the next BiCG step's beta from (rtilde, r_{j+1})
       if (!e)
-        e = j + 1 < ell ? matvec_dot(vr[j], vr[j + 1], kBlBeta) : RhsDevice(vr[j], vr[j + 1], 1);
-    }
-    // modified Gram-Schmidt
-    for (int j = 1; j <= ell && !e; ++j) {
-      for (int i = 1; i < j && !e; ++i) {
-        e = dot_step(vr[i], vr[j], 0, kBlTau, i, j);
-        if (!e) e = axpy(vr[j], vr[j], vr[i], &S->tau[i][j], -1.);
+        e = Check(LaunchBicglPairs(rp, n, take(kBlAlpha, 0, 0), true, stream_), "bicgstab(l) r");
+      // r_{j+1} = A r_j, with the next BiCG step's (rtilde, r_{j+1}) or, of
+      // two steps, the first Gram-Schmidt products
+      if (!e && j + 1 < ell) {
+        e = matvec_dot(vr[j], vr[j + 1]);
+      } else if (!e && ell == 2 && mb > 0) {
+        pb ^= 1;
+        npart = mb;
+        e = Check(LaunchRhsGeneralDot(args_, vr[1], vr[2], 1, 2, vr[1], vr[0], part[pb], stream_),
+                  "rhs_general dot");
+      } else if (!e) {
+        e = RhsDevice(vr[j], vr[j + 1], 1);
+        pb ^= 1;
+        if (!e)
+          e = Check(LaunchBicglGram(vr[1], nullptr, vr[0], ell > 1 ? vr[1] : nullptr,
+                                    ell > 1 ? vr[2] : nullptr, true, n, take(kBlNone, 0, 0), 0, 0,
+                                    part[pb], &npart, stream_),
+                    "bicgstab(l) products");
       }
-      // (for j = ell this also solves for g, gpp and omega)
-      if (!e) e = dot2_step(vr[j], vr[j], vr[j], vr[0], 0, kBlSigma, ell, j);
     }
-    // x += g_1 r_0 + sum gpp_j r_j (before r_0 changes), then
-    // r_0 -= gp_ell r_ell + sum gp_j r_j and u_0 -= g_ell u_ell + sum g_j u_j
-    ZTerms tx{}, tr{}, tu{};
-    tx.b[0] = vr[0], tx.c[0] = &S->g[1], tx.sign[0] = 1.;
-    tr.b[0] = vr[ell], tr.c[0] = &S->gp[ell], tr.sign[0] = -1.;
-    tu.b[0] = vu[ell], tu.c[0] = &S->g[ell], tu.sign[0] = -1.;
-    for (int j = 1; j <= ell - 1; ++j) {
-      tx.b[j] = vr[j], tx.c[j] = &S->gpp[j], tx.sign[j] = 1.;
-      tr.b[j] = vr[j], tr.c[j] = &S->gp[j], tr.sign[j] = -1.;
-      tu.b[j] = vu[j], tu.c[j] = &S->g[j], tu.sign[j] = -1.;
+    // modified Gram-Schmidt: r_j -= tau_ij r_i, i < j, each pass with the
+    // products of the next (after i = j - 1: sigma_j, gp_j and tau_{1,j+1})
+    for (int j = 2; j <= ell && !e; ++j)
+      for (int i = 1; i < j && !e; ++i) {
+        const BicglTake t = i == 1 ? take(kBlSigma, ell, j - 1) : take(kBlTau, i, j);
+        const bool last = i == j - 1, more = last && j < ell;
+        pb ^= 1;
+        e = Check(LaunchBicglGram(vr[j], vr[i], last ? vr[0] : vr[i + 1], more ? vr[1] : nullptr,
+                                  more ? vr[j + 1] : nullptr, last, n, t, i, j, part[pb], &npart,
+                                  stream_),
+                  "bicgstab(l) orthogonalise");
+      }
+    if (!e) {
+      BicglVectors v{};
+      for (int j = 0; j <= ell; ++j) v.r[j] = vr[j], v.u[j] = vu[j];
+      const BicglTake t = take(kBlSigma, ell, ell);
+      pb ^= 1;
+      e = Check(LaunchBicglEnd(x, v, ell, rt, n, t, part[pb], &npart, stream_),
+                "bicgstab(l) end of cycle");
     }
-    tx.count = tr.count = tu.count = ell;
-    if (!e) e = comb(x, tx);
-    if (!e) e = comb(vr[0], tr);
-    if (!e) e = comb(vu[0], tu);
-    if (!e) e = dot2_step(vr[0], vr[0], rt, vr[0], 2, kBlEnd, ell, 0);
     return e;
   };
   // Batches of cycles (about 16 BiCG steps) between the host's checks,
@@ -1522,7 +1525,13 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
   const int batch = std::max(1, 16 / ell);
   auto enqueue_batch = [&]() -> int {
     int e = kOk;
-    for (int b = 0; b < batch && !e; ++b) e = enqueue_cycle();
+    for (int b = 0; b < batch && !e; ++b) e = enqueue_cycle(b == 0);
+    if (!e) {
+      BicglTake t = take(kBlEnd, ell, 0);
+      t.out = S;
+      cur = 0;
+      e = Check(LaunchBicglFinish(t, stream_), "bicgstab(l) close");
+    }
     return e;
   };
   BicglScalars hs{};
@@ -1559,7 +1568,7 @@ int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* 
   const int rc_sync = Synchronize();
   Free(S);
   Free(hist);
-  Free(pmv);
+  for (auto p : part) Free(p);
   cleanup();
   if (!rc) rc = rc_sync;
   if (iters) *iters = hs.it;

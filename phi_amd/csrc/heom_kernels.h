@@ -233,10 +233,9 @@ hipError_t LaunchBicgFinish(const BicgScalars* prev, BicgScalars* next, const do
                             int nblocks, double* hist, double tol, int max_iter, hipStream_t s);
 
 // BiCGSTAB(ell) with its scalars on the device (Sleijpen and Fokkema 1993,
-// Algorithm 3.1).  Dot products land in dot[0..3] through
-// LaunchBicglDotStep or LaunchBicglDot2Step, whose reduction kernel then
-// runs a scalar step on one thread to derive the scalars from them; the vector
-// updates read their coefficient from this record.  stop (breakdown,
+// Algorithm 3.1).  Dot products land in dot[0..3], and a scalar step on one
+// thread derives the scalars from them; the vector updates take their
+// coefficient from this record.  stop (breakdown,
 // convergence or the step cap) turns every later step and update into a
 // no-op, so whole cycles can be enqueued ahead of the host's check.
 constexpr int kBicglMaxEll = 8;
@@ -266,27 +265,40 @@ struct BicglScalars {
 // rho1 = dot[3] = (rtilde, r_0).  A zero rho0 or dot[0] (alpha) or a
 // non-positive sigma, or omega = 0 at the end, is a breakdown.
 enum { kBlInit = 0, kBlBeta, kBlAlpha, kBlTau, kBlSigma, kBlEnd };
-// LaunchDot's reduction of conj(u) . v into S->dot[k] followed, in the same
-// one-block kernel, by the scalar step op.
-hipError_t LaunchBicglDotStep(const double* u, const double* v, size_t n, double* partial,
-                              int nblocks, BicglScalars* S, int k, int op, int i, int j,
-                              double tol, int max_iter, double* hist, int hist_cap,
-                              hipStream_t s);
-// The reduction of nb complex partials (as LaunchRhsGeneralDot's dot 1
-// writes them) into S->dot[k], then the scalar step op.
-hipError_t LaunchBicglReduceStep(const double* partial, int nb, BicglScalars* S, int k, int op,
-                                 int i, int j, double tol, int max_iter, double* hist,
-                                 int hist_cap, hipStream_t s);
 // Two dot products in one pass, conj(a) . b into S->dot[k] and conj(c) . d
-// into S->dot[k + 1] (k = 0..2), then the scalar step op; partial holds 4
-// doubles per block (nblocks blocks).
+// into S->dot[k + 1] (k = 0..2), then the scalar step op, by a kernel of one
+// block; partial holds 4 doubles per block (nblocks blocks).
 hipError_t LaunchBicglDot2Step(const double* a, const double* b, const double* c,
                                const double* d, size_t n, double* partial, int nblocks,
                                BicglScalars* S, int k, int op, int i, int j, double tol,
                                int max_iter, double* hist, int hist_cap, hipStream_t s);
+// Inside a batch of cycles no kernel runs only to reduce: the pass that needs
+// a scalar sums the nb partials of the pass before it and takes the scalar
+// step in every block alike; block 0 writes the record for the next pass to
+// out, which is not in (the other blocks still read that).  op kBlSigma takes
+// 6 doubles a block (|r_j|^2, 0, conj(r_j) r_0, conj(r_1) r_{j+1}) and, for
+// j < i, is followed by kBlTau (1, j + 1); kBlEnd takes 4, kBlNone nothing
+// (in is final), the others 2.  A cycle of ell = 2 over 6435 7-site nodes
+// took 22 launches and 130 us with a reduction kernel (4 us) per scalar and
+// a pass per update, 10 and about 105 us this way; the passes now run at the rate of
+// their 5 MB vectors (4.6 TB/s in the end of a cycle) plus 3 us a step.
+// Loads issued behind the partials' ahead of the step: slower (15.6 against
+// 14.0 ms a solution), half the blocks in the Gram-Schmidt pass: 14.2.
+constexpr int kBlNone = -1;
+constexpr int kBicglBlocks = 1024;  // most blocks of the passes below
+struct BicglTake {
+  const BicglScalars* in;
+  BicglScalars* out;
+  const double* part;
+  int nb, op, i, j;
+  double tol;
+  int max_iter;
+  double* hist;
+  int hist_cap;
+};
 // Several updates with one coefficient, one pass: y_p = a_p + sign_p *
-// (*c) * b_p for p < count (count <= kBicglMaxEll + 1; no y_p may be an
-// input of another pair); nothing when *stop.
+// c * b_p for p < count (count <= kBicglMaxEll + 1; no y_p may be an
+// input of another pair), c = alpha or beta; nothing once stopped.
 struct ZPairs {
   double* y[kBicglMaxEll + 1];
   const double* a[kBicglMaxEll + 1];
@@ -294,23 +306,24 @@ struct ZPairs {
   double sign[kBicglMaxEll + 1];
   int count;
 };
-hipError_t LaunchZaxpyPairs(const ZPairs& pr, size_t n, const double2* c, const int* stop,
+hipError_t LaunchBicglPairs(const ZPairs& pr, size_t n, const BicglTake& t, bool alpha,
                             hipStream_t s);
-// One output from several terms: y = a + sum_t sign_t * (*c_t) * b_t over
-// t < count (count <= kBicglMaxEll; y may alias a, no b_t); nothing when
-// *stop.
-struct ZTerms {
-  const double* b[kBicglMaxEll];
-  const double2* c[kBicglMaxEll];
-  double sign[kBicglMaxEll];
-  int count;
+// y -= tau[ti][tj] b (b null: no update and no step), then the partials of
+// conj(a) y (2 doubles a block), or with norm |y|^2, 0, conj(y) a and, c
+// non-null, conj(c) d (6 doubles); *blocks = the blocks.  c and d are not y.
+hipError_t LaunchBicglGram(double* y, const double* b, const double* a, const double* c,
+                           const double* d, bool norm, size_t n, const BicglTake& t, int ti,
+                           int tj, double* partial, int* blocks, hipStream_t s);
+// x += g_1 r_0 + sum gpp_j r_j, then r_0 -= gp_ell r_ell + sum gp_j r_j and
+// u_0 -= g_ell u_ell + sum g_j u_j, and the partials of |r_0|^2 and (rt, r_0).
+struct BicglVectors {
+  double* r[kBicglMaxEll + 1];
+  double* u[kBicglMaxEll + 1];
 };
-hipError_t LaunchZcombDev(double* y, const double* a, const ZTerms& t, size_t n, const int* stop,
-                          hipStream_t s);
-// y = a + sign * (*c) * b elementwise over n complex values (y may alias a
-// or b); nothing when *stop.
-hipError_t LaunchZaxpyDev(double* y, const double* a, const double* b, size_t n,
-                          const double2* c, double sign, const int* stop, hipStream_t s);
+hipError_t LaunchBicglEnd(double* x, const BicglVectors& v, int ell, const double* rt, size_t n,
+                          const BicglTake& t, double* partial, int* blocks, hipStream_t s);
+// The step alone, one block (out may be in).
+hipError_t LaunchBicglFinish(const BicglTake& t, hipStream_t s);
 
 }  // namespace phi
 

@@ -143,7 +143,8 @@ __device__ __forceinline__ void block_sum(const double* a, double* __restrict__ 
 // The same with H, H^dagger and the ADOs of T nodes per block in LDS (one
 // load of each per element instead of 2N): for N*N*(T+2) complex within
 // the LDS budget.  DOT fuses the solver's next reduction into the matvec:
-// 1 = the block's sum of conj(w) y (2 doubles per block), 3 = the block's
+// 1 = the block's sum of conj(w) y (2 doubles per block), 2 = |w|^2,
+// conj(w) w2 and conj(w) y (6 doubles, the second zero), 3 = the block's
 // sums of conj(y) w, |y|^2, conj(w2) y and conj(w2) w (7 doubles per block).
 template <int DOT>
 __global__ void __launch_bounds__(256) rhs_general_lds(RhsArgs A, const double* __restrict__ x,
@@ -178,13 +179,19 @@ __global__ void __launch_bounds__(256) rhs_general_lds(RhsArgs A, const double* 
       // the dot operands load while the element is evaluated
       double2 q = make_double2(0., 0.), h = make_double2(0., 0.);
       if constexpr (DOT != 0) q = reinterpret_cast<const double2*>(w)[g];
-      if constexpr (DOT == 3) h = reinterpret_cast<const double2*>(w2)[g];
+      if constexpr (DOT >= 2) h = reinterpret_cast<const double2*>(w2)[g];
       const double2 v = general_elem(A, x, sx + te * NE, sH, sHd, n, r, a, b, act,
                                      trace_row && g == 0);
       reinterpret_cast<double2*>(y)[g] = v;
       if constexpr (DOT == 1) {
         acc[0] += q.x * v.x + q.y * v.y;
         acc[1] += q.x * v.y - q.y * v.x;
+      } else if constexpr (DOT == 2) {
+        acc[0] += q.x * q.x + q.y * q.y;
+        acc[2] += q.x * h.x + q.y * h.y;
+        acc[3] += q.x * h.y - q.y * h.x;
+        acc[4] += q.x * v.x + q.y * v.y;
+        acc[5] += q.x * v.y - q.y * v.x;
       } else if constexpr (DOT == 3) {
         acc[0] += v.x * q.x + v.y * q.y;
         acc[1] += v.x * q.y - v.y * q.x;
@@ -197,6 +204,7 @@ __global__ void __launch_bounds__(256) rhs_general_lds(RhsArgs A, const double* 
     }
   }
   if constexpr (DOT == 1) block_sum<2>(acc, partial);
+  if constexpr (DOT == 2) block_sum<6>(acc, partial);
   if constexpr (DOT == 3) block_sum<7>(acc, partial);
 }
 
@@ -489,7 +497,8 @@ __device__ __forceinline__ double2 bicg_omega(const BicgScalars* st) {
 
 // Sum of component c of nb partials (stride NC), fixed order; every
 // thread of the (256-thread) block gets the NC results.  Called by all.
-// Thread t sums records t, t + 256, ... (four loads in flight at a time),
+// Thread t sums records t, t + 256, ... (eight loads in flight at a time: a
+// chain of them is what this costs, the records come from other XCDs),
 // each wavefront folds its 64 sums by shuffles, and the four wavefront sums
 // are added in wavefront order: the same order in every block, so every
 // block derives the same scalars from them.
@@ -500,21 +509,20 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ parti
   double acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
-  int i = threadIdx.x;
-  for (; i + 768 < nb; i += 1024) {
-    double v[4][NC];
+  for (int i = threadIdx.x; i < nb; i += 2048) {
+    double v[8][NC];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 8; ++u) {
+      const int k = i + 256 * u < nb ? i + 256 * u : nb - 1;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) v[u][c] = partial[NC * (i + 256 * u) + c];
+      for (int c = 0; c < NC; ++c) v[u][c] = partial[NC * k + c];
+    }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 8; ++u)
+      if (i + 256 * u < nb)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) acc[c] += v[u][c];
+        for (int c = 0; c < NC; ++c) acc[c] += v[u][c];
   }
-  for (; i < nb; i += 256)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] += partial[NC * i + c];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
@@ -526,8 +534,6 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ parti
 #pragma unroll
   for (int c = 0; c < NC; ++c) out[c] = ((sw[0][c] + sw[1][c]) + sw[2][c]) + sw[3][c];
 }
-
-
 // Closes an iteration (every thread of every block computes the same
 // values; reduce_partials is called by all threads): from the record
 // `prev` of the iteration and the partials of |r|^2 its x/r/p update wrote,
@@ -873,10 +879,13 @@ hipError_t LaunchRhsGeneralDot(const RhsArgs& a, const double* x, double* y, int
                                hipStream_t s) {
   int T, blocks;
   RhsLdsShape(a, &T, &blocks);
-  if (blocks == 0 || (dot != 1 && dot != 3)) return hipErrorInvalidValue;
+  if (blocks == 0 || dot < 1 || dot > 3) return hipErrorInvalidValue;
   const size_t sh = (size_t)(T + 2) * a.NE * sizeof(double2);
   if (dot == 1)
     hipLaunchKernelGGL(dev::rhs_general_lds<1>, dim3((unsigned)blocks), dim3(256), sh, s, a, x,
+                       y, trace_row, (const unsigned char*)nullptr, T, w, w2, partial);
+  else if (dot == 2)
+    hipLaunchKernelGGL(dev::rhs_general_lds<2>, dim3((unsigned)blocks), dim3(256), sh, s, a, x,
                        y, trace_row, (const unsigned char*)nullptr, T, w, w2, partial);
   else
     hipLaunchKernelGGL(dev::rhs_general_lds<3>, dim3((unsigned)blocks), dim3(256), sh, s, a, x,
@@ -1207,128 +1216,273 @@ __global__ void __launch_bounds__(256) bicgl_dot2_step(const double* __restrict_
   }
 }
 
-// dot_final into S->dot[k], then the scalar step op (thread 0).
-__global__ void __launch_bounds__(256) bicgl_dot_step(const double* __restrict__ partial, int nb,
-                                                      BicglScalars* S, int k, int op, int i,
-                                                      int j, double tol, int max_iter,
-                                                      double* hist, int hist_cap) {
-  double re, im;
-  dot_reduce(partial, nb, &re, &im);
+// The scalar step(s) of t by every block of the launch: the record in -> LDS,
+// the partials into its dot products, the step on one thread.  Block 0
+// writes the record to t.out (t.out may be t.in only in a one-block launch).
+// Called by every thread; returns the block's copy.
+__device__ __forceinline__ const BicglScalars* bicgl_take(const BicglTake& t) {
+  __shared__ __align__(16) BicglScalars rec;
+  constexpr int kWords = sizeof(BicglScalars) / sizeof(double);
+  static_assert(sizeof(BicglScalars) % sizeof(double) == 0 && kWords <= 256,
+                "record copied by one double a thread");
+  const double* src = reinterpret_cast<const double*>(t.in);
+  double* dst = reinterpret_cast<double*>(&rec);
+  const int w = min((int)threadIdx.x, kWords - 1);
+  const double word = src[w];
+  double q[6] = {0, 0, 0, 0, 0, 0};
+  if (t.op == kBlEnd)
+    reduce_partials<4>(t.part, t.nb, q);
+  else if (t.op == kBlSigma)
+    reduce_partials<6>(t.part, t.nb, q);
+  else if (t.op != kBlNone)
+    reduce_partials<2>(t.part, t.nb, q);
+  dst[w] = word;  // (the threads past the record repeat its last word)
+  __syncthreads();
+  if (t.op == kBlNone) return &rec;
   if (threadIdx.x == 0) {
-    S->dot[k] = make_double2(re, im);
-    bicgl_body(S, op, i, j, tol, max_iter, hist, hist_cap);
+    // (hist_cap 0: only block 0 keeps the residuals)
+    const int cap = blockIdx.x == 0 ? t.hist_cap : 0;
+    const int k = t.op == kBlEnd ? 2 : 0;
+    rec.dot[k] = make_double2(q[0], q[1]);
+    if (t.op == kBlEnd || t.op == kBlSigma) rec.dot[k + 1] = make_double2(q[2], q[3]);
+    bicgl_body(&rec, t.op, t.i, t.j, t.tol, t.max_iter, t.hist, cap);
+    if (t.op == kBlSigma && t.j < t.i) {
+      rec.dot[0] = make_double2(q[4], q[5]);
+      bicgl_body(&rec, kBlTau, 1, t.j + 1, t.tol, t.max_iter, t.hist, cap);
+    }
   }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    double* out = reinterpret_cast<double*>(t.out);
+    out[w] = dst[w];
+  }
+  return &rec;
 }
 
-__global__ void __launch_bounds__(256) zaxpy_dev(double* y, const double* a, const double* b,
-                                                 size_t n, const double2* c, double sign,
-                                                 const int* stop) {
-  if (*stop) return;  // uniform: every block returns
-  const double2 cc = make_double2(sign * c->x, sign * c->y);
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    const double2 av = reinterpret_cast<const double2*>(a)[i];
-    const double2 bv = reinterpret_cast<const double2*>(b)[i];
-    reinterpret_cast<double2*>(y)[i] =
-        make_double2(av.x + (cc.x * bv.x - cc.y * bv.y), av.y + (cc.x * bv.y + cc.y * bv.x));
-  }
+__global__ void __launch_bounds__(256) bicgl_finish(BicglTake t) {
+  bicgl_take(t);
 }
 
-__global__ void __launch_bounds__(256) zaxpy_pairs(ZPairs pr, size_t n, const double2* c,
-                                                   const int* stop) {
-  if (*stop) return;  // uniform: every block returns
-  const double2 cc = *c;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
+// y_p = a_p + sign_p c b_p with c = beta or alpha of the step t.  Bounded by
+// its 3 count passes over memory; the first elements' loads are in flight
+// while the step is taken (two elements a trip, so that 7 sites to depth 8
+// run in one trip).
+template <int MP>
+__global__ void __launch_bounds__(256) bicgl_pairs(ZPairs pr, size_t n, BicglTake t, int use_alpha) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double2 av[MP][2], bv[MP][2];
+  auto load = [&](size_t i) {
 #pragma unroll
-    for (int p = 0; p < kBicglMaxEll + 1; ++p) {
-      if (p < pr.count) {
-        const double2 av = reinterpret_cast<const double2*>(pr.a[p])[i];
-        const double2 bv = reinterpret_cast<const double2*>(pr.b[p])[i];
-        const double2 k = make_double2(pr.sign[p] * cc.x, pr.sign[p] * cc.y);
-        reinterpret_cast<double2*>(pr.y[p])[i] =
-            make_double2(av.x + (k.x * bv.x - k.y * bv.y), av.y + (k.x * bv.y + k.y * bv.x));
-      }
+    for (int e = 0; e < 2; ++e) {
+      const size_t k = i + e * stride < n ? i + e * stride : n - 1;
+#pragma unroll
+      for (int p = 0; p < MP; ++p)
+        if (p < pr.count) {
+          av[p][e] = reinterpret_cast<const double2*>(pr.a[p])[k];
+          bv[p][e] = reinterpret_cast<const double2*>(pr.b[p])[k];
+        }
+    }
+  };
+  load(i0);
+  const BicglScalars* S = bicgl_take(t);
+  if (S->stop) return;  // uniform
+  const double2 c = use_alpha ? S->alpha : S->beta;
+  for (size_t i = i0; i < n; i += 2 * stride) {
+    if (i != i0) load(i);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const size_t k = i + e * stride;
+      if (k >= n) break;
+#pragma unroll
+      for (int p = 0; p < MP; ++p)
+        if (p < pr.count) {
+          const double2 f = make_double2(pr.sign[p] * c.x, pr.sign[p] * c.y);
+          const double2 u = av[p][e], v = bv[p][e];
+          reinterpret_cast<double2*>(pr.y[p])[k] =
+              make_double2(u.x + (f.x * v.x - f.y * v.y), u.y + (f.x * v.y + f.y * v.x));
+        }
     }
   }
 }
 
-__global__ void __launch_bounds__(256) zcomb_dev(double* y, const double* a, ZTerms t, size_t n,
-                                                 const int* stop) {
-  if (*stop) return;  // uniform: every block returns
-  double2 k[kBicglMaxEll];
+__device__ __forceinline__ void zdotc(double* acc, double2 u, double2 v) {
+  acc[0] += u.x * v.x + u.y * v.y;
+  acc[1] += u.x * v.y - u.y * v.x;
+}
+
+// One Gram-Schmidt update and the dot products of the next in one pass:
+// v = y - tau b (b null: v = y, nothing stored), then
+//   next == 0: conj(a) v                                        (2 doubles)
+//   next == 1: |v|^2, conj(v) a, and conj(c) d unless c is null (6 doubles)
+// with tau = tau[ti][tj] of the step t.
+template <int NEXT>
+__global__ void __launch_bounds__(256) bicgl_gram(double* y, const double* b, const double* a,
+                                                  const double* c, const double* d, size_t n,
+                                                  BicglTake t, int ti, int tj,
+                                                  double* __restrict__ partial) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double2 yv[2], av[2], bv[2], cv[2], dv[2];
+  auto load = [&](size_t i) {
 #pragma unroll
-  for (int q = 0; q < kBicglMaxEll; ++q)
-    k[q] = q < t.count ? make_double2(t.sign[q] * t.c[q]->x, t.sign[q] * t.c[q]->y)
-                       : make_double2(0., 0.);
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    double2 acc = reinterpret_cast<const double2*>(a)[i];
-#pragma unroll
-    for (int q = 0; q < kBicglMaxEll; ++q) {
-      if (q < t.count) {
-        const double2 bv = reinterpret_cast<const double2*>(t.b[q])[i];
-        acc.x += k[q].x * bv.x - k[q].y * bv.y;
-        acc.y += k[q].x * bv.y + k[q].y * bv.x;
+    for (int e = 0; e < 2; ++e) {
+      const size_t k = i + e * stride < n ? i + e * stride : n - 1;
+      yv[e] = reinterpret_cast<const double2*>(y)[k];
+      av[e] = reinterpret_cast<const double2*>(a)[k];
+      if (b) bv[e] = reinterpret_cast<const double2*>(b)[k];
+      if (NEXT != 0 && c) {
+        cv[e] = reinterpret_cast<const double2*>(c)[k];
+        dv[e] = reinterpret_cast<const double2*>(d)[k];
       }
     }
-    reinterpret_cast<double2*>(y)[i] = acc;
+  };
+  double2 tau = make_double2(0., 0.);
+  if (b) {
+    const BicglScalars* S = bicgl_take(t);
+    if (S->stop) return;  // uniform
+    tau = S->tau[ti][tj];
   }
+  double acc[6] = {0, 0, 0, 0, 0, 0};
+  for (size_t i = i0; i < n; i += 2 * stride) {
+    load(i);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (i + e * stride >= n) break;
+      double2 v = yv[e];
+      if (b) {
+        const double2 u = bv[e], f = make_double2(-tau.x, -tau.y);
+        v = make_double2(v.x + (f.x * u.x - f.y * u.y), v.y + (f.x * u.y + f.y * u.x));
+        reinterpret_cast<double2*>(y)[i + e * stride] = v;
+      }
+      if (NEXT == 0) {
+        zdotc(acc, av[e], v);
+      } else {
+        acc[0] += v.x * v.x + v.y * v.y;
+        zdotc(acc + 2, v, av[e]);
+        if (c) zdotc(acc + 4, cv[e], dv[e]);
+      }
+    }
+  }
+  if (NEXT == 0)
+    block_sum<2>(acc, partial);
+  else
+    block_sum<6>(acc, partial);
+}
+
+// The end of a cycle in one pass: x += g_1 r_0 + sum gpp_j r_j, r_0 -= gp_ell
+// r_ell + sum gp_j r_j, u_0 -= g_ell u_ell + sum g_j u_j, and the partials of
+// |r_0|^2 and (rtilde, r_0) (4 doubles).
+template <int ME>
+__global__ void __launch_bounds__(256) bicgl_end(double* x, BicglVectors vec, int ell,
+                                                 const double* __restrict__ rt, size_t n,
+                                                 BicglTake t, double* __restrict__ partial) {
+  constexpr int E = ME <= 2 ? 2 : 1;  // elements a trip
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  double2 r[E][ME + 1], u[E][ME + 1], xv[E], w[E];
+  auto load = [&](size_t i) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const size_t k = i + e * stride < n ? i + e * stride : n - 1;
+#pragma unroll
+      for (int q = 0; q <= ME; ++q)
+        if (q <= ell) {
+          r[e][q] = reinterpret_cast<const double2*>(vec.r[q])[k];
+          u[e][q] = reinterpret_cast<const double2*>(vec.u[q])[k];
+        }
+      xv[e] = reinterpret_cast<const double2*>(x)[k];
+      w[e] = reinterpret_cast<const double2*>(rt)[k];
+    }
+  };
+  const BicglScalars* S = bicgl_take(t);
+  if (S->stop) return;  // uniform
+  auto add = [](double2& s, double2 k, double2 v) {
+    s.x += k.x * v.x - k.y * v.y;
+    s.y += k.x * v.y + k.y * v.x;
+  };
+  auto neg = [](double2 k) { return make_double2(-k.x, -k.y); };
+  double acc[4] = {0, 0, 0, 0};
+  for (size_t i = i0; i < n; i += E * stride) {
+    load(i);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const size_t k = i + e * stride;
+      if (k >= n) break;
+      add(xv[e], S->g[1], r[e][0]);
+#pragma unroll
+      for (int q = 1; q <= ME; ++q)
+        if (q == ell) {
+          add(r[e][0], neg(S->gp[q]), r[e][q]);
+          add(u[e][0], neg(S->g[q]), u[e][q]);
+        }
+#pragma unroll
+      for (int q = 1; q < ME; ++q)
+        if (q < ell) {
+          add(xv[e], S->gpp[q], r[e][q]);
+          add(r[e][0], neg(S->gp[q]), r[e][q]);
+          add(u[e][0], neg(S->g[q]), u[e][q]);
+        }
+      reinterpret_cast<double2*>(x)[k] = xv[e];
+      reinterpret_cast<double2*>(vec.r[0])[k] = r[e][0];
+      reinterpret_cast<double2*>(vec.u[0])[k] = u[e][0];
+      acc[0] += r[e][0].x * r[e][0].x + r[e][0].y * r[e][0].y;
+      zdotc(acc + 2, w[e], r[e][0]);
+    }
+  }
+  block_sum<4>(acc, partial);
 }
 
 }  // namespace dev
 
-static int ZBlocks(size_t n) {
-  int blocks = (int)((n + 255) / 256);
-  if (blocks > 8192) blocks = 8192;
-  return blocks < 1 ? 1 : blocks;
+// Blocks of the BiCGSTAB(ell) vector kernels: two elements a thread, each
+// block reduces the partials it needs itself.
+static int BicglBlocks(size_t n) {
+  size_t blocks = (n + 511) / 512;
+  if (blocks > (size_t)kBicglBlocks) blocks = kBicglBlocks;
+  return blocks < 1 ? 1 : (int)blocks;
 }
 
-hipError_t LaunchZaxpyPairs(const ZPairs& pr, size_t n, const double2* c, const int* stop,
+hipError_t LaunchBicglPairs(const ZPairs& pr, size_t n, const BicglTake& t, bool alpha,
                             hipStream_t s) {
   if (pr.count < 1 || pr.count > kBicglMaxEll + 1) return hipErrorInvalidValue;
-  // unused slots repeat slot 0 (never stored to), so every pointer is valid
-  ZPairs q = pr;
-  for (int p = q.count; p < kBicglMaxEll + 1; ++p) {
-    q.y[p] = q.y[0];
-    q.a[p] = q.a[0];
-    q.b[p] = q.b[0];
-    q.sign[p] = 0;
-  }
-  hipLaunchKernelGGL(dev::zaxpy_pairs, dim3(ZBlocks(n)), dim3(256), 0, s, q, n, c, stop);
+  if (pr.count <= 3)
+    hipLaunchKernelGGL(dev::bicgl_pairs<3>, dim3(BicglBlocks(n)), dim3(256), 0, s, pr, n, t,
+                       alpha ? 1 : 0);
+  else
+    hipLaunchKernelGGL(dev::bicgl_pairs<kBicglMaxEll + 1>, dim3(BicglBlocks(n)), dim3(256), 0, s,
+                       pr, n, t, alpha ? 1 : 0);
   return hipGetLastError();
 }
 
-hipError_t LaunchZcombDev(double* y, const double* a, const ZTerms& t, size_t n, const int* stop,
-                          hipStream_t s) {
-  if (t.count < 1 || t.count > kBicglMaxEll) return hipErrorInvalidValue;
-  // unused slots repeat slot 0 with weight 0, so every pointer is valid
-  ZTerms q = t;
-  for (int k = q.count; k < kBicglMaxEll; ++k) {
-    q.b[k] = q.b[0];
-    q.c[k] = q.c[0];
-    q.sign[k] = 0;
-  }
-  hipLaunchKernelGGL(dev::zcomb_dev, dim3(ZBlocks(n)), dim3(256), 0, s, y, a, q, n, stop);
+hipError_t LaunchBicglGram(double* y, const double* b, const double* a, const double* c,
+                           const double* d, bool norm, size_t n, const BicglTake& t, int ti,
+                           int tj, double* partial, int* blocks, hipStream_t s) {
+  *blocks = BicglBlocks(n);
+  if (norm)
+    hipLaunchKernelGGL(dev::bicgl_gram<1>, dim3(*blocks), dim3(256), 0, s, y, b, a, c, d, n, t,
+                       ti, tj, partial);
+  else
+    hipLaunchKernelGGL(dev::bicgl_gram<0>, dim3(*blocks), dim3(256), 0, s, y, b, a, c, d, n, t,
+                       ti, tj, partial);
   return hipGetLastError();
 }
 
-hipError_t LaunchBicglDotStep(const double* u, const double* v, size_t n, double* partial,
-                             int nblocks, BicglScalars* S, int k, int op, int i, int j, double tol,
-                             int max_iter, double* hist, int hist_cap, hipStream_t s) {
-  if (k < 0 || k > 3) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(dev::dot_partial, dim3(nblocks), dim3(256), 0, s, u, v, n, 0, partial);
-  hipLaunchKernelGGL(dev::bicgl_dot_step, dim3(1), dim3(256), 0, s, partial, nblocks, S, k, op,
-                     i, j, tol, max_iter, hist, hist_cap);
+hipError_t LaunchBicglEnd(double* x, const BicglVectors& v, int ell, const double* rt, size_t n,
+                          const BicglTake& t, double* partial, int* blocks, hipStream_t s) {
+  if (ell < 1 || ell > kBicglMaxEll) return hipErrorInvalidValue;
+  *blocks = BicglBlocks(n);
+  if (ell <= 2)
+    hipLaunchKernelGGL(dev::bicgl_end<2>, dim3(*blocks), dim3(256), 0, s, x, v, ell, rt, n, t,
+                       partial);
+  else
+    hipLaunchKernelGGL(dev::bicgl_end<kBicglMaxEll>, dim3(*blocks), dim3(256), 0, s, x, v, ell,
+                       rt, n, t, partial);
   return hipGetLastError();
 }
 
-hipError_t LaunchBicglReduceStep(const double* partial, int nb, BicglScalars* S, int k, int op,
-                                int i, int j, double tol, int max_iter, double* hist,
-                                int hist_cap, hipStream_t s) {
-  if (k < 0 || k > 3) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(dev::bicgl_dot_step, dim3(1), dim3(256), 0, s, partial, nb, S, k, op, i, j,
-                     tol, max_iter, hist, hist_cap);
+hipError_t LaunchBicglFinish(const BicglTake& t, hipStream_t s) {
+  hipLaunchKernelGGL(dev::bicgl_finish, dim3(1), dim3(256), 0, s, t);
   return hipGetLastError();
 }
 
@@ -1340,15 +1494,6 @@ hipError_t LaunchBicglDot2Step(const double* a, const double* b, const double* c
   hipLaunchKernelGGL(dev::dot2_partial, dim3(nblocks), dim3(256), 0, s, a, b, c, d, n, partial);
   hipLaunchKernelGGL(dev::bicgl_dot2_step, dim3(1), dim3(256), 0, s, partial, nblocks, S, k, op,
                      i, j, tol, max_iter, hist, hist_cap);
-  return hipGetLastError();
-}
-
-hipError_t LaunchZaxpyDev(double* y, const double* a, const double* b, size_t n,
-                          const double2* c, double sign, const int* stop, hipStream_t s) {
-  int blocks = (int)((n + 255) / 256);
-  if (blocks > 8192) blocks = 8192;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(dev::zaxpy_dev, dim3(blocks), dim3(256), 0, s, y, a, b, n, c, sign, stop);
   return hipGetLastError();
 }
 

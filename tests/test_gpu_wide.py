@@ -1,6 +1,7 @@
 """Kernels by node size: full coupling operators (whole nodes in a wave, one
 to four elements a thread, operators all in LDS or bath by bath) and states
-above 32 (the product on the matrix cores), against the oracle."""
+above 32 (the product on the matrix cores), and the passes of BiCGSTAB(ell) by
+vector length and ell, against the oracle."""
 
 import os
 import sys
@@ -85,3 +86,42 @@ def test_more_than_32_states(N, lh, terms, precision, complex_h):
     print("wide", N, lh, terms, precision, err, flush=True)
     # FP32: the increments (|dt L| < 1 of the state) are rounded
     assert err <= (3e-14 if precision == "fp64" else 2e-6)
+
+
+class Operator:
+    """The oracle's steady-state operator as a matrix of krylov_oracle."""
+
+    def __init__(self, orc, shape):
+        self.orc, self.shape = orc, shape
+
+    def __matmul__(self, v):
+        return self.orc.steady_matvec(v.reshape(self.shape)).reshape(-1)
+
+
+@pytest.mark.parametrize("N,lh,precision,ell", [
+    (2, 2, "fp64", 2),      # fewer elements than a block has threads
+    (9, 8, "fp64", 2),      # several trips of the passes
+    (36, 2, "fp64", 1), (33, 2, "fp32", 2), (17, 3, "fp64", 3), (5, 4, "fp64", 8)])
+def test_steady_state_passes_by_size(N, lh, precision, ell):
+    from oracle import krylov_oracle as KO
+
+    rng = np.random.default_rng([N, lh])
+    H = rng.normal(0.0, 0.4, (N, N)) + 0j
+    H = H + H.T
+    rho0 = np.eye(N, dtype=complex) / N
+    kw = dict(gamma=[1.0 + 0.02 * i for i in range(N)], lambda_=[0.05] * N, temperature=0.7, lh=lh)
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    ctx = P.Context(p, precision=precision)
+    orc = HO.Oracle(HO.Problem(H=H, rho0=rho0, hbar=1.0, kb=1.0, **kw), threads=4)
+    x0 = np.zeros((ctx.num_nodes, N, N), dtype=complex)
+    x0[0] = rho0
+    b = np.zeros(x0.size, dtype=complex)
+    b[0] = 1
+    res, _ = KO.bicgstab_l(Operator(orc, x0.shape), b, x0, ell, 2)
+    ctx.set_state(x0)
+    rc, it, got = ctx.steady_state_l(ell, 1e-30, 2 * ell)
+    print("steady", N, lh, precision, ell, got, res[2], flush=True)
+    assert it == 2 * ell
+    # residuals of the same recurrence, |A|^ell ulp of the first (1e-9 to ell
+    # = 2, 1e-8 to 4 where |A| is 20; here |A| < 4)
+    assert abs(got - res[2]) <= 1e-8 * res[0]
