@@ -15,15 +15,16 @@ value    node-steps/s of the FP32-bulk ensemble run (whole slab).  The same
          ensemble in plain FP64 is reported beside it ("fp64"), and the
          FP32-bulk result's population and coherence errors against it
          (every member's rho_0 and the member average).
-roofline the dominant kernel, stream_stage (ensemble instantiation; the
+roofline the dominant kernel, packed_stage (ensemble instantiation; the
          four launches of each RK4 step, nothing else but the snapshot of
          every 10th step runs in the loop): algorithmic bytes per launch over
          the mean launch duration, i.e. a step's bytes over the timed
          region's HIP-event time per step (events on the engine's stream).
          Algorithmic bytes per node (increment form of the nested RK4
-         step, s = bytes per bulk complex element): stage 0 N^2 (16 + s),
-         stage 1 N^2 2 s, stage 2 N^2 3 s, stage 3 N^2 (32 + 2 s),
-         N^2 (48 + 8 s) per step; neighbour columns count as cache hits.  classic_accounting repeats the figures with
+         step of packed Hermitian ADOs, N^2 reals a node, s = bytes per
+         bulk complex element): stage 0 N^2 (8 + s/2), stage 1 N^2 s, stage 2
+         N^2 3 s/2, stage 3 N^2 (16 + s), N^2 (24 + 4 s) per step; neighbour
+         columns count as cache hits.  classic_accounting repeats the figures with
          the bytes of classic RK4, N^2 (160 + 6 s) per node-step.  traffic =
          calibrated HBM bytes per launch (FETCH_SIZE + WRITE_SIZE) of the
          four stages from the committed rocprofv3 counter summary.
@@ -35,7 +36,7 @@ c2_single  the 7-site depth-8 hierarchy alone (6435 nodes), FP64 and FP32
 c3_fp32  the 24-site ring at depth 4 (20475 nodes of 24x24), FP32-bulk RK4:
          node-steps/s, population / coherence error vs FP64, HBM fraction.
 c3_rkf45 the 24-site ring with RKF45 (abs tol 1e-8) to 1 ps, FP64 and FP32
-         bulk: attempts, time to 1 ps, HBM fraction of N^2 (112 + 29 s) per
+         bulk: attempts, time to 1 ps, HBM fraction of N^2 (112 + 29 s)/2 per
          attempted node-step, FP32-vs-FP64 population / coherence error.
 c2_steady_state  BiCGSTAB to residual 1e-10 from the 7-site state at 1 ps,
          and BiCGSTAB(2) from the same state.
@@ -73,12 +74,13 @@ def log(*a):
 
 def stage_bytes(N, s):
     """Algorithmic bytes per node of the four stage kernels of the increment
-    form (the default RK4 order of the persistent kernels): stage 0 reads
+    form (the default RK4 order of the persistent kernels) on packed
+    Hermitian ADOs, N^2 reals each: stage 0 reads
     rho and writes K, stage 1 reads K and writes D, stage 2 reads D and K
     and writes D', stage 3 reads D', K and rho and writes rho:
-    N^2 (48 + 8 s) per node-step."""
+    N^2 (24 + 4 s) per node-step."""
     ne = N * N
-    return [ne * (16 + s), ne * (2 * s), ne * (3 * s), ne * (32 + 2 * s)]
+    return [ne * (8 + s // 2), ne * s, ne * 3 * s // 2, ne * (16 + s)]
 
 
 def classic_stage_bytes(N, s):
@@ -287,7 +289,7 @@ def run_steady_state(P, np, p, steps, tol=1e-10, max_iter=20000):
 def run_c3_rkf45(P, np, log):
     """The 24-site ring with RKF45 (abs tol 1e-8) to 1 ps, FP64 and FP32
     bulk: attempts, time to 1 ps, attempted node-steps/s and the HBM
-    fraction of the attempt bytes N^2 (112 + 29 s)."""
+    fraction of the attempt bytes N^2 (112 + 29 s)/2 (packed Hermitian ADOs)."""
     out = {}
     for prec in ("fp64", "fp32"):
         p3 = P.PhiParameters.read(CFG3, "rkf45")
@@ -301,7 +303,7 @@ def run_c3_rkf45(P, np, log):
         N = r.shape[0]
         s = 8 if prec == "fp32" else 16
         nodes = int(info["num_nodes"])
-        bytes_attempt = nodes * N * N * (112 + 29 * s)
+        bytes_attempt = nodes * N * N * (112 + 29 * s) / 2
         out[prec] = {"attempts": int(info["steps"]), "accepted": int(info["accepted"]),
                      "time_to_1ps_s": info["seconds"],
                      "node_steps_per_s": nodes * info["steps"] / info["seconds"],
@@ -476,10 +478,11 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": mean_traffic(PROFILE_ENS, "fp32"),
-                     "kernel": "stream_stage, ensemble instantiation (the 4 launches of an "
+                     "kernel": "packed_stage, ensemble instantiation (the 4 launches of an "
                                "RK4 step, increment form, FP32 bulk)",
                      "bytes_per_launch": per_launch, "launch_ms": launch_ms,
-                     "accounting": "increment-form RK4, N^2 (48 + 8 s) per node-step, s = 8",
+                     "accounting": "increment-form RK4 on packed Hermitian ADOs, N^2 (24 + 4 s) "
+                                   "per node-step, s = 8",
                      "classic_accounting": {
                          "bytes_per_launch": classic,
                          "achieved": classic / (launch_ms * 1e-3) / 1e9,

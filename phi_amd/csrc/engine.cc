@@ -1335,8 +1335,9 @@ int Engine::Rk4StageTimes(long long nsteps, double dt, double ms[4]) {
 // a^H b: each cycle takes ell BiCG steps (u_0..u_ell, r_0..r_ell and their
 // images under A), then minimises |r_0 - sum_j gamma_j r_j| over the
 // Krylov polynomial of degree ell (modified Gram-Schmidt on r_1..r_ell).
-// Scalars on the device, derived by the passes that use them.  PHI's BicgstabLSteadyState (hierarchy_integrator.cc:
-// 3112-3489) follows the same outline.
+// Scalars on the device, derived by the passes that use them.  PHI's
+// BicgstabLSteadyState (hierarchy_integrator.cc:3112-3489) follows the same
+// outline.
 int Engine::SteadyStateL(int ell, double tol, int max_iter, int* iters, double* resid,
                          std::vector<double>* history) {
   if (members_) return Unsupported("the steady state");
