@@ -473,7 +473,10 @@ __global__ void __launch_bounds__(512)
     // (2) the previous tile's stores, then this iteration's loads
     flush();
     int got = 0;
-    const bool fetch = claims && taken == kClaim;
+    // (a claim is left at the first of its tiles past the end, so that no such
+    // tile stands in the pipeline before one of the next claim: claims of one
+    // round interleave, and the loop ends at the first tile past the end)
+    const bool fetch = claims && (taken == kClaim || i2 + step >= tile_end);
     if constexpr (kMore) {
       if (ENS && fetch && tid == 0)
         got = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

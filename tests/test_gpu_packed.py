@@ -115,6 +115,26 @@ def test_ensemble_members_equal_single_runs(N, terms, depths, blocks, precision)
         assert np.abs(got[m] - ctx.rho0()).max() <= TOL[precision] * 40
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,terms,members,blocks", [
+    (10, 2, 60, 0), (10, 2, 61, 200), (7, 1, 150, 0), (7, 1, 77, 333), (5, 2, 90, 65)])
+def test_claimed_tiles_equal_one_tile_a_block(N, terms, members, blocks, precision):
+    """Every tile is taken once whatever order the blocks' claims come in: the
+    results equal, bit for bit, those of a grid of one block per tile."""
+    rng = np.random.default_rng([N, members])
+    depths = [int(d) for d in rng.integers(2, 5, members)]
+    H, rho0, kw = problem(N, max(depths), terms, False)
+    Hs = [H + np.diag(rng.normal(0.0, 0.3, N)) for _ in range(members)]
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    out = []
+    for grid in (1 << 20, blocks):
+        ens = P.Ensemble(p, Hs, depths, precision=precision)
+        ens.set_launch(2, 0, 0, grid)
+        ens.rk4_steps(70, 0.01)
+        out.append(ens.member_rho0())
+    assert np.array_equal(out[0], out[1])
+
+
 def test_a_state_that_is_not_hermitian_takes_the_full_layout():
     H, rho0, kw = problem(7, 4, 1, False)
     ctx, x = context(H, rho0, kw, "fp64")
