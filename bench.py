@@ -139,10 +139,14 @@ def cpu_baseline(Hs, depths, seconds=12.0, steps_per_member=10):
 
 def profile_traffic(path, kernel_stage, prec):
     """HBM bytes per launch of a stage kernel from a committed counter
-    summary (lines 'stage=<s> prec=<p> fetch_bytes=<F> write_bytes=<W>')."""
+    summary (lines 'stage=<s> prec=<p> fetch_bytes=<F> write_bytes=<W>');
+    None unless the summary is of the packed kernels."""
     if not os.path.exists(path):
         return None
-    for line in open(path):
+    lines = open(path).read().splitlines()
+    if not any("packed_stage" in line for line in lines):
+        return None
+    for line in lines:
         m = re.match(r"\s*stage=(\d) prec=(\w+) fetch_bytes=([\d.eE+]+) write_bytes=([\d.eE+]+)",
                      line)
         if m and int(m.group(1)) == kernel_stage and m.group(2) == prec:
