@@ -13,8 +13,7 @@ enum Epilogue {
   kGelu,          // Z = acc + bias[j], C = GELU(Z)
   kMseGrad,       // d = acc + bias[j] - T(row i, j): C = scale d, loss partials of d^2
   kGeluGrad,      // C = acc GELU'(Z)
-  kWeight         // gradient, and row sums of A as the bias gradient: stored in C and
-                  // bias_out, or (p non-null) taken by an Adam step of p and bias p
+  kWeight         // gradient: stored in C, or (p non-null) taken by an Adam step of p
 };
 
 struct AdamArgs {
@@ -40,7 +39,7 @@ struct GemmArgs {
   const float* T;       // kMseGrad: N apart
   float scale;
   double* partial;      // kMseGrad: one sum per block
-  float* bias_out;      // kWeight
+  float* bias_out;      // kWeight: the bias gradient, sums of A(i, k) over k
   float *p, *m, *v;     // kWeight with Adam: parameters and moments (ldc = N apart)
   float *bp, *bm, *bv;  // the bias'
 };

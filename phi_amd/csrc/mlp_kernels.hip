@@ -26,14 +26,17 @@ using act::gelu_grad;
 // what bounds them is latency and launches, not the matrix cores (a training
 // step's 0.8 GFLOP is under 1 us of them) or bytes (all operands stay in L2).
 // So a wave takes a 32 x 32 tile straight from global memory into MFMA
-// fragments, with no LDS and no barrier in the loop.  The layers accumulate
-// over K in order (the fused closure pass does, and evaluates the same
-// function to the bit), one wave a block so that 128 tiles reach 128 CUs.  The
-// gradients' longer sums (K = outputs or batch rows) are split: a block's
-// four waves take the K steps w, w + 4, ... of one tile and are added through
-// LDS in wave order (deterministic).  The epilogue does what would be further launches: bias,
-// GELU, the loss and its gradient, GELU', the bias gradient (row sums of the
-// FP32 A operand) and Adam.  A training step of batch 512 is 6 launches
+// fragments, with no LDS and no barrier in the loop.  Every product
+// accumulates over K in order, whatever the tile (the fused closure pass does,
+// and evaluates the same function to the bit; a training run carries each
+// bfloat16 rounding on, so another order of the gradients' sums ends 1e-4
+// away).  A layer is one wave a block so that 128 tiles reach 128 CUs.  The
+// gradients' longer sums (K = outputs or batch rows) take four waves a tile:
+// the loads and roundings of 16 K steps are split over the waves, the
+// fragments meet in LDS, and each wave accumulates one 16 x 16 quarter over
+// all K.  The epilogue does what would be further launches: bias, GELU, the
+// loss and its gradient, GELU' and Adam; the bias gradients are blocks of the
+// weight gradients' launch.  A training step of batch 512 is 6 launches
 // instead of 17.
 //
 // v_mfma_f32_16x16x32_bf16: lane l holds A[l%16][8(l/16) .. +7] and
@@ -110,12 +113,18 @@ __device__ __forceinline__ void adam_one(float* p, float* m, float* v, long long
   p[o] = x.p - a.lr_t * mi / (sqrtf(vi) + a.eps_t);
 }
 
+// LDS of a block, 16 bytes each: with four waves the fragments of kChunk K
+// steps (A's rows, then B's columns), then the tile's sums.
+constexpr int kChunk = 16;
+constexpr int kTileLds = (kTile * (kTile + 1) * sizeof(float) + 15) / 16;
+constexpr int ProductLds(int epi) { return epi > kMseGrad ? kChunk * 2 * 2 * 64 : kTileLds; }
+
 template <int EPI>
-__device__ __forceinline__ void product(const GemmArgs& g, int block, const AdamArgs& adam) {
+__device__ __forceinline__ void product(const GemmArgs& g, int block, const AdamArgs& adam,
+                                        bf16x8* lds) {
   constexpr bool kSplit = EPI > kMseGrad;
-  constexpr int kWaves = kSplit ? 4 : 1;
-  __shared__ float part[kWaves][kTile][kTile + 1];
-  __shared__ float bsum[kWaves][4][kTile];
+  bf16x8 (*frag)[2][2][64] = reinterpret_cast<bf16x8 (*)[2][2][64]>(lds);
+  float (*part)[kTile + 1] = reinterpret_cast<float (*)[kTile + 1]>(lds);
   constexpr bool kAk = EPI != kWeight;                 // A rows contiguous along k
   constexpr bool kBk = EPI <= kMseGrad;                // B columns contiguous along k
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -147,7 +156,7 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
   for (int r = 0; r < kRows; ++r)
     ie[r] = min(i0 + (kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r), g.M - 1);
   float in[kRows], bias = 0.f;
-  AdamIn ad[kRows], adb{0.f, 0.f, 0.f};
+  AdamIn ad[kRows];
   if constexpr (EPI <= kMseGrad) bias = g.bias[jc];
   if constexpr (EPI == kMseGrad) {
     int row[kRows];
@@ -165,82 +174,103 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
 #pragma unroll
       for (int r = 0; r < kRows; ++r)
         ad[r] = adam_load(g.p, g.m, g.v, (long long)ie[r] * g.ldc + jc);
-      adb = adam_load(g.bp, g.bm, g.bv, min(i0 + (tid & 31), g.M - 1));
     }
   }
-  floatx4 acc[2][2];
-  float rs[2] = {0.f, 0.f};
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = (floatx4){0.f, 0.f, 0.f, 0.f};
-  // `count` K steps from st, all their loads in flight before the first use.
-  constexpr int kInc = kSplit ? 4 : 1;
-  auto steps = [&](int st, auto count, auto whole) {
-    constexpr int kCount = decltype(count)::value;
+  // One K step's operands of rows ri and columns cj.
+  auto load = [&](int st, auto whole, float va[2][8], float vb[2][8]) {
     constexpr bool kWhole = decltype(whole)::value;
-    float va[kCount][2][8], vb[kCount][2][8];
+    const int k = st * kStep + 8 * q;
 #pragma unroll
-    for (int u = 0; u < kCount; ++u) {
-      const int k = (st + u * kInc) * kStep + 8 * q;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if constexpr (kAk) load_rowk<kWhole>(pa[t], k, g.K, va[u][t]);
-        else load_colk<kWhole>(g.A, g.lda, nullptr, ri[t], k, g.K, va[u][t]);
-        if constexpr (kBk) load_rowk<kWhole>(pb[t], k, g.K, vb[u][t]);
-        else load_colk<kWhole>(g.B, g.ldb, EPI == kWeight ? g.rows : nullptr, cj[t], k, g.K,
-                               vb[u][t]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kCount; ++u) {
-      bf16x8 fa[2], fb[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if constexpr (EPI == kWeight) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) rs[t] += va[u][t][e];
-        }
-        fa[t] = pack8(va[u][t]);
-        fb[t] = pack8(vb[u][t]);
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+    for (int t = 0; t < 2; ++t) {
+      if constexpr (kAk) load_rowk<kWhole>(pa[t], k, g.K, va[t]);
+      else load_colk<kWhole>(g.A, g.lda, nullptr, ri[t], k, g.K, va[t]);
+      if constexpr (kBk) load_rowk<kWhole>(pb[t], k, g.K, vb[t]);
+      else load_colk<kWhole>(g.B, g.ldb, EPI == kWeight ? g.rows : nullptr, cj[t], k, g.K, vb[t]);
     }
   };
-  const int nwhole = g.K / kStep;
-  int st = kSplit ? wave : 0;
-  for (; st + 3 * kInc < nwhole; st += 4 * kInc) steps(st, Int<4>{}, Int<1>{});
-  if (st + kInc < nwhole) {
-    steps(st, Int<2>{}, Int<1>{});
-    st += 2 * kInc;
-  }
-  if (st < nwhole) {
-    steps(st, Int<1>{}, Int<1>{});
-    st += kInc;
-  }
-  if (g.K % kStep != 0 && st == nwhole) steps(st, Int<1>{}, Int<0>{});
+  const int nwhole = g.K / kStep, nsteps = (g.K + kStep - 1) / kStep;
+  if constexpr (kSplit) {
+    floatx4 acc = (floatx4){0.f, 0.f, 0.f, 0.f};
+    const int ta = wave >> 1, tb = wave & 1;  // this wave's quarter
+    for (int s0 = 0; s0 < nsteps; s0 += kChunk) {
+      // this wave's steps of the chunk, all their loads in flight
+      float va[4][2][8], vb[4][2][8];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+      for (int u = 0; u < 4; ++u) {
+        const int st = s0 + wave + 4 * u;
+        if (st < nwhole) load(st, Int<1>{}, va[u], vb[u]);
+        else if (st < nsteps) load(st, Int<0>{}, va[u], vb[u]);
+      }
+      if (s0 > 0) __syncthreads();
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+      for (int u = 0; u < 4; ++u)
+        if (s0 + wave + 4 * u < nsteps)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) part[wave][16 * a + 4 * q + r][16 * b + c] = acc[a][b][r];
-  if constexpr (EPI == kWeight) {
-    bsum[wave][q][c] = rs[0];
-    bsum[wave][q][16 + c] = rs[1];
+          for (int t = 0; t < 2; ++t) {
+            frag[wave + 4 * u][0][t][lane] = pack8(va[u][t]);
+            frag[wave + 4 * u][1][t][lane] = pack8(vb[u][t]);
+          }
+      __syncthreads();
+      const int n = min(kChunk, nsteps - s0);
+#pragma unroll 4
+      for (int u = 0; u < n; ++u)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[u][0][ta][lane], frag[u][1][tb][lane],
+                                                      acc, 0, 0, 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[16 * ta + 4 * q + r][16 * tb + c] = acc[r];
+  } else {
+    floatx4 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    // `count` K steps from st, all their loads in flight before the first use.
+    auto steps = [&](int st, auto count, auto whole) {
+      constexpr int kCount = decltype(count)::value;
+      float va[kCount][2][8], vb[kCount][2][8];
+#pragma unroll
+      for (int u = 0; u < kCount; ++u) load(st + u, whole, va[u], vb[u]);
+#pragma unroll
+      for (int u = 0; u < kCount; ++u) {
+        bf16x8 fa[2], fb[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          fa[t] = pack8(va[u][t]);
+          fb[t] = pack8(vb[u][t]);
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+      }
+    };
+    int st = 0;
+    for (; st + 3 < nwhole; st += 4) steps(st, Int<4>{}, Int<1>{});
+    if (st + 1 < nwhole) {
+      steps(st, Int<2>{}, Int<1>{});
+      st += 2;
+    }
+    if (st < nwhole) {
+      steps(st, Int<1>{}, Int<1>{});
+      ++st;
+    }
+    if (st < nsteps) steps(st, Int<1>{}, Int<0>{});
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[16 * a + 4 * q + r][16 * b + c] = acc[a][b][r];
   }
   __syncthreads();
   double loss = 0;
 #pragma unroll
   for (int r = 0; r < kRows; ++r) {
     const int row = kSplit ? (tid >> 5) + 8 * r : (lane >> 5) + 2 * r;
-    float x = part[0][row][col];
-    if constexpr (kSplit)
-      x = ((x + part[1][row][col]) + part[2][row][col]) + part[3][row][col];
+    float x = part[row][col];
     const long long o = (long long)ie[r] * g.ldc + jc;
     const bool ok = i0 + row < g.M && j < g.N;
     if constexpr (EPI == kBias) {
@@ -268,38 +298,66 @@ __device__ __forceinline__ void product(const GemmArgs& g, int block, const Adam
       }
     }
   }
-  if constexpr (EPI == kWeight) {
-    if (j0 == 0 && tid < kTile && i0 + tid < g.M) {
-      float x = 0.f;
-      for (int w = 0; w < 4; ++w)
-        for (int u = 0; u < 4; ++u) x += bsum[w][u][tid];
-      if (g.bp) adam_one(g.bp, g.bm, g.bv, i0 + tid, x, adb, adam);
-      else g.bias_out[i0 + tid] = x;
-    }
-  }
   if constexpr (EPI == kMseGrad) {
     for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
     if (lane == 0) g.partial[block] = loss;
   }
 }
 
-template <int EPI>
-__global__ void __launch_bounds__(EPI > kMseGrad ? 256 : 64) gemm_bf16(GemmArgs g) {
-  product<EPI>(g, blockIdx.x, AdamArgs{});
+// Bias gradients: the sums over the rows k of A(i, k), 16 columns a block, in
+// a fixed order: thread (grp, c) sums rows grp, grp + 16, ... (8 loads in
+// flight), then the 16 groups' sums are added in group order.
+constexpr int kSumCols = 16, kSumGroups = 16;
+
+__device__ __forceinline__ void bias_grad(const GemmArgs& g, int block, const AdamArgs& adam,
+                                          bf16x8* lds) {
+  float (*part)[kSumCols] = reinterpret_cast<float (*)[kSumCols]>(lds);
+  const int c = threadIdx.x % kSumCols, grp = threadIdx.x / kSumCols;
+  const int i = block * kSumCols + c, ic = min(i, g.M - 1);
+  AdamIn ad{0.f, 0.f, 0.f};
+  if (g.bp) ad = adam_load(g.bp, g.bm, g.bv, ic);
+  float s = 0.f;
+  int k = grp;
+  for (; k + 7 * kSumGroups < g.K; k += 8 * kSumGroups) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = g.A[(long long)(k + u * kSumGroups) * g.lda + ic];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  for (; k < g.K; k += kSumGroups) s += g.A[(long long)k * g.lda + ic];
+  part[grp][c] = s;
+  __syncthreads();
+  if (grp == 0 && i < g.M) {
+    float x = part[0][c];
+    for (int u = 1; u < kSumGroups; ++u) x += part[u][c];
+    if (g.bp) adam_one(g.bp, g.bm, g.bv, i, x, ad, adam);
+    else g.bias_out[i] = x;
+  }
 }
 
-// Layers' weight gradients, one after the other in the grid.
+template <int EPI>
+__global__ void __launch_bounds__(EPI > kMseGrad ? 256 : 64) gemm_bf16(GemmArgs g) {
+  __shared__ bf16x8 lds[ProductLds(EPI)];
+  product<EPI>(g, blockIdx.x, AdamArgs{}, lds);
+}
+
+// Layers' weight gradients, one after the other in the grid, then their bias
+// gradients.
 struct WeightArgs {
   GemmArgs g[3];
-  int first[4];
+  int first[7];
   AdamArgs adam;
 };
 
 __global__ void __launch_bounds__(256) weight_grads(WeightArgs w) {
+  __shared__ bf16x8 lds[ProductLds(kWeight)];
   const int b = blockIdx.x;
-  if (b < w.first[1]) product<kWeight>(w.g[0], b, w.adam);
-  else if (b < w.first[2]) product<kWeight>(w.g[1], b - w.first[1], w.adam);
-  else product<kWeight>(w.g[2], b - w.first[2], w.adam);
+  int l = 0;
+  while (l < 5 && b >= w.first[l + 1]) ++l;
+  const int i = b - w.first[l];
+  if (l < 3) product<kWeight>(w.g[l], i, w.adam, lds);
+  else bias_grad(w.g[l - 3], i, w.adam, lds);
 }
 
 }  // namespace mlp
@@ -340,7 +398,9 @@ hipError_t LaunchWeightGrads(const mlp::GemmArgs* g, int count, const mlp::AdamA
     w.g[i] = g[i];
     w.first[i + 1] = w.first[i] + Tiles(g[i].M, g[i].N);
   }
-  hipLaunchKernelGGL(mlp::weight_grads, dim3(w.first[3]), dim3(256), 0, s, w);
+  for (int i = 0; i < 3; ++i)
+    w.first[i + 4] = w.first[i + 3] + (g[i].M + mlp::kSumCols - 1) / mlp::kSumCols;
+  hipLaunchKernelGGL(mlp::weight_grads, dim3(w.first[6]), dim3(256), 0, s, w);
   return hipGetLastError();
 }
 

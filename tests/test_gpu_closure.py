@@ -69,6 +69,80 @@ def test_mlp_forward_and_gradients_match_oracle(dims, batch):
         assert ew < 5e-3 and eb < 5e-3
 
 
+def _bf16(v):
+    """float32 rounded to bfloat16 (nearest even)."""
+    b = np.asarray(v, np.float32).view(np.uint32)
+    return ((b + 0x7FFF + ((b >> 16) & 1)) & np.uint32(0xFFFF0000)).view(np.float32)
+
+
+@pytest.mark.parametrize("n_out,batch", [(686, 512), (64, 97), (32, 777), (1100, 128)])
+def test_gradient_sums_run_in_order(n_out, batch):
+    """The gradients' sums have one fixed order: the products' over K steps of
+    32 in ascending order, the bias gradients' over the rows of a residue
+    modulo 16 in ascending order, then over the residues.
+
+    Each sum holds +big, later -big, and small terms that +big absorbs (at most
+    one term per K step, so a step adds one exact product): what is left are
+    the small terms after -big.  Any other order keeps other ones."""
+    n_in, n_hid = 9, 48
+    rng = np.random.default_rng(batch)
+    net = P.Mlp(n_in, n_hid, n_out, max_batch=1024)
+    scale = np.float32(2.0) / np.float32(batch * n_out)
+
+    def cancelling(steps, shape, big, small):
+        """(steps, *shape) terms, and the steps of -big."""
+        v = np.full((steps,) + shape, small, np.float32)
+        b = rng.integers(1, steps, shape)
+        a = rng.integers(0, b)
+        np.put_along_axis(v, a[None], np.float32(big), 0)
+        np.put_along_axis(v, b[None], np.float32(-big), 0)
+        return v, b
+
+    def params(W3):
+        # hidden activations GELU(8) = 8 whatever the input
+        z = [np.zeros((n_hid, n_in)), np.full(n_hid, 8.0), np.zeros((n_hid, n_hid)),
+             np.full(n_hid, 8.0), W3, np.zeros(n_out)]
+        return np.concatenate([np.ravel(q) for q in z]).astype(np.float32)
+
+    x = rng.standard_normal((batch, n_in)).astype(np.float32)
+    # Weight and bias gradients of the last layer: outputs 0, errors -t.
+    net.set_params(params(np.zeros((n_out, n_hid))))
+    assert not net.forward(x).any()
+    steps = (batch + 31) // 32
+    d, last = cancelling(steps, (n_out,), 2.0 ** 24, 2.0 ** -10)
+    t = np.zeros((batch, n_out), np.float32)
+    rows = np.minimum(32 * np.arange(steps) + rng.integers(0, 32, steps), batch - 1)
+    t[rows] = -d
+    _, g = net.gradients(x, t)
+    (_, _), (_, _), (dW, db) = _unflat(g, [n_in, n_hid, n_hid, n_out])
+    dY = scale * (np.float32(0) - t)
+    left = 8.0 * (steps - 1 - last) * _bf16(scale * np.float32(2.0 ** -10))
+    assert np.allclose(dW, left[:, None], rtol=1e-5, atol=0)
+    s = np.zeros((16, n_out), np.float32)
+    for k in range(batch):
+        s[k % 16] += dY[k]
+    total = s[0]
+    for q in range(1, 16):
+        total = total + s[q]
+    assert np.array_equal(db, total)
+    # Input gradient of the last layer, seen in the bias gradient of the layer
+    # before: one row with errors, W3 all ones in one output per K step.
+    steps = (n_out + 31) // 32
+    outs = np.minimum(32 * np.arange(steps) + rng.integers(0, 32, steps), n_out - 1)
+    if steps > 1:
+        W3 = np.zeros((n_out, n_hid))
+        W3[outs] = 1.0
+        net.set_params(params(W3))
+        t = net.forward(x)
+        d, last = cancelling(steps, (), 2.0 ** 24, 2.0 ** -10)
+        t[0, outs] -= d
+        assert np.array_equal(net.forward(x)[0, outs] - t[0, outs], d)
+        _, g = net.gradients(x, t)
+        db = _unflat(g, [n_in, n_hid, n_hid, n_out])[1][1]
+        left = (steps - 1 - last) * _bf16(scale * np.float32(2.0 ** -10))
+        assert np.allclose(db, left, rtol=1e-5, atol=0)
+
+
 def test_mlp_training_reduces_loss():
     rng = np.random.default_rng(3)
     n_in, n_hid, n_out = 24, 64, 16
