@@ -106,8 +106,10 @@ __device__ __forceinline__ AdamIn adam_load(const float* p, const float* m, cons
 }
 __device__ __forceinline__ void adam_one(float* p, float* m, float* v, long long o, float g,
                                          const AdamIn& x, const AdamArgs& a) {
-  const float mi = a.beta1 * x.m + (1.f - a.beta1) * g;
-  const float vi = a.beta2 * x.v + (1.f - a.beta2) * g * g;
+  // (the rounding of the sums written out: left to the compiler, it depends on
+  // the code around them)
+  const float mi = fmaf(1.f - a.beta1, g, a.beta1 * x.m);
+  const float vi = fmaf((1.f - a.beta2) * g, g, a.beta2 * x.v);
   m[o] = mi;
   v[o] = vi;
   p[o] = x.p - a.lr_t * mi / (sqrtf(vi) + a.eps_t);

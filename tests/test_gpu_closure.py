@@ -143,6 +143,37 @@ def test_gradient_sums_run_in_order(n_out, batch):
         assert np.allclose(db, left, rtol=1e-5, atol=0)
 
 
+def test_adam_steps_round_one_way():
+    """Three steps on one sample against Adam in float32, its two moment updates
+    as one fused multiply-add each: the same parameters to the bit."""
+    n_in, n_hid, n_out = 9, 48, 32
+    rng = np.random.default_rng(11)
+    f32 = np.float32
+    X = rng.standard_normal((1, n_in)).astype(f32)
+    T = rng.standard_normal((1, n_out)).astype(f32)
+    p = _flat(M.init_params(n_in, n_hid, n_out, seed=4))
+    start = p.copy()
+    net = P.Mlp(n_in, n_hid, n_out, max_batch=16)
+
+    def fma(a, b, c):
+        return (np.float64(a) * np.float64(b) + np.float64(c)).astype(f32)
+
+    b1, b2, lr = f32(0.9), f32(0.999), f32(1e-2)
+    m, v = np.zeros_like(p), np.zeros_like(p)
+    for step in (1, 2, 3):
+        net.set_params(p)
+        _, g = net.gradients(X, T)
+        c1, c2 = 1.0 - np.float64(b1) ** step, 1.0 - np.float64(b2) ** step
+        lr_t = f32(np.float64(lr) * np.sqrt(c2) / c1)
+        eps_t = f32(np.float64(f32(1e-8)) * np.sqrt(c2))
+        m = fma(f32(1) - b1, g, b1 * m)
+        v = fma((f32(1) - b2) * g, g, b2 * v)
+        p = p - lr_t * m / (np.sqrt(v) + eps_t)
+    net.set_params(start)
+    net.train(X, T, batch=1, epochs=3, lr=float(lr))
+    assert np.array_equal(net.get_params(), p)
+
+
 def test_mlp_training_reduces_loss():
     rng = np.random.default_rng(3)
     n_in, n_hid, n_out = 24, 64, 16
