@@ -385,9 +385,11 @@ int Engine::CreateEnsemble(const PhiParameters& base, int members,
 int Engine::BuildTiles() {
   if (members_ == 0) return kOk;
   const int T = ActiveTile();
-  // launches in flight still read the list
+  // launches in flight still read the list, and a captured block of steps
+  // would read the new one with the old tile
   const int rs = Synchronize();
   if (rs) return rs;
+  DropGraph();
   std::vector<TileDesc> t;
   for (int m = 0; m < members_; ++m)
     for (int lb = 0; lb < mreal_[m]; lb += T)
@@ -1183,8 +1185,9 @@ void Engine::DropGraph() {
 // launch argument changes.  Only kernels are captured.
 int Engine::GraphBlock(int steps, int snap_every, double dt) {
   GraphKey key{steps, snap_every, dt, fp32_, StepForm(), args_.col_nm,
-               args_.col_tile[0], args_.col_tile[1], args_.col_threads[0], args_.col_threads[1],
-               args_.col_grid[0], args_.col_grid[1], d_y_[0],
+               args_.col_tile[0], args_.col_tile[1], args_.pk_tile[0], args_.pk_tile[1],
+               args_.ntiles, args_.col_threads[0], args_.col_threads[1],
+               args_.col_grid[0], args_.col_grid[1], d_y_[0], d_aux_,
                RunsPacked() ? d_prho_ : d_rho_, d_tiles_, {}};
   for (int f = 0; f < 2; ++f)
     for (int s = 0; s < 4; ++s) {

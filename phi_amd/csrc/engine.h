@@ -268,20 +268,26 @@ class Engine {
   // kernels with tile t of precision f; *th = the resolved count.
   int StreamThreads(int t, bool fp32, int threads, int* th);
 
+  // What a captured block of steps depends on: a stage kernel's tile is
+  // col_tile on the full layout and pk_tile on the packed one (also its LDS
+  // size and its number of tiles).  An ensemble's tile list is read when the
+  // graph runs, so rebuilding the list drops the graph (BuildTiles).
   struct GraphKey {
     int steps, snap_every;
     double dt;
     bool fp32;
-    int form, col_nm, tile0, tile1, th0, th1, grid0, grid1;
+    int form, col_nm, tile0, tile1, pk_tile0, pk_tile1, ntiles, th0, th1, grid0, grid1;
     const void* y0;
+    const void* aux;
     const void* rho;
     const void* tiles;
     std::array<int, 16> stage;  // stage_threads_ and stage_grid_
     bool operator==(const GraphKey& o) const {
       return steps == o.steps && snap_every == o.snap_every && dt == o.dt && fp32 == o.fp32 &&
              form == o.form && col_nm == o.col_nm && tile0 == o.tile0 && tile1 == o.tile1 &&
+             pk_tile0 == o.pk_tile0 && pk_tile1 == o.pk_tile1 && ntiles == o.ntiles &&
              th0 == o.th0 && th1 == o.th1 && grid0 == o.grid0 && grid1 == o.grid1 &&
-             y0 == o.y0 && rho == o.rho && tiles == o.tiles && stage == o.stage;
+             y0 == o.y0 && aux == o.aux && rho == o.rho && tiles == o.tiles && stage == o.stage;
     }
   };
   static constexpr int kGraphSteps = 32;

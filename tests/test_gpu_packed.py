@@ -102,7 +102,8 @@ def test_ensemble_members_equal_single_runs(N, terms, depths, blocks, precision)
     ens = P.Ensemble(p, Hs, depths, precision=precision)
     if blocks:
         ens.set_launch(2, 2, 0, blocks)   # many tiles and several claims per block
-    ens.rk4_steps(40, 0.01)               # eager head, graph blocks
+    ens.rk4_steps(70, 0.01)               # eager head, two graph blocks, eager tail
+    assert ens.launch_counts()[0] == 64
     got = ens.member_rho0()
     for m, (H, d) in enumerate(zip(Hs, depths)):
         kw["lh"] = d
@@ -111,8 +112,8 @@ def test_ensemble_members_equal_single_runs(N, terms, depths, blocks, precision)
         x = np.zeros((ctx.num_nodes, N, N), dtype=complex)
         x[0] = rho0
         ctx.set_state(x)
-        ctx.rk4_steps(40, 0.01)
-        assert np.abs(got[m] - ctx.rho0()).max() <= TOL[precision] * 40
+        ctx.rk4_steps(70, 0.01)
+        assert np.abs(got[m] - ctx.rho0()).max() <= TOL[precision] * 70
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
@@ -133,6 +134,33 @@ def test_claimed_tiles_equal_one_tile_a_block(N, terms, members, blocks, precisi
         ens.rk4_steps(70, 0.01)
         out.append(ens.member_rho0())
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,tile", [(4, 32), (5, 20), (7, 10), (10, 5)])
+def test_graph_blocks_follow_the_launch_shape(N, tile, precision):
+    """Graph blocks before and after a change of the shape, also to the tile
+    that the full layout takes by default (512 // N^2, the packed one takes
+    256 // (N (N + 1) / 2)): the same results as launches one by one."""
+    depths = [5, 3, 4, 5, 2, 4, 5, 5]
+    Hs = []
+    for m in range(len(depths)):
+        H, rho0, kw = problem(N, max(depths), 1, False, seed=m)
+        Hs.append(H)
+    p = P.params_from_problem(Hs[0], rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    out = []
+    for graphs in (True, False):
+        ens = P.Ensemble(p, Hs, depths, precision=precision)
+        ens.set_graphs(graphs)
+        runs = []
+        for shape in ((), (2, tile), (2, 3), (2, tile), ()):
+            ens.set_launch(*shape)
+            ens.rk4_steps(70, 0.01)
+            assert ens.launch_counts()[0] == (64 if graphs else 0)
+            runs.append(ens.state())
+        out.append(runs)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
 
 
 def test_a_state_that_is_not_hermitian_takes_the_full_layout():
