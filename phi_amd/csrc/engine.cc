@@ -132,7 +132,9 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
   }
   e->slab_nodes_ = h.num_nodes;
   e->rho0_init_.assign(p.initial_density_matrix.begin(), p.initial_density_matrix.end());
-  const size_t bytes = e->state_elems() * 2 * sizeof(double);
+  // (RKF45 swaps d_rho_ with d_aux_, which packed stages read past a short
+  // tile's end: both are padded)
+  const size_t bytes = (e->state_elems() * 2 + kPackedPad) * sizeof(double);
   if (!rc) rc = e->Check(hipMalloc((void**)&e->d_rho_, bytes), "alloc rho");
   if (!rc) rc = e->Check(hipMemset(e->d_rho_, 0, bytes), "zero rho");
   e->hist_capacity_ = kHistoryCapacity;

@@ -114,8 +114,9 @@ hipError_t LaunchRkf45Stage(const RhsArgs& a, bool fp32, int stage, const void* 
 
 // Packed Hermitian slabs (heom_packed.h).  LDS bytes of a block.
 size_t PackedTileLdsBytes(int N, int D, int L, int mps, int tile, bool fp32);
-// Nodes past a slab's (and its tables') end that a short tile's loads touch
-// reals of: buffers and tables are this much longer.
+// Reals past a slab's end that a short tile's loads touch (a tile is at most
+// 1024 reals): every buffer a packed stage reads is this much longer, and the
+// tables by the nodes that hold as many.
 constexpr int kPackedPad = 1024 + 64;
 // The increment form's stage and RKF45's on packed slabs (rho, K, yout and
 // the RKF45 buffers all packed).

@@ -222,6 +222,26 @@ def test_layout_changes_between_calls(precision):
     assert np.abs(got - rk4(rk4(orc.state()))).max() <= 1e-9 + tol
 
 
+@pytest.mark.parametrize("N,tile", [(4, 64), (5, 40), (7, 20)])
+def test_packed_steps_after_an_accepted_full_layout_attempt(N, tile):
+    """An accepted RKF45 attempt on the full layout exchanges the state with
+    the buffer that packed stages use next: tiles larger than the slab."""
+    H, rho0, kw = problem(N, 2, 1, False)
+    ctx, x = context(H, rho0, kw, "fp64")
+    ctx.set_launch(2, tile)
+    ctx.set_state(x)
+    ctx.rk4_steps(3, 0.01)
+    ref = ctx.state()
+    bent = x.copy()
+    bent[1, 0, 1] += 0.5j                 # not Hermitian
+    ctx.set_state(bent)
+    ctx.rkf45_attempt(np.full(24, 0.001))
+    ctx.rkf45_accept()
+    ctx.set_state(x)
+    ctx.rk4_steps(3, 0.01)
+    assert np.array_equal(ctx.state(), ref)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("N,lh,terms,complex_h", [
     (1, 9, 1, False), (2, 9, 2, False), (2, 2, 1, True), (3, 4, 2, True), (3, 8, 1, False),
