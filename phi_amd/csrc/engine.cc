@@ -629,13 +629,17 @@ int Engine::Unsupported(const char* what) {
 
 namespace {
 
+// packed: the layout the candidates ran on (a shape means other kernels on
+// each, and the state decides between them).
 struct TuneKey {
   int dev, N, D, L, nodes, mps, members;
   bool fp32;
   int form;
+  bool packed, closure;
   bool operator<(const TuneKey& o) const {
-    return std::tie(dev, N, D, L, nodes, mps, members, fp32, form) <
-           std::tie(o.dev, o.N, o.D, o.L, o.nodes, o.mps, o.members, o.fp32, o.form);
+    return std::tie(dev, N, D, L, nodes, mps, members, fp32, form, packed, closure) <
+           std::tie(o.dev, o.N, o.D, o.L, o.nodes, o.mps, o.members, o.fp32, o.form, o.packed,
+                    o.closure);
   }
 };
 struct TuneVal {
@@ -687,9 +691,13 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
       return kOk;
     }
   }
+  const bool stream_ok = N <= 32 && mps_ <= 2 && d_edge_ != nullptr;
+  rc = EnterState(stream_ok && !closure_ && rk4_form_ == kRk4Increment && PackedUsable());
+  if (rc) return rc;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  const TuneKey key{dev, N, h_.D, h_.L, slab_nodes_, mps_, members_, fp32_, rk4_form_};
+  const TuneKey key{dev,      N,     h_.D,      h_.L,    slab_nodes_,        mps_,
+                    members_, fp32_, rk4_form_, packed_, closure_ != nullptr};
   {
     std::lock_guard<std::mutex> lock(g_tune_mu);
     auto it = g_tune.find(key);
@@ -719,7 +727,6 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   // a reference point.
   struct Cand { int col_nm, tile, threads, blocks; };
   std::vector<Cand> cands;
-  const bool stream_ok = N <= 32 && mps_ <= 2 && d_edge_ != nullptr;
   const int grids[] = {0, cus, 2 * cus, 3 * cus, 4 * cus};
   if (stream_ok) {
     const int tiles[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128, 192, 256};
@@ -737,8 +744,6 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   if (N <= 32) cands.push_back({1, 0, 0, 0});
   cands.push_back({0, 0, 0, 0});
   // Save the state; tuning steps advance it.
-  rc = EnterState(stream_ok && !closure_ && rk4_form_ == kRk4Increment && PackedUsable());
-  if (rc) return rc;
   // (the candidates run on the state's current form; one of another form
   // runs on the other buffer, whose values do not matter)
   const bool was_packed = packed_;

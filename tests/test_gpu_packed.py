@@ -182,6 +182,21 @@ def test_a_state_that_is_not_hermitian_takes_the_full_layout():
     assert np.array_equal(ctx.state(), ctx.state().conj().transpose(0, 2, 1))
 
 
+def test_tuned_shapes_are_kept_per_layout():
+    """A shape tuned on a state that is not Hermitian (full layout) is not the
+    answer for a Hermitian one of the same sizes; another Hermitian context
+    gets the kept one."""
+    H, rho0, kw = problem(6, 6, 1, False)
+    ms = []
+    for bend in (0.25j, 0, 0):
+        ctx, x = context(H, rho0, kw, "fp64")
+        x[2, 0, 1] += bend
+        ctx.set_state(x)
+        ms.append(ctx.autotune(0.001, steps=2)[0])
+        assert np.array_equal(ctx.state(), x)
+    assert ms[0] != ms[1] == ms[2]
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_layout_changes_between_calls(precision):
     """RK4, an RKF45 attempt, an accepted one, the RHS and the autotuner on one
