@@ -916,11 +916,6 @@ bool Engine::PackedUsable() const {
   // half the data, outweighs the pairs: 55 members of 3 sites 41 us a step
   // on the full kernels, 50 packed; 96 members of 4 sites 46 and 46.
   if (h_.N < 4 || !PackedLayout()) return false;
-  // FP32 of a wide hierarchy with fewer nodes than CUs: launches bound it in
-  // either layout (84 steps of 24 23-site nodes 1.89 ms packed, 2.07 full;
-  // 171 17-site nodes 1.95 and 1.90), and the few ADOs leave the rounding of
-  // each layout's sums visible (4e-6 of the rms from 64 bits, each its own).
-  if (fp32_ && !members_ && h_.N > 16 && h_.num_nodes < 256) return false;
   if (args_.col_nm != 2) return true;
   // no more LDS than the other kernels take
   return PackedTileLdsBytes(h_.N, h_.D, h_.L, mps_, args_.pk_tile[f], f == 1) <= kLdsBudget;

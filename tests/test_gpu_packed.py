@@ -163,6 +163,24 @@ def test_graph_blocks_follow_the_launch_shape(N, tile, precision):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,lh", [(5, 5), (16, 3), (17, 3), (20, 2), (24, 2)])
+def test_a_single_hierarchy_steps_as_the_only_member(N, lh, precision):
+    """One arithmetic for a system, alone or as an ensemble's member, however
+    few its nodes are."""
+    H, rho0, kw = problem(N, lh, 1, False, seed=2)
+    p = P.params_from_problem(H, rho0, hbar=1.0, kb=1.0, precision=precision, **kw)
+    ens = P.Ensemble(p, [H], [lh], precision=precision)
+    ctx = P.Context(p, precision=precision)
+    x = np.zeros((ctx.num_nodes, N, N), dtype=complex)
+    x[0] = rho0
+    ctx.set_state(x)
+    ens.rk4_steps(5, 0.01)
+    ctx.set_launch(2, 2)                  # the stage kernels for the smallest too
+    ctx.rk4_steps(5, 0.01)
+    assert np.array_equal(ens.state().reshape(-1), ctx.state().reshape(-1))
+
+
 def test_a_state_that_is_not_hermitian_takes_the_full_layout():
     H, rho0, kw = problem(7, 4, 1, False)
     ctx, x = context(H, rho0, kw, "fp64")
