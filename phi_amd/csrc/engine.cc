@@ -879,9 +879,9 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
   return kOk;
 }
 
+// (No tile list here: the state's layout, which decides the tile, is settled
+// by the EnterState that follows every call.)
 int Engine::AllocBulk() {
-  const int rt = EnsureTiles();
-  if (rt) return rt;
   if (bulk_alloc_ && bulk_is_fp32_ == fp32_) return kOk;
   Free(d_y_[0]);
   Free(d_y_[1]);
