@@ -337,7 +337,8 @@ int phi_hip_launch_counts(const phi_ctx* c, long long* graph_steps, long long* e
  * unchanged.  Cached per device and problem shape for the process.
  * *best_ms = milliseconds per step; shape[4] = {gemm, tile, threads,
  * blocks} of the common shape as in phi_hip_set_launch
- * (phi_hip_stage_launch gives the stages' own). */
+ * (phi_hip_stage_launch gives the stages' own); {-1, 0, 0, 0}, the default,
+ * where whole steps run inside one workgroup. */
 int phi_hip_autotune(phi_ctx* c, int steps, double dt, double* best_ms, int* shape);
 
 #ifdef __cplusplus

@@ -684,10 +684,10 @@ int Engine::Autotune(int steps, double dt, double* best_ms, int shape_out[4]) {
       Free(saved);
       if (rc || rs || ry) return rc ? rc : rs ? rs : ry;
       *best_ms = ms / steps;
-      shape_out[0] = args_.col_nm;
-      shape_out[1] = args_.col_tile[f];
-      shape_out[2] = args_.col_threads[f];
-      shape_out[3] = args_.col_grid[f];
+      // the default shape, which SetLaunch takes back to the same kernel (an
+      // explicit one asks for the stage kernels)
+      shape_out[0] = -1;
+      shape_out[1] = shape_out[2] = shape_out[3] = 0;
       return kOk;
     }
   }

@@ -307,6 +307,12 @@ def test_one_workgroup_runs_longer_than_a_launch_match_the_oracle():
     ctx.set_state(x)
     ms, shape = ctx.autotune(0.001, steps=5)
     assert ms > 0 and np.array_equal(ctx.state(), x)
+    # the shape it gives sets the same kernel: no graph blocks of stage kernels
+    other = P.Context(p)
+    other.set_launch(*shape)
+    other.set_state(x)
+    other.rk4_steps(70, 0.001)
+    assert other.launch_counts() == (0, 70)
     hist = ctx.rk4_history(5000, 0.001, 500)
     assert hist.shape[0] == 10
     orc = HO.Oracle(HO.Problem(H, rho0, hbar=1.0, kb=1.0, **kw))
