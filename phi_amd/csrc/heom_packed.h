@@ -258,8 +258,13 @@ __global__ void __launch_bounds__(512)
   if constexpr (ENS) {
     const int G = gridDim.x, X = G < 8 ? G : 8;
     const int x = blockIdx.x % X;
-    tile = (int)(((long long)x * ntiles) / X) + (int)(blockIdx.x / X);
-    tile_end = (int)(((long long)(x + 1) * ntiles) / X);
+    // (the first runs one longer, as the first ones have one block more: with
+    // a block a tile every block has one.  Runs of rounded eighths gave some
+    // blocks two: 8 members of 6 sites, 228 FP64 tiles, 7.3 us a stage, 5.6
+    // this way)
+    const int q = ntiles / X, r = ntiles % X, first = x * q + min(x, r);
+    tile = first + (int)(blockIdx.x / X);
+    tile_end = first + q + (x < r ? 1 : 0);
     step = G / X + (x < G % X ? 1 : 0);
     ctr = A.tile_ctr + 16 * (8 * A.ctr_set + x);
   } else {

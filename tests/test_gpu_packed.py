@@ -118,7 +118,8 @@ def test_ensemble_members_equal_single_runs(N, terms, depths, blocks, precision)
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("N,terms,members,blocks", [
-    (10, 2, 60, 0), (10, 2, 61, 200), (7, 1, 150, 0), (7, 1, 77, 333), (5, 2, 90, 65)])
+    (10, 2, 60, 0), (10, 2, 61, 200), (7, 1, 150, 0), (7, 1, 77, 333), (5, 2, 90, 65),
+    (6, 1, 5, 0), (7, 1, 3, 5), (4, 1, 2, 0)])
 def test_claimed_tiles_equal_one_tile_a_block(N, terms, members, blocks, precision):
     """Every tile is taken once whatever order the blocks' claims come in: the
     results equal, bit for bit, those of a grid of one block per tile."""
