@@ -700,6 +700,10 @@ int ResidentBlocks(const void* kernel, int threads, size_t lds);
 // prefetches a member's H fragments two per thread.
 inline int PackedThreads(const RhsArgs& a, int ept, bool ens) {
   int th = ((a.tile * a.PE + ept - 1) / ept + 63) / 64 * 64;
+  // (17 to 19 sites: a wave more than the elements need, so that the four
+  // items of a node's product are one round: 18 17-site nodes, FP64, 6.0 us
+  // a stage without, 5.1 with)
+  if (a.N > 16 && ept == 1 && th < 256) th = 256;
   if (ens) th = th > (dev::StreamFragCount(a.N) / 2 + 63) / 64 * 64
                     ? th : (dev::StreamFragCount(a.N) / 2 + 63) / 64 * 64;
   return th;
