@@ -532,8 +532,16 @@ int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
       const int rt = StreamThreads(t, f == 1, threads, &th);
       if (rt) return rt;
       // Packed kernels: the given tile, or by default about 256 elements of
-      // one thread each.
-      a.pk_tile[f] = tile > 0 ? t : std::max(1, 256 / a.PE);
+      // one thread each.  Of a single hierarchy of up to 8 sites whose tiles
+      // all run at once either way, half as many, with a wave for every 16
+      // columns of the product (256 elements of fewer than 7 sites have more
+      // such slices than waves): FP64 us a stage, 8 or 5 nodes a tile against
+      // 25 or 12, 4 sites 210 nodes 4.6 / 5.0, 1287 nodes 4.6 / 5.3, 6 sites
+      // 462 nodes 4.9 / 5.6, 5005 nodes (1001 tiles) 6.2 / 6.6; 7 sites 6435
+      // nodes (1609 tiles) 7.2 / 7.2, 8 sites 6435 nodes (2145) 7.9 / 7.7.
+      const int few = std::max(1, std::min(128 / a.PE, 32 / N));
+      const bool small = !members_ && N <= 8 && h_.num_nodes <= 1024 * few;
+      a.pk_tile[f] = tile > 0 ? t : small ? few : std::max(1, 256 / a.PE);
       // Kernels without a persistent form (RKF45) run the one-shot
       // matrix-core kernels with 256 threads and their default tile.
       int t1 = std::max(1, std::min(64, 256 / NE));

@@ -54,7 +54,7 @@ def context(H, rho0, kw, precision):
 @pytest.mark.parametrize("N,lh,terms,complex_h", [
     (4, 5, 1, False), (4, 4, 2, True), (5, 4, 1, True), (7, 5, 1, False), (7, 3, 2, False),
     (8, 4, 1, False), (9, 3, 2, True), (13, 3, 1, False), (16, 3, 1, False), (17, 3, 1, True),
-    (19, 3, 1, False), (24, 2, 1, False), (24, 3, 1, False)])
+    (4, 13, 1, False), (6, 5, 2, True), (7, 9, 1, False), (19, 3, 1, False), (24, 2, 1, False), (24, 3, 1, False)])
 def test_packed_steps_equal_the_full_layout(N, lh, terms, complex_h, precision):
     H, rho0, kw = problem(N, lh, terms, complex_h)
     ctx, x = context(H, rho0, kw, precision)
