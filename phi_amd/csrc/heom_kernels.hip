@@ -497,31 +497,48 @@ __device__ __forceinline__ double2 bicg_omega(const BicgScalars* st) {
 
 // Sum of component c of nb partials (stride NC), fixed order; every
 // thread of the (256-thread) block gets the NC results.  Called by all.
-// Thread t sums records t, t + 256, ... (eight loads in flight at a time: a
-// chain of them is what this costs, the records come from other XCDs),
+// Thread t sums records t, t + 256, ... (up to eight loads in flight at a time:
+// a chain of them is what this costs, the records come from other XCDs),
 // each wavefront folds its 64 sums by shuffles, and the four wavefront sums
 // are added in wavefront order: the same order in every block, so every
-// block derives the same scalars from them.
-template <int NC>
+// block derives the same scalars from them.  FIT: no more loads than there
+// are records (BiCGSTAB, whose passes have 512 records or the matvec's: 160
+// iterations on 1716 7-site nodes 4.93 ms, 5.24 with eight throughout); the
+// passes of BiCGSTAB(ell) have their vectors' loads in flight beside the sums'
+// and run slower with a choice of widths (ell = 2, 160 steps on 6435 7-site
+// nodes: 8.3 ms with eight throughout, 9.0 fitted).
+template <int NC, bool FIT>
 __device__ __forceinline__ void reduce_partials(const double* __restrict__ partial, int nb,
                                                 double* out) {
   __shared__ double sw[4][NC];
   double acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = 0;
-  for (int i = threadIdx.x; i < nb; i += 2048) {
-    double v[8][NC];
+  // U records a thread from record `base`, the last ones clamped and not used.
+  auto add = [&](int i, auto width) {
+    constexpr int U = decltype(width)::value;
+    double v[U][NC];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int k = i + 256 * u < nb ? i + 256 * u : nb - 1;
 #pragma unroll
       for (int c = 0; c < NC; ++c) v[u][c] = partial[NC * k + c];
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < U; ++u)
       if (i + 256 * u < nb)
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[c] += v[u][c];
+  };
+  const int tid = threadIdx.x;
+  if constexpr (FIT) {
+    int base = 0;
+    for (; nb - base > 1024; base += 2048) add(base + tid, std::integral_constant<int, 8>{});
+    if (nb - base > 512) add(base + tid, std::integral_constant<int, 4>{});
+    else if (nb - base > 256) add(base + tid, std::integral_constant<int, 2>{});
+    else if (nb - base > 0) add(base + tid, std::integral_constant<int, 1>{});
+  } else {
+    for (int i = tid; i < nb; i += 2048) add(i, std::integral_constant<int, 8>{});
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
@@ -545,7 +562,7 @@ __device__ __forceinline__ BicgScalars bicg_close(const BicgScalars* prev, const
   BicgScalars c = *prev;
   if (c.done) return c;  // uniform
   double q[1];
-  reduce_partials<1>(xr_part, nb, q);
+  reduce_partials<1, true>(xr_part, nb, q);
   c.rn2 = make_double2(q[0], 0.);
   const double2 al = zdiv(c.rho_new, c.rv), om = bicg_omega(&c);
   c.alpha = al;
@@ -587,7 +604,7 @@ __global__ void __launch_bounds__(256) bicg_s(double* __restrict__ y, size_t n,
   }
   if (done) return;  // uniform
   double pr[2];
-  reduce_partials<2>(rv_part, nb, pr);
+  reduce_partials<2, true>(rv_part, nb, pr);
   const double2 rv = make_double2(pr[0], pr[1]);
   if (blockIdx.x == 0 && threadIdx.x == 0) cur->rv = rv;
   const double2 al = zdiv(rho, rv);
@@ -652,7 +669,7 @@ __global__ void __launch_bounds__(256) bicg_xrp(double* __restrict__ x, double* 
                                                 int nb, double* __restrict__ partial) {
   if (st->done) return;  // uniform: every block returns
   double q[7];
-  reduce_partials<7>(ts_part, nb, q);
+  reduce_partials<7, true>(ts_part, nb, q);
   const double2 ts = make_double2(q[0], q[1]), tt = make_double2(q[2], 0.);
   const double2 rt = make_double2(q[3], q[4]), rs = make_double2(q[5], q[6]);
   const double2 al = zdiv(st->rho_new, st->rv);
@@ -1231,11 +1248,11 @@ __device__ __forceinline__ const BicglScalars* bicgl_take(const BicglTake& t) {
   const double word = src[w];
   double q[6] = {0, 0, 0, 0, 0, 0};
   if (t.op == kBlEnd)
-    reduce_partials<4>(t.part, t.nb, q);
+    reduce_partials<4, false>(t.part, t.nb, q);
   else if (t.op == kBlSigma)
-    reduce_partials<6>(t.part, t.nb, q);
+    reduce_partials<6, false>(t.part, t.nb, q);
   else if (t.op != kBlNone)
-    reduce_partials<2>(t.part, t.nb, q);
+    reduce_partials<2, false>(t.part, t.nb, q);
   dst[w] = word;  // (the threads past the record repeat its last word)
   __syncthreads();
   if (t.op == kBlNone) return &rec;
