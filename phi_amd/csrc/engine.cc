@@ -444,6 +444,7 @@ Engine::~Engine() {
                   d_elem_, d_place_, d_prho_, d_pnew_, d_hfrag_, d_tile_ctr_};
   for (void* p : ptrs) Free(p);
   if (h_stage_) (void)hipHostFree(h_stage_);
+  if (h_flag_) (void)hipHostFree(h_flag_);
   if (h_ops_) (void)hipHostFree(h_ops_);
   if (h_tlstage_) (void)hipHostFree(h_tlstage_);
   delete tl_;
@@ -993,18 +994,10 @@ int Engine::EnterState(bool want_packed) {
       }
       prho_reals_ = reals;
     }
-    int bad = 0;
-    rc = Check(LaunchFillU64(reinterpret_cast<unsigned long long*>(d_err_), 0ull, 1, stream_),
-               "zero flag");
-    if (!rc) rc = Check(LaunchPack(args_, slab_nodes_, d_rho_, d_prho_,
-                                   reinterpret_cast<int*>(d_err_), stream_), "pack state");
-    if (!rc) rc = Check(hipMemcpyAsync(&bad, d_err_, sizeof(int), hipMemcpyDeviceToHost, stream_),
-                        "hermitian flag");
+    rc = EnqueuePack();
     if (!rc) rc = Synchronize();
     if (rc) return rc;
-    not_hermitian_ = bad != 0;
-    packed_ = !not_hermitian_;
-    full_fresh_ = packed_;
+    PackDone();
   }
   if (!rc && packed_) rc = BuildFrag();
   if (!rc && tile_ctr_dirty_ && d_tile_ctr_) {
@@ -1015,11 +1008,38 @@ int Engine::EnterState(bool want_packed) {
   return rc ? rc : EnsureTiles();
 }
 
+// d_rho_ into the packed slab; *h_flag_ != 0 once it ran on a state that is not
+// Hermitian (in host memory, so that no copy is needed to read it).
+int Engine::EnqueuePack() {
+  int rc = kOk;
+  if (!h_flag_) rc = Check(hipHostMalloc((void**)&h_flag_, sizeof(int)), "alloc flag");
+  if (rc) {
+    h_flag_ = nullptr;
+    return rc;
+  }
+  *h_flag_ = 0;
+  return Check(LaunchPack(args_, slab_nodes_, d_rho_, d_prho_, h_flag_, stream_), "pack state");
+}
+
+void Engine::PackDone() {
+  not_hermitian_ = *const_cast<volatile int*>(h_flag_) != 0;
+  packed_ = full_fresh_ = !not_hermitian_;
+}
+
 int Engine::SetState(const std::complex<double>* host) {
   StateReplaced();
   int rc = Check(hipMemcpyAsync(d_rho_, host, state_elems() * sizeof(std::complex<double>),
                                 hipMemcpyHostToDevice, stream_), "set state");
-  return rc ? rc : Synchronize();
+  // A context that has stepped packed will again: packed behind the copy,
+  // under the same wait (96 us for a state of 252 5-site nodes, one step and
+  // its rho_0 with a wait, a fill and a copy of the flag of its own).
+  const bool pack = !rc && d_prho_ && prho_reals_ == state_elems() + kPackedPad &&
+                    (PackedForm() || ResidentForm());
+  if (pack) rc = EnqueuePack();
+  const int rs = Synchronize();
+  if (!rc) rc = rs;
+  if (!rc && pack) PackDone();
+  return rc;
 }
 
 int Engine::GetState(std::complex<double>* host) {

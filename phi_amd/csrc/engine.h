@@ -394,6 +394,9 @@ class Engine {
     return RunsPacked() ? args_.pk_tile[f] : args_.col_tile[f];
   }
   int EnterState(bool want_packed);  // makes packed_ as wanted where it can
+  int EnqueuePack();                 // and, when it has run, PackDone
+  void PackDone();
+  int* h_flag_ = nullptr;            // pinned: the packing kernel's verdict
   int UseFull();                     // d_rho_ becomes the state
   int SyncFull();                    // d_rho_ mirrors the state
   void StateReplaced() {             // d_rho_ holds a new state

@@ -135,8 +135,8 @@ bool ResidentFits(const RhsArgs& a, bool fp32);
 hipError_t LaunchResidentRk4(const RhsArgs& a, bool fp32, double* rho, long long nsteps,
                              double dt, long long step_offset, int snap_every, double* hist,
                              int* counter, int capacity, hipStream_t s);
-// packed <- full; *flag (zeroed before) = 1 unless every ADO equals its
-// conjugate transpose exactly.
+// packed <- full; *flag (zeroed before; device or pinned host memory) = 1
+// unless every ADO equals its conjugate transpose exactly.
 hipError_t LaunchPack(const RhsArgs& a, int nodes, const double* full, double* packed, int* flag,
                       hipStream_t s);
 // full <- packed for `nodes` nodes.

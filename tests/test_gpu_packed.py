@@ -182,6 +182,25 @@ def test_a_single_hierarchy_steps_as_the_only_member(N, lh, precision):
     assert np.array_equal(ens.state().reshape(-1), ctx.state().reshape(-1))
 
 
+def test_states_set_one_after_the_other():
+    """Hermitian and other states in turn on one context, each read back as
+    set and stepped as on a context of its own."""
+    H, rho0, kw = problem(7, 4, 1, False)
+    ctx, x = context(H, rho0, kw, "fp64")
+    bent = x.copy()
+    bent[3, 1, 2] += 0.25j
+    for y in (x, bent, bent * 0.5, x * 0.5, x):
+        ctx.set_state(y)
+        assert np.array_equal(ctx.state(), y)
+        assert np.array_equal(ctx.rho0(), y[0])
+        ctx.rk4_steps(2, 0.01)
+        one, _ = context(H, rho0, kw, "fp64")
+        one.set_state(y)
+        one.rk4_steps(2, 0.01)
+        assert np.array_equal(ctx.state(), one.state())
+        ctx.set_state(x * 2.0)            # and one that is never stepped
+
+
 def test_a_state_that_is_not_hermitian_takes_the_full_layout():
     H, rho0, kw = problem(7, 4, 1, False)
     ctx, x = context(H, rho0, kw, "fp64")
