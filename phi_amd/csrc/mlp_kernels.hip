@@ -25,7 +25,7 @@ using act::gelu_grad;
 // The network's products are small (512 x 256 x 105 up to 686 x 256 x 512):
 // what bounds them is latency and launches, not the matrix cores (a training
 // step's 0.8 GFLOP is under 1 us of them) or bytes (all operands stay in L2).
-// So a wave takes a 32 x 32 tile straight from global memory into MFMA
+// So (but for large batches or layers: gemm_big) a wave takes a 32 x 32 tile straight from global memory into MFMA
 // fragments, with no LDS and no barrier in the loop.  Every product
 // accumulates over K in order, whatever the tile (the fused closure pass does,
 // and evaluates the same function to the bit; a training run carries each
@@ -338,6 +338,120 @@ __device__ __forceinline__ void bias_grad(const GemmArgs& g, int block, const Ad
   }
 }
 
+// The same products (all but kWeight) from 64 x 64 tiles, for operands that no
+// longer come for free: four waves of 32 x 32, each operand element loaded and
+// rounded once a block into LDS, the next K step's loads in flight while the
+// current one is multiplied (two buffers, one barrier a step).  The same order
+// over K, so the same results to the bit.
+constexpr int kBig = 64, kPad = 8, kPer = kBig * kStep / 256;
+
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_big(GemmArgs g) {
+  static_assert(EPI != kWeight, "layers and input gradients");
+  __shared__ __align__(16) unsigned short As[2][kBig][kStep + kPad];
+  __shared__ __align__(16) unsigned short Bs[2][kBig][kStep + kPad];  // Bs[j][k]
+  constexpr bool kBk = EPI <= kMseGrad;  // B columns contiguous along k
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int wm = wave >> 1, wn = wave & 1, q = lane >> 4, c = lane & 15;
+  const int tj = (g.N + kBig - 1) / kBig;
+  const int i0 = blockIdx.x / tj * kBig, j0 = blockIdx.x % tj * kBig;
+  // This thread's elements of a step: (tile row, k) = (tid / 32 + 8 t, tid % 32)
+  // where the operand is contiguous along k, else (tid % 64, tid / 64 + 4 t).
+  // (Rows and columns past the matrices repeat the last one; unused.)
+  const int ak = tid & (kStep - 1);
+  const float *pa[kPer], *pb[kPer];
+  int br[kPer], bk[kPer];
+#pragma unroll
+  for (int t = 0; t < kPer; ++t) {
+    const int i = min(i0 + (tid >> 5) + 8 * t, g.M - 1);
+    const bool gather = (EPI == kBias || EPI == kGelu) && g.rows;
+    pa[t] = g.A + (long long)(gather ? g.rows[i] : i) * g.lda;
+    br[t] = kBk ? (tid >> 5) + 8 * t : (tid & 63);
+    bk[t] = kBk ? ak : (tid >> 6) + 4 * t;
+    const int j = min(j0 + br[t], g.N - 1);
+    pb[t] = kBk ? g.B + (long long)j * g.ldb : g.B + j;
+  }
+  float ra[kPer], rb[kPer];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+      const int ka = k0 + ak, kb = k0 + bk[t], kac = min(ka, g.K - 1), kbc = min(kb, g.K - 1);
+      const float va = pa[t][kac];
+      const float vb = kBk ? pb[t][kbc] : pb[t][(long long)kbc * g.ldb];
+      ra[t] = ka < g.K ? va : 0.f;
+      rb[t] = kb < g.K ? vb : 0.f;
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int t = 0; t < kPer; ++t) {
+      As[buf][(tid >> 5) + 8 * t][ak] = act::to_bf16(ra[t]);
+      Bs[buf][br[t]][bk[t]] = act::to_bf16(rb[t]);
+    }
+  };
+  floatx4 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = (floatx4){0.f, 0.f, 0.f, 0.f};
+  load(0);
+  put(0);
+  __syncthreads();
+  const int nsteps = (g.K + kStep - 1) / kStep;
+  for (int st = 0; st < nsteps; ++st) {
+    const int cur = st & 1;
+    load((st + 1) * kStep);  // past the end: the last element, then zero
+    bf16x8 fa[2], fb[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      fa[a] = *reinterpret_cast<const bf16x8*>(&As[cur][wm * 32 + a * 16 + c][8 * q]);
+      fb[a] = *reinterpret_cast<const bf16x8*>(&Bs[cur][wn * 32 + a * 16 + c][8 * q]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+    if (st + 1 < nsteps) put(cur ^ 1);
+    __syncthreads();
+  }
+  double loss = 0;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + wm * 32 + a * 16 + 4 * q + r, ic = min(i, g.M - 1);
+      const long long trow = EPI == kMseGrad ? (g.rows ? g.rows[ic] : ic) : 0;
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int j = j0 + wn * 32 + b * 16 + c;
+        if (i >= g.M || j >= g.N) continue;
+        const long long o = (long long)i * g.ldc + j;
+        float x = acc[a][b][r];
+        if constexpr (EPI == kBias) {
+          g.C[o] = x + g.bias[j];
+        } else if constexpr (EPI == kGelu) {
+          x += g.bias[j];
+          g.Z[o] = x;
+          g.C[o] = gelu(x);
+        } else if constexpr (EPI == kMseGrad) {
+          const float d = x + g.bias[j] - g.T[trow * g.N + j];
+          g.C[o] = g.scale * d;
+          loss += (double)d * d;
+        } else {
+          g.C[o] = x * gelu_grad(g.Z[o]);
+        }
+      }
+    }
+  if constexpr (EPI == kMseGrad) {
+    __shared__ double red[4];
+    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
+    if (lane == 0) red[wave] = loss;
+    __syncthreads();
+    if (tid == 0) g.partial[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+  }
+}
+
 template <int EPI>
 __global__ void __launch_bounds__(EPI > kMseGrad ? 256 : 64) gemm_bf16(GemmArgs g) {
   __shared__ bf16x8 lds[ProductLds(EPI)];
@@ -366,29 +480,45 @@ __global__ void __launch_bounds__(256) weight_grads(WeightArgs w) {
 
 // --- Host launchers ---------------------------------------------------------------
 
-static int Tiles(int M, int N) {
-  return (M + mlp::kTile - 1) / mlp::kTile * ((N + mlp::kTile - 1) / mlp::kTile);
+static int Tiles(int M, int N, int tile) {
+  return (M + tile - 1) / tile * ((N + tile - 1) / tile);
 }
 
-int LayerBlocks(int M, int N) { return Tiles(M, N); }
+// 64 x 64 tiles where they fill the chip, else the 32 x 32 ones that spread a
+// small product over more CUs.  The line in 64 x 64 tiles, us of one launch,
+// small / big tiles: layers at 176 (1024 x 686, K 256) 10.2 / 10.8 and (K
+// 1024) 27.7 / 30.2, at 256 (1024 x 1024, K 1024) 36.1 / 31.1, at 512 (8192 x
+// 256, K 256) 21.8 / 15.0, at 1408 (8192 x 686, K 256) 49.7 / 26.3 and (K
+// 2048) 347 / 139; input gradients, whose B is strided in either, at 256
+// (4096 x 256, K 256) 11.9 / 13.8, at 512 (8192 x 256) 22.3 / 16.0.
+static bool UseBig(int M, int N, bool input_grad) {
+  return Tiles(M, N, mlp::kBig) >= (input_grad ? 512 : 256);
+}
+
+int LayerBlocks(int M, int N) {
+  return Tiles(M, N, UseBig(M, N, false) ? mlp::kBig : mlp::kTile);
+}
+
+template <int EPI>
+static hipError_t LaunchProduct(const mlp::GemmArgs& g, hipStream_t s) {
+  constexpr bool kGrad = EPI == mlp::kGeluGrad;
+  if (UseBig(g.M, g.N, kGrad))
+    hipLaunchKernelGGL(mlp::gemm_big<EPI>, dim3(Tiles(g.M, g.N, mlp::kBig)), dim3(256), 0, s, g);
+  else
+    hipLaunchKernelGGL(mlp::gemm_bf16<EPI>, dim3(Tiles(g.M, g.N, mlp::kTile)),
+                       dim3(kGrad ? 256 : 64), 0, s, g);
+  return hipGetLastError();
+}
 
 hipError_t LaunchLayer(const mlp::GemmArgs& g, mlp::Epilogue e, hipStream_t s) {
-  const dim3 grid(LayerBlocks(g.M, g.N)), block(64);
-  if (e == mlp::kBias)
-    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kBias>, grid, block, 0, s, g);
-  else if (e == mlp::kGelu)
-    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kGelu>, grid, block, 0, s, g);
-  else if (e == mlp::kMseGrad)
-    hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kMseGrad>, grid, block, 0, s, g);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (e == mlp::kBias) return LaunchProduct<mlp::kBias>(g, s);
+  if (e == mlp::kGelu) return LaunchProduct<mlp::kGelu>(g, s);
+  if (e == mlp::kMseGrad) return LaunchProduct<mlp::kMseGrad>(g, s);
+  return hipErrorInvalidValue;
 }
 
 hipError_t LaunchInputGrad(const mlp::GemmArgs& g, hipStream_t s) {
-  hipLaunchKernelGGL(mlp::gemm_bf16<mlp::kGeluGrad>, dim3(Tiles(g.M, g.N)), dim3(256), 0, s,
-                     g);
-  return hipGetLastError();
+  return LaunchProduct<mlp::kGeluGrad>(g, s);
 }
 
 hipError_t LaunchWeightGrads(const mlp::GemmArgs* g, int count, const mlp::AdamArgs& adam,
@@ -398,7 +528,7 @@ hipError_t LaunchWeightGrads(const mlp::GemmArgs* g, int count, const mlp::AdamA
   w.adam = adam;
   for (int i = 0; i < 3; ++i) {
     w.g[i] = g[i];
-    w.first[i + 1] = w.first[i] + Tiles(g[i].M, g[i].N);
+    w.first[i + 1] = w.first[i] + Tiles(g[i].M, g[i].N, mlp::kTile);
   }
   for (int i = 0; i < 3; ++i)
     w.first[i + 4] = w.first[i + 3] + (g[i].M + mlp::kSumCols - 1) / mlp::kSumCols;

@@ -75,8 +75,9 @@ def _bf16(v):
     return ((b + 0x7FFF + ((b >> 16) & 1)) & np.uint32(0xFFFF0000)).view(np.float32)
 
 
-@pytest.mark.parametrize("n_out,batch", [(686, 512), (64, 97), (32, 777), (1100, 128)])
-def test_gradient_sums_run_in_order(n_out, batch):
+@pytest.mark.parametrize("n_out,batch,n_hid", [(686, 512, 48), (64, 97, 48), (32, 777, 48),
+                                               (1100, 128, 48), (96, 8192, 256)])
+def test_gradient_sums_run_in_order(n_out, batch, n_hid):
     """The gradients' sums have one fixed order: the products' over K steps of
     32 in ascending order, the bias gradients' over the rows of a residue
     modulo 16 in ascending order, then over the residues.
@@ -84,9 +85,9 @@ def test_gradient_sums_run_in_order(n_out, batch):
     Each sum holds +big, later -big, and small terms that +big absorbs (at most
     one term per K step, so a step adds one exact product): what is left are
     the small terms after -big.  Any other order keeps other ones."""
-    n_in, n_hid = 9, 48
+    n_in = 9
     rng = np.random.default_rng(batch)
-    net = P.Mlp(n_in, n_hid, n_out, max_batch=1024)
+    net = P.Mlp(n_in, n_hid, n_out, max_batch=8192)
     scale = np.float32(2.0) / np.float32(batch * n_out)
 
     def cancelling(steps, shape, big, small):
@@ -141,6 +142,32 @@ def test_gradient_sums_run_in_order(n_out, batch):
         db = _unflat(g, [n_in, n_hid, n_hid, n_out])[1][1]
         left = (steps - 1 - last) * _bf16(scale * np.float32(2.0 ** -10))
         assert np.allclose(db, left, rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize("dims,batch", [((105, 256, 686), 8192), ((37, 520, 131), 2049),
+                                        ((9, 1030, 40), 1025)])
+def test_large_batches_equal_small_ones(dims, batch):
+    """Products of large batches run from larger tiles: the outputs of every row
+    are those of a batch of 100 to the bit, loss and gradients those of the
+    oracle (bounds as for the small networks above)."""
+    rng = np.random.default_rng(batch)
+    params = M.init_params(*dims, seed=3)
+    params = [(W, (rng.standard_normal(b.shape) * 0.1).astype(np.float32)) for W, b in params]
+    net = P.Mlp(*dims, max_batch=8192)
+    net.set_params(_flat(params))
+    x = rng.standard_normal((batch, dims[0])).astype(np.float32)
+    y = net.forward(x)
+    for r in range(0, batch, 100):
+        assert np.array_equal(y[r:r + 100], net.forward(x[r:r + 100]))
+    t = rng.standard_normal((batch, dims[2])).astype(np.float32)
+    loss, g = net.gradients(x, t)
+    d = (y - t).astype(np.float64)
+    assert abs(loss - np.mean(d * d)) < 1e-12 * np.mean(d * d) * np.sqrt(d.size)
+    yk, ck = M.forward(params, x, exact=False)
+    gk = M.backward(params, ck, yk, t, exact=False)
+    for (dW, db), (dWk, dbk) in zip(_unflat(g, [dims[0], dims[1], dims[1], dims[2]]), gk):
+        assert np.abs(dW - dWk).max() < 5e-3 * np.abs(dWk).max()
+        assert np.abs(db - dbk).max() < 5e-3 * np.abs(dbk).max()
 
 
 def test_adam_steps_round_one_way():
