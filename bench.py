@@ -46,7 +46,9 @@ c5_closure   the learned truncation closure: trained on depth-10 runs,
 --shape-ens/--shape-fp64/--shape-fp32/--shape-c3 pin a leg's launch shape
 instead of autotuning it (profiles of the shape an earlier run chose):
 form,tile,threads,blocks, optionally followed by threads,blocks of each of
-the four RK4 stages (the 12 values a leg's kernel_shape records).
+the four RK4 stages (the 12 values a leg's kernel_shape records: the shape
+asked for; a packed block of T nodes has ceil(T N (N + 1) / 2 / e) threads in
+whole wavefronts, e = ceil(T N^2 / threads), 3 taken as 4).
 """
 
 import argparse
@@ -64,8 +66,8 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 CFG = os.path.join(ROOT, "phi_amd", "configs", "c2.prm")
 CFG3 = os.path.join(ROOT, "phi_amd", "configs", "c3.prm")
-PROFILE_C2 = os.path.join(ROOT, "profiles", "rk4_stage_7site_depth8_traffic.txt")
-PROFILE_ENS = os.path.join(ROOT, "profiles", "rk4_stage_ensemble_512x7site.txt")
+PROFILE_C2 = os.path.join(ROOT, "profiles", "packed_stage_7site_depth8_and_24site_depth4.txt")
+PROFILE_ENS = os.path.join(ROOT, "profiles", "packed_stage_ensemble_512x7site.txt")
 
 
 def log(*a):
