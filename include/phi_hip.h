@@ -258,7 +258,8 @@ int phi_hip_rk4_steps_timed(phi_ctx* c, long long nsteps, double dt, double* ms)
 /* Stage-kernel timing: stage s (RK4 order, RK4's buffers) launched nsteps
  * times back to back between two HIP events on the context's stream;
  * ms[s] = total milliseconds of those nsteps launches.  The state is
- * restored afterwards. */
+ * restored afterwards.  (A small hierarchy that steps inside one workgroup has
+ * no stage launches: the stage kernels it would run otherwise are timed.) */
 int phi_hip_rk4_stage_times(phi_ctx* c, long long nsteps, double dt, double* ms);
 /* One RKF45 attempt.  coefs: 15 b's (b10, b20, b21, ..., b54), 4 c's of y4
  * (c50, c52, c53, c54) and 5 of y5 (c60, c62, c63, c64, c65), all already
@@ -294,7 +295,13 @@ int phi_hip_synchronize(phi_ctx* c);
  * persistent form: up to 1024 with one element per thread, up to 256 with
  * 2..4, 0 = one element per thread); blocks = grid of the persistent
  * kernels (0 = as many as are resident at once).  Every RK4 stage takes
- * this shape.  Results do not depend on the shape beyond rounding.  No
+ * this shape.  Results do not depend on the shape beyond rounding.
+ * A Hermitian state of at least 4 sites runs the persistent kernels' packed
+ * form, where threads decides how many elements of a tile's full matrices a
+ * thread stands for (ceil(tile N^2 / threads), 3 taken as 4), and a block has
+ * ceil(tile N (N + 1) / 2 / that) threads in whole wavefronts; without a tile
+ * it takes one of its own.  A small hierarchy in the default shape steps
+ * inside one workgroup instead, which has no shape.  No
  * counterpart in PHI, whose partitioning is PartitionHierarchy,
  * hierarchy_integrator.cc:636-808. */
 int phi_hip_set_launch(phi_ctx* c, int gemm, int tile, int threads, int blocks);
@@ -304,7 +311,8 @@ int phi_hip_set_launch(phi_ctx* c, int gemm, int tile, int threads, int blocks);
  * first and last stage move the FP64 state and can prefer another grid.
  * No counterpart in PHI. */
 int phi_hip_set_stage_launch(phi_ctx* c, int stage, int threads, int blocks);
-/* threads[4], blocks[4] of the four RK4 stages in the context's precision. */
+/* threads[4], blocks[4] of the four RK4 stages in the context's precision, as
+ * they were asked for (see phi_hip_set_launch for what the packed form runs). */
 int phi_hip_stage_launch(const phi_ctx* c, int* threads, int* blocks);
 /* Stage order of phi_hip_rk4_steps (the RK4 loop body of Rk4Integrate,
  * hierarchy_integrator.cc:2709-2825): 0 = PHI's k0..k3 form with an

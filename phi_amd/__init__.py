@@ -476,8 +476,9 @@ class Context:
         """Stage-kernel shape of every RK4 stage: gemm 0 = element path,
         1 = matrix cores, 2 = persistent matrix-core kernels, -1 = default;
         tile = nodes per block (0 = default); threads = threads per block
-        (0 = 256, or one element per thread for the persistent kernels);
-        blocks = grid of the persistent kernels (0 = all resident)."""
+        (0 = 256, or one element per thread for the persistent kernels, whose
+        packed form of Hermitian states takes from it the elements per
+        thread); blocks = grid of the persistent kernels (0 = all resident)."""
         _check(lib().phi_hip_set_launch(self._h, int(gemm), int(tile), int(threads),
                                         int(blocks)))
 
@@ -488,7 +489,7 @@ class Context:
 
     def stage_launch(self):
         """((threads of stages 0..3), (blocks of stages 0..3)) in the
-        context's precision."""
+        context's precision, as asked for."""
         th = (ctypes.c_int * 4)()
         bl = (ctypes.c_int * 4)()
         _check(lib().phi_hip_stage_launch(self._h, th, bl))

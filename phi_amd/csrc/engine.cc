@@ -458,8 +458,8 @@ namespace {
 constexpr size_t kLdsBudget = 64 * 1024;
 // Largest stage of the one-workgroup kernel, in clocks of LDS reads.  Both
 // ways of stepping, us a step: dimer of 495 nodes (FP64, 2 228 clocks) 8.8
-// against 17.5 on the stage kernels, 84 6-site nodes (3 528) 9.7 against 16.4,
-// 66 10-site nodes (FP32, 5 445) 17.8 against 14.9.
+// against 14.6 on the stage kernels, 84 6-site nodes (3 528) 9.7 against 14.6,
+// 66 10-site nodes (FP32, 5 445) 17.8 against 14.7.
 constexpr double kResidentReads = 4000;
 }  // namespace
 
@@ -550,7 +550,9 @@ int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
       a.v1_tile[f] = t1;
     } else {
       // Nodes per block: enough elements for every thread, fewer when the
-      // tile's LDS exceeds the budget.
+      // tile's LDS exceeds the budget.  (Above kElementMaxN states the kernels
+      // keep H out of LDS; the budget counts it all the same, which only
+      // matters for what is refused: the default tile there is one node.)
       t = tile > 0 ? tile : std::max(1, std::min(64, th / NE));
       while (t > 1 && TileLdsBytes(N, D, L, t, f == 1, with_h) > kLdsBudget) --t;
       if (TileLdsBytes(N, D, L, t, f == 1, with_h) > kLdsBudget) {
@@ -1259,7 +1261,7 @@ int Engine::Rk4Steps(long long nsteps, double dt, long long step_offset, int sna
   rc = EnterState(resident || PackedForm());
   if (rc) return rc;
   if (resident && packed_) {
-    // at most 4096 steps (some 20 ms) a launch
+    // at most 4096 steps a launch (10 to 45 ms: a step is 2.4 to 11 us)
     for (long long s = 0; s < nsteps && !rc; s += 4096)
       rc = Check(LaunchResidentRk4(args_, fp32_, d_prho_, std::min(nsteps - s, 4096LL), dt,
                                    step_offset + s, snap_every, d_hist_, d_hist_count_,

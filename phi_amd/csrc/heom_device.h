@@ -260,7 +260,8 @@ __device__ __forceinline__ void rhs_phase(const RhsArgs& A, const TI* __restrict
   const TB ih = (TB)A.inv_hbar;
   if (N > kElementMaxN) {
     // kBatch elements at a time, their first mode's gathers all in flight
-    // (an absent neighbour or an element past the tile loads its own).
+    // (an absent neighbour loads node 0's element, an element past the tile
+    // the last one's; neither is used).
     constexpr int kBatch = 5;
     const int tot = nt * NE;
     for (int e0 = threadIdx.x; e0 < tot; e0 += kBatch * blockDim.x) {

@@ -161,7 +161,8 @@ hipError_t LaunchRhsGeneral(const RhsArgs& a, const double* x, double* y, int tr
 int RhsGeneralDotBlocks(const RhsArgs& a);
 // LaunchRhsGeneral (no active flags) fused with the next reductions of the
 // steady-state solver, per block: dot 1 = sum conj(w) y (2 doubles), dot 2 =
-// |w|^2, 0, conj(w) w2 and conj(w) y (6 doubles), dot 3 = sums of conj(y) w, |y|^2, conj(w2) y and conj(w2) w (7 doubles).
+// |w|^2, 0, conj(w) w2 and conj(w) y (6 doubles), dot 3 = sums of conj(y) w,
+// |y|^2, conj(w2) y and conj(w2) w (7 doubles).
 hipError_t LaunchRhsGeneralDot(const RhsArgs& a, const double* x, double* y, int trace_row,
                                int dot, const double* w, const double* w2, double* partial,
                                hipStream_t s);

@@ -25,7 +25,8 @@ def random_state(rng, nodes, N):
 
 @pytest.mark.parametrize("N,M,terms,lh", [
     (2, 2, 1, 4), (3, 1, 3, 3), (5, 2, 2, 3), (7, 3, 1, 4), (8, 2, 1, 3), (8, 30, 1, 2),
-    (9, 2, 1, 3), (16, 1, 2, 3), (17, 2, 1, 2), (22, 2, 1, 2), (23, 1, 1, 3), (24, 1, 2, 2)])
+    (9, 2, 1, 3), (16, 1, 2, 3), (17, 2, 1, 2), (22, 2, 1, 2), (23, 1, 1, 3), (24, 1, 2, 2),
+    (26, 1, 1, 2)])
 def test_full_operators(N, M, terms, lh):
     rng = np.random.default_rng([N, M, terms, lh])
     H = rng.normal(0.0, 0.4, (N, N)) + 0j
