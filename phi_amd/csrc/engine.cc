@@ -126,9 +126,13 @@ int Engine::Create(const PhiParameters& p, Engine** out, std::string* why) {
         for (int i = bj; i < j; ++i) put(i, j);
       for (int j = bj; j < ej; ++j) put(j, j);
     }
-    rc = e->Check(Upload(&e->d_elem_, elem.data(), elem.size()), "upload elements");
-    if (!rc) rc = e->Check(Upload(&e->d_place_, place.data(), place.size()), "upload places");
+    // (one buffer and one copy for both: each costs a new context about 35 us)
     e->h_place_ = place;
+    place.resize((NE + 3) / 4 * 4);
+    for (int k = 0; k < (int)place.size(); k += 4)
+      elem.push_back(make_int4(place[k], place[k + 1], place[k + 2], place[k + 3]));
+    rc = e->Check(Upload(&e->d_elem_, elem.data(), elem.size()), "upload elements");
+    if (!rc) e->d_place_ = reinterpret_cast<int*>(e->d_elem_ + N * (N + 1) / 2);
   }
   e->slab_nodes_ = h.num_nodes;
   e->rho0_init_.assign(p.initial_density_matrix.begin(), p.initial_density_matrix.end());
@@ -441,7 +445,7 @@ Engine::~Engine() {
                   d_tiles_, d_cbmi_, d_csite_, d_cslot_, d_cx_, d_cs_, d_cy_, d_cpack_, d_cfall_, d_active_, d_kf_[0], d_kf_[1],
                   d_kf_[2], d_kf_[3], d_kf_[4], d_kf_[5], d_rot_,
                   d_ops_, d_alpha_, d_corr_, d_tlq_, d_tlsite_, d_mrho_,
-                  d_elem_, d_place_, d_prho_, d_pnew_, d_hfrag_, d_tile_ctr_};
+                  d_elem_, d_prho_, d_pnew_, d_hfrag_, d_tile_ctr_};
   for (void* p : ptrs) Free(p);
   if (h_stage_) (void)hipHostFree(h_stage_);
   if (h_flag_) (void)hipHostFree(h_flag_);
@@ -540,7 +544,9 @@ int Engine::SetLaunch(int col_nm, int tile, int threads, int blocks) {
       // 25 or 12, 4 sites 210 nodes 4.6 / 5.0, 1287 nodes 4.6 / 5.3, 6 sites
       // 462 nodes 4.9 / 5.6, 5005 nodes (1001 tiles) 6.2 / 6.6; 7 sites 6435
       // nodes (1609 tiles) 7.2 / 7.2, 8 sites 6435 nodes (2145) 7.9 / 7.7.
-      const int few = std::max(1, std::min(128 / a.PE, 32 / N));
+      // Of 8 sites 5 nodes, three waves and slices: 165 nodes 3.8, 1287 nodes
+      // 4.30 (3 nodes a tile 3.7 and 4.46, 7 nodes 3.9 and 4.38).
+      const int few = N == 8 ? 5 : std::max(1, std::min(128 / a.PE, 32 / N));
       const bool small = !members_ && N <= 8 && h_.num_nodes <= 1024 * few;
       a.pk_tile[f] = tile > 0 ? t : small ? few : std::max(1, 256 / a.PE);
       // Kernels without a persistent form (RKF45) run the one-shot

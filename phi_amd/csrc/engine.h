@@ -371,7 +371,7 @@ class Engine {
   // state is checked (every ADO equal to its conjugate transpose) once after
   // it was set; not_hermitian_ keeps a state that failed on the full kernels.
   int4* d_elem_ = nullptr;
-  int* d_place_ = nullptr;
+  int* d_place_ = nullptr;      // behind the elements, in their buffer
   std::vector<int> h_place_;
   void* d_hfrag_ = nullptr;     // H fragments of the packed kernels
   int hfrag_fp32_ = -1;         // precision they are built for (-1: stale)
