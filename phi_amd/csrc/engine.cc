@@ -1041,9 +1041,9 @@ int Engine::SetState(const std::complex<double>* host) {
   // A context that has stepped packed will again: packed behind the copy,
   // under the same wait (96 us for a state of 252 5-site nodes, one step and
   // its rho_0 with a wait, a fill and a copy of the flag of its own).
+  // (a failure to queue it leaves the state as set, to be packed later)
   const bool pack = !rc && d_prho_ && prho_reals_ == state_elems() + kPackedPad &&
-                    (PackedForm() || ResidentForm());
-  if (pack) rc = EnqueuePack();
+                    (PackedForm() || ResidentForm()) && EnqueuePack() == kOk;
   const int rs = Synchronize();
   if (!rc) rc = rs;
   if (!rc && pack) PackDone();
